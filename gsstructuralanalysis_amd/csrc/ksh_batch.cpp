@@ -70,7 +70,7 @@ int BatchDevice::ensure_desc(size_t n)
 {
     int rc;
     if ((rc = m_desc.ensure(n * sizeof(InstDesc)))) return rc;
-    if ((rc = m_bdesc.ensure(2 * n * kBandDescBytes))) return rc;
+    if ((rc = m_bdesc.ensure(std::max(2 * n * kBandDescBytes, factor_desc_bytes(n))))) return rc;
     if ((rc = m_rdesc.ensure(n * sizeof(RefDesc)))) return rc;
     if ((rc = m_stats.ensure(n * 4 * sizeof(double)))) return rc;
     if ((rc = m_info.ensure(n * sizeof(int)))) return rc;
@@ -394,7 +394,7 @@ int BatchDevice::recount_async(const std::vector<Matrix *> &ms, const std::vecto
     }
     const size_t n = rest.size();
     const size_t hb = n * (sizeof(int) + 4 * sizeof(double));
-    if ((rc = ensure_desc(n)) || (rc = B->desc.ensure(n * kBandDescBytes)) || (rc = B->info.ensure(n * sizeof(int))) ||
+    if ((rc = ensure_desc(n)) || (rc = B->desc.ensure(factor_desc_bytes(n))) || (rc = B->info.ensure(n * sizeof(int))) ||
         (rc = B->stats.ensure(n * 4 * sizeof(double))))
         return rc;
     if (B->host_bytes < hb) {
@@ -485,10 +485,10 @@ int BatchDevice::launch_early(const std::vector<Matrix *> &ms)
     int rc;
     const size_t n = ms.size();
     const size_t hb = n * (sizeof(int) + 4 * sizeof(double));
-    if (m_ebdesc.bytes < n * kBandDescBytes || m_einfo.bytes < n * sizeof(int) || m_estats.bytes < n * 4 * sizeof(double) ||
+    if (m_ebdesc.bytes < factor_desc_bytes(n) || m_einfo.bytes < n * sizeof(int) || m_estats.bytes < n * 4 * sizeof(double) ||
         m_hearly_bytes < hb)
         KSH_HIP(hipStreamSynchronize(m_early_stream));  // buffers about to be replaced
-    if ((rc = m_ebdesc.ensure(n * kBandDescBytes)) || (rc = m_einfo.ensure(n * sizeof(int))) ||
+    if ((rc = m_ebdesc.ensure(factor_desc_bytes(n))) || (rc = m_einfo.ensure(n * sizeof(int))) ||
         (rc = m_estats.ensure(n * 4 * sizeof(double))))
         return rc;
     if (m_hearly_bytes < hb) {

@@ -11,22 +11,21 @@
 //
 // Layout: lower band, column major, fac[j*ld + (i-j)], ld = bw+1, factored in place into unit L
 // and D.  Right-looking in panels of NB = 64 columns.  Panel step at c0:
-//   1. panel (one workgroup of 512 threads per band), two sub-panels of 32 columns: wave 0
-//      factors the 32 x 32 diagonal block (lane = row, column jj broadcast with v_readlane),
-//      each panel row below it is solved against L_dd D (row-wise TRSM); between the two
-//      sub-panels the second one's columns take the first one's rank-32 update (on MFMA in the
-//      register-resident form).  (One workgroup per band: a second one would read the diagonal
-//      block while the first writes it back.)  The register-resident form (bw <= 480) computes in
-//      the storage precision: in FP32 its 101 VGPRs and 80 KB of LDS let a panel workgroup share
-//      its CU with a trailing-update workgroup of the same step launch (in FP64, 212 VGPRs and
-//      157 KB, one workgroup per CU); the general form (wider bands) computes in FP64.
-//   2. trailing update: the lower triangle of the bw x bw trailing window is cut into 32 x 32
-//      blocks, one per wave, each a 2 x 2 set of 16 x 16 MFMA tiles (v_mfma_f64_16x16x4f64 /
-//      v_mfma_f32_16x16x4f32) over the NB panel columns; panel operands -d_k L[j][k] and
-//      L[i][k] come from L2, the block is read, updated and written once.
-// Plain schedule: k_band_panel, then k_band_trailing over every block, per step.  Lookahead
-// schedule: the blocks of the next panel's columns first (k_band_trailing), then k_band_step,
-// whose first workgroups factor the next panel while the others apply the remaining blocks.
+//   1. rows (k_band_rows, one wave per one or two 16-row tiles): L = A L_dd^-T D^-1 against the factored
+//      64 x 64 diagonal block, on MFMA, spread over as many workgroups as the band has rows for;
+//   2. trailing update (k_band_trailing): the lower triangle of the bw x bw trailing window is cut into
+//      32 x 32 blocks, one wave each, 2 x 2 MFMA tiles (v_mfma_f64_16x16x4f64 /
+//      v_mfma_f32_16x16x4f32) over the NB panel columns; panel operands -d_k L[j][k] and L[i][k]
+//      come from L2, the block is read, updated and written once.  The launch's first workgroups
+//      (one per band, four waves) update and factor the next diagonal block, 16 columns at a time.
+// The chain from one diagonal block to the next (rows of the next 64 columns, update, 64 pivots) is what
+// bounds a single band and small batches; the panel of one workgroup per band that these kernels
+// replace (diagonal blocks of 32 by v_readlane, rows by substitution) took 38 us a step in FP64 at
+// bw 326 and 107 us at bw 1166, against 16 + 6 us now, most of it the diagonal block's 12 us:
+// factors of a 32 x 32 roof 2.5 -> 1.3 ms, of the 128 x 128 plate 89 -> 17 ms.
+// Plain schedule: rows, then every block, per step.  Lookahead schedule: the blocks of the next panel's
+// columns first (k_band_trailing), then k_band_step, whose first workgroups solve the next panel's
+// rows while the others apply the remaining blocks.
 // Bands are sorted by order, largest first, so a step's grids cover exactly the bands that are
 // still active.  Work per band: about n bw^2 multiply-adds; HBM traffic about 2 n bw^2 / NB
 // entries (the trailing window of a step, read and written).
@@ -41,6 +40,7 @@
 #include <vector>
 
 #include "ksh_devutil.hpp"
+#include "ksh_elim_steps.hpp"
 #include "ksh_internal.hpp"
 #include "ksh_mfma.hpp"
 #include "ksh_profile.hpp"
@@ -50,314 +50,314 @@ namespace ksh {
 
 namespace {
 
-constexpr int kNS = 32;       // sub-panel width (diagonal block factored by one wave)
-constexpr int kNB = 2 * kNS;  // panel width (rank of one trailing update)
-constexpr int kPT = 512;      // panel kernel threads (TRSM rows per pass)
-constexpr int kUW = 4;        // waves per trailing-update workgroup
-constexpr int kXr = kNS + 1;  // row stride of the panel update's per-wave LDS region
+constexpr int kQ = 16;        // tile edge
+constexpr int kNB = 64;       // panel width (rank of one trailing update)
+constexpr int kPT = 512;      // lookahead step kernel threads
+constexpr int kUW = 4;        // waves per trailing-update / row-solve workgroup; the diagonal block's strips
 
-// Factor of a 32 x 32 diagonal block held in LDS (blk[kk*32 + r], lower triangle, unit pivots
-// past w) by one wave: lane r owns row r (lanes >= 32 shadow row r - 32) in registers; at step jj
-// column jj (every lane's entry jj) is broadcast with v_readlane, so the wave's FMAs take it as a
-// scalar operand and no LDS round trip sits on the chain of dependent steps.  Entries above the
-// diagonal take updates too; never read.  On return blk holds L below the diagonal and D on it;
-// dval / dinv the pivots and their inverses.  The first bad pivot (zero, not finite, or not
-// finite in the storage precision T) is recorded in *info; `clear` resets it first.
+// ---- tiles ------------------------------------------------------------------------------------
+// A 16 x 16 tile of rows R and columns K of the band lives in a wave "transposed": lane l, register
+// v hold A[R + l % 16][K + krow(l, v)], krow = Mfma16<C>::row.  In this form a product of MFMAs is at
+// once the next one's operand: with the k index of step s taken as krow(l, s) on both sides (the sum
+// over k is in another order, nothing else), the result registers of D = A B are the B operand of the
+// next product, and the same registers of another tile (L[j][k], lane = j) are an A operand.  No
+// lane exchange sits between dependent products.
+
+// -1 / d from the hardware estimate r and Newton steps (rounding of the last place; the quotient's full
+// division sequence is about twice as long and sits on the chain of the 64 pivots)
+__device__ __forceinline__ double neg_recip(double d, double r)
+{
+    r = __builtin_fma(__builtin_fma(d, r, 1.0), r, r);
+    return __builtin_fma(__builtin_fma(d, r, 1.0), r, r);
+}
+__device__ __forceinline__ float neg_recip(float d, float r) { return __builtin_fmaf(__builtin_fmaf(d, r, 1.0f), r, r); }
+__device__ __forceinline__ double rcp_estimate(double d) { return __builtin_amdgcn_rcp(d); }
+__device__ __forceinline__ float rcp_estimate(float d) { return __builtin_amdgcn_rcpf(d); }
+
+// Elimination of a 16 x 16 block from step J on, lane = row r: e[k] = A[r][k], w[q] = columns krow(l, q)
+// of the unit matrix, nr = -1 / d_J.  Afterwards e[k] = L[r][k] d_k for k < r and d_r for k = r, w holds
+// the inverse of the unit lower factor, and dsel[v] = 1 / d_k of k = krow(l, v).  A step is a
+// reciprocal, a multiply and 19 - J multiply-adds.  Rows up to J take the update of e too (their entries
+// right of the diagonal are not read again), but not that of w.
+template <int J, typename C>
+__device__ __forceinline__ void eliminate(C (&e)[kQ], C (&w)[4], C (&dsel)[4], int r, int lk, C nr)
+{
+    constexpr int v = sizeof(C) == 8 ? J / 4 : J % 4, grp = sizeof(C) == 8 ? J % 4 : J / 4;  // krow(l, v) = J
+    if constexpr (J + 1 < kQ) {
+        const C m = e[J] * nr;
+        const C mw = r > J ? m : C(0);
+        C est;
+        const C d = elim_step<J>(e, w, m, mw, est);
+        const C next = neg_recip(d, est);
+        dsel[v] = lk == grp ? -nr : dsel[v];
+        eliminate<J + 1, C>(e, w, dsel, r, lk, next);
+    } else {
+        dsel[v] = lk == grp ? -nr : dsel[v];
+    }
+}
+
+// What the row solves of a panel need beside its factored block, per band: the operands of the four
+// 16 x 16 inverses (step s of sub-block c at [(4 c + s) * 64 + lane]), then 1 / d of the 64 columns.
+constexpr int kWorkInv = 4 * 4 * 64;
+template <typename C>
+__device__ __forceinline__ C *panel_work(void *work, int band)
+{
+    return (C *)((unsigned char *)work + (size_t)band * kBandWorkBytes);
+}
+static_assert((kWorkInv + kNB) * sizeof(double) <= kBandWorkBytes, "factor workspace");
+
+// Diagonal block of the panel at c0 (64 columns, unit pivots past n): four waves, wave w owning the
+// 16-row strip w (tiles (w, 0..w)).  With `update`, the block first takes the rank-64 update of the
+// panel at c0 - 64, whose 64 x 64 operand block goes through LDS (one memory latency for the whole
+// block).  Then for c = 0..3: wave c factors tile (c, c) by rows; the strips below solve their tile
+// (i, c) against it (one product with the 16 x 16 inverse) and update their remaining tiles.  The
+// inverses are of 16 x 16 unit lower blocks only: between sub-blocks the solve is a substitution.
+// Bound by its chain: 64 pivots of about 100 cycles each (reciprocal and broadcasts), four LDS round
+// trips and product chains between the sub-blocks.
+template <typename C>
+struct DiagLds {
+    C panel[kNB * kNB];   // L[c0 + row][c0 - 64 + k] at k * 64 + (row ^ 16 (k % 4))
+    C nd[kNB];            // -d of the previous panel
+    C tr[kQ * (kQ + 1)];  // a diagonal tile on its way to lane = row
+    C inv[4 * 64];        // sub-block c: operands of the inverse
+    C dinv[4 * 64];       // and 1 / d, by (register, lane)
+    C dk[kNB];            // 1 / d of the block
+    C l[4][4 * 64];       // the strips' L[i][c]: operands of the other strips' updates
+    int bad;
+};
+
 template <typename T, typename C>
-__device__ __forceinline__ void diag_factor(C *blk, C *dval, C *dinv, int w, int col0, int *info, bool clear)
+__device__ __forceinline__ void diag_panel(const BandDesc &d, int c0, bool update, C *work)
 {
-    const int lane = threadIdx.x & 63;
-    const int r = lane & (kNS - 1);
-    C a[kNS];
-#pragma unroll
-    for (int kk = 0; kk < kNS; ++kk) a[kk] = blk[kk * kNS + r];
-    int bad = 0;
-#pragma unroll
-    for (int jj = 0; jj < kNS; ++jj) {
-        const C cv = a[jj];  // A[r][jj]; lane kk's value is A[kk][jj]
-        // the whole column first, into distinct scalar registers: the reads issue back to back and
-        // the reciprocal overlaps them, instead of a read / wait / multiply-add triple per entry
-        C col[kNS];
-#pragma unroll
-        for (int kk = jj; kk < kNS; ++kk) col[kk] = bcast(cv, kk);
-        const C djj = col[jj];
-        if (jj < w && bad == 0 && (djj == C(0) || !isfinite(djj) || !isfinite((double)(T)djj))) bad = col0 + jj + 1;
-        const C l = cv * (C(1) / djj);
-#pragma unroll
-        for (int kk = jj + 1; kk < kNS; ++kk) a[kk] -= l * col[kk];
-        if (r > jj) a[jj] = l;
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (lane == 0 && info && (clear || (bad != 0 && *info == 0))) *info = bad;
-    C ar = C(0);  // a[r] by selects: a lane-dependent index would put a[] in scratch memory
-#pragma unroll
-    for (int kk = 0; kk < kNS; ++kk) ar = kk == r ? a[kk] : ar;
-    dval[r] = ar;
-    dinv[r] = C(1) / ar;
-#pragma unroll
-    for (int kk = 0; kk < kNS; ++kk) blk[kk * kNS + r] = kk <= r ? a[kk] : C(0);
-}
-
-// Sub-panel at column cs (width ws = min(32, n - cs)): factor the diagonal block in LDS (wave 0),
-// write it back, and solve the rows below it within the band (row-wise TRSM).  Rows cs+32 ..
-// cs+63 of the result are also left in `lnext` (for the next sub-panel's update).  The panel's
-// arithmetic is FP64 for both storage precisions (an FP32 band is read, and its factor written,
-// in FP32; the trailing update, almost all of the work, runs in the storage precision).
-template <typename T>
-__device__ __forceinline__ void sub_panel(const BandDesc &d, __amdgpu_buffer_rsrc_t rs, int cs, double *blk, double *dinv,
-                                          double *dval, double (*lnext)[kNS + 1])
-{
-    const int n = d.n, bw = d.bw;
-    const int w = min(kNS, n - cs), nr = min(n - cs, w + bw);
-    const unsigned ldu = (unsigned)bw + 1;
-    constexpr unsigned es = sizeof(T);
-    const int tid = threadIdx.x, wave = tid >> 6;
-    constexpr int kQ = kNS * kNS / kPT;
-    // stage the diagonal block (unit pivots pad the last panel)
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) {
-        const int idx = tid + kPT * q, kk = idx / kNS, r = idx % kNS;
-        const bool ok = r >= kk && r < w && r - kk <= bw;
-        const double v = (double)load_if<T>(ok, rs, ((unsigned)(cs + kk) * ldu + (unsigned)(r - kk)) * es);
-        blk[idx] = (r >= w && r == kk) ? 1.0 : v;
-    }
-    __syncthreads();
-    if (wave == 0) diag_factor<T, double>(blk, dval, dinv, w, cs, d.info, cs == 0);
-    __syncthreads();
-    // write the factored block back (L below the diagonal, D on it)
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) {
-        const int idx = tid + kPT * q, kk = idx / kNS, r = idx % kNS;
-        const bool ok = r >= kk && r < w && r - kk <= bw;
-        store_if<T>(ok, rs, ((unsigned)(cs + kk) * ldu + (unsigned)(r - kk)) * es, (T)blk[idx]);
-    }
-    // TRSM: row r of the sub-panel, L[r][0:32] = A[r][0:32] (D L_dd^T)^-1
-    for (int r = w + tid; r < nr; r += kPT) {
-        double a[kNS];
-#pragma unroll
-        for (int kk = 0; kk < kNS; ++kk) {
-            const bool ok = kk < w && r - kk <= bw;
-            a[kk] = (double)load_if<T>(ok, rs, ((unsigned)(cs + kk) * ldu + (unsigned)(r - kk)) * es);
-        }
-#pragma unroll
-        for (int kk = 0; kk < kNS; ++kk) {
-            const double t = a[kk];  // = L[r][kk] d_kk
-#pragma unroll
-            for (int jj = kk + 1; jj < kNS; ++jj) a[jj] -= t * blk[kk * kNS + jj];
-            a[kk] = t * dinv[kk];
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int kk = 0; kk < kNS; ++kk) {
-            const bool ok = kk < w && r - kk <= bw;
-            store_if<T>(ok, rs, ((unsigned)(cs + kk) * ldu + (unsigned)(r - kk)) * es, (T)a[kk]);
-        }
-        if (r >= kNS && r < 2 * kNS) {
-#pragma unroll
-            for (int kk = 0; kk < kNS; ++kk) lnext[r - kNS][kk] = a[kk];
-        }
-    }
-}
-
-// Panel of 64 columns at c0 as two sub-panels of 32: the second sub-panel's columns take the
-// first one's rank-32 update (A[r][j] -= sum_k L[r][k] d_k L[j][k]) between the two.
-template <typename T>
-__device__ __forceinline__ void panel_general(const BandDesc &d, int c0)
-{
-    __shared__ double blk[kNS * kNS];     // blk[kk*32 + r] = A / L[cs+r][cs+kk] for r >= kk, zero above
-    __shared__ double dinv[kNS], dval[kNS];
-    __shared__ double lnext[kNS][kNS + 1];  // L[c0+32+j][c0+k] of the first sub-panel
-    const int n = d.n, bw = d.bw;
-    if (c0 >= n) return;
-    T *fac = (T *)d.fac;
-    const unsigned ldu = (unsigned)bw + 1;
-    constexpr unsigned es = sizeof(T);
-    const __amdgpu_buffer_rsrc_t rs = band_rsrc(fac, (unsigned)((size_t)n * ldu * es));
-    sub_panel<T>(d, rs, c0, blk, dinv, dval, lnext);
-    const int c1 = c0 + kNS;
-    if (c1 >= n) return;  // uniform: the last panel has one sub-panel
-    const int w0 = kNS, w1 = min(kNS, n - c1), nr0 = min(n - c0, w0 + bw);
-    __syncthreads();  // lnext complete, TRSM stores visible
-    // update of columns c1 .. c1+w1-1, rows r (relative to c0) in [32, nr0)
-    for (int r = kNS + (int)threadIdx.x; r < nr0; r += kPT) {
-        double l[kNS];
-#pragma unroll
-        for (int kk = 0; kk < kNS; ++kk) {
-            const bool ok = r - kk <= bw;
-            l[kk] = (double)load_if<T>(ok, rs, ((unsigned)(c0 + kk) * ldu + (unsigned)(r - kk)) * es) * dval[kk];
-        }
-        for (int j = 0; j < w1; ++j) {
-            const int col = kNS + j;  // relative to c0
-            const bool ok = r >= col && r - col <= bw;
-            const unsigned off = ((unsigned)(c0 + col) * ldu + (unsigned)(r - col)) * es;
-            double acc = (double)load_if<T>(ok, rs, off);
-#pragma unroll
-            for (int kk = 0; kk < kNS; ++kk) acc -= l[kk] * lnext[j][kk];
-            store_if<T>(ok, rs, off, (T)acc);
-        }
-    }
-    __syncthreads();  // updated columns visible to the second sub-panel's loads
-    sub_panel<T>(d, rs, c1, blk, dinv, dval, lnext);
-}
-
-// Panel of 64 columns at c0 with every panel row below the first diagonal block owned by one
-// thread for the whole kernel (bands with bw <= kPT - 32): the thread loads its row's 64 entries
-// once (in two halves, each just before use), solves the first sub-panel's part (TRSM), applies the first sub-panel's
-// rank-32 update to the second part and solves that (TRSM) in registers; the two diagonal
-// blocks go through LDS.  A row's entries are read once and written once.
-template <typename T>
-__device__ __forceinline__ void panel_rows(const BandDesc &d, int c0)
-{
-    using C = T;  // arithmetic in the storage precision
     using M = Mfma16<C>;
-    __shared__ C blk1[kNS * kNS], blk2[kNS * kNS];
-    __shared__ C dval1[kNS], dinv1[kNS], dval2[kNS], dinv2[kNS];
-    __shared__ C lnext[kNS][kNS + 1];  // L[c0+32+j][c0+k] of the first sub-panel
-    __shared__ C xr[kPT / 64][64 * kXr];  // per wave: its 64 rows, first L d, then the update
+    using acc_t = typename M::acc_t;
+    __shared__ DiagLds<C> sh;
     const int n = d.n, bw = d.bw;
     if (c0 >= n) return;
-    T *fac = (T *)d.fac;
     const unsigned ldu = (unsigned)bw + 1;
     constexpr unsigned es = sizeof(T);
-    const __amdgpu_buffer_rsrc_t rs = band_rsrc(fac, (unsigned)((size_t)n * ldu * es));
-    const int tid = threadIdx.x, wave = tid >> 6;
-    const int w = min(kNB, n - c0), w1 = min(kNS, w), w2 = w - w1;
-    const int nrr = min(n - c0, kNB + bw);  // panel rows (relative to c0)
-    const int r = kNS + tid;                // this thread's row
-    const bool has_row = r < nrr;
-    constexpr int kQ = kNS * kNS / kPT;
-    // loads: the first diagonal block, and this thread's row (columns 0..63 of the panel)
+    const __amdgpu_buffer_rsrc_t rs = band_rsrc(d.fac, (unsigned)((size_t)n * ldu * es));
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int w = min(kNB, n - c0);
+    if (tid == 0) sh.bad = 0;
+    const int i = kQ * wv + li;  // this lane's row
+    constexpr int kP = kNB * kNB / (64 * kUW);
+    T pv[kP], dv = T(0);
+    if (update) {  // panel operands: lanes along a column's rows
+        const int cp = c0 - kNB;
 #pragma unroll
-    for (int q = 0; q < kQ; ++q) {
-        const int idx = tid + kPT * q, kk = idx / kNS, rr = idx % kNS;
-        const bool ok = rr >= kk && rr < w1 && rr - kk <= bw;
-        const C v = load_if<T>(ok, rs, ((unsigned)(c0 + kk) * ldu + (unsigned)(rr - kk)) * es);
-        blk1[idx] = (rr >= w1 && rr == kk) ? C(1) : v;
+        for (int q = 0; q < kP; ++q) {
+            const int k = kUW * q + wv;
+            pv[q] = load_if<T>(lane < w && lane + kNB - k <= bw, rs, ((unsigned)(cp + k) * ldu + (unsigned)(lane + kNB - k)) * es);
+        }
+        dv = load_if<T>(tid < kNB, rs, (unsigned)(cp + lane) * ldu * es);
     }
-    __syncthreads();
-    if (wave == 0) diag_factor<T, C>(blk1, dval1, dinv1, w1, c0, d.info, c0 == 0);
-    __syncthreads();
-    // the row is loaded in two halves, each just before it is needed, so that no more than 64
-    // of its values are in registers at once (and none in the factoring wave during a factor)
-    C x[kNB];
+    acc_t acc[4];
 #pragma unroll
-    for (int k = 0; k < kNS; ++k) {
-        const bool ok = has_row && k < w && r - k <= bw;
-        x[k] = load_if<T>(ok, rs, ((unsigned)(c0 + k) * ldu + (unsigned)(r - k)) * es);
-    }
-    // first diagonal block back to the band
+    for (int j = 0; j < 4; ++j) {
+        if (j > wv) continue;
 #pragma unroll
-    for (int q = 0; q < kQ; ++q) {
-        const int idx = tid + kPT * q, kk = idx / kNS, rr = idx % kNS;
-        const bool ok = rr >= kk && rr < w1 && rr - kk <= bw;
-        store_if<T>(ok, rs, ((unsigned)(c0 + kk) * ldu + (unsigned)(rr - kk)) * es, (T)blk1[idx]);
-    }
-    // TRSM of the first sub-panel: L[r][0:32] = A[r][0:32] (D L_dd^T)^-1
-#pragma unroll
-    for (int kk = 0; kk < kNS; ++kk) {
-        const C tk = x[kk];
-#pragma unroll
-        for (int jj = kk + 1; jj < kNS; ++jj) x[jj] -= tk * blk1[kk * kNS + jj];
-        x[kk] = tk * dinv1[kk];
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    {
-        const int ro = opaque(r);  // store masks recomputed, not kept from the loads
-#pragma unroll
-        for (int k = 0; k < kNS; ++k) {
-            const bool ok = has_row && k < w1 && ro - k <= bw;
-            store_if<T>(ok, rs, ((unsigned)(c0 + k) * ldu + (unsigned)(ro - k)) * es, (T)x[k]);
+        for (int v = 0; v < 4; ++v) {
+            const int col = kQ * j + M::row(lane, v);
+            const int hi = max(i, col), lo = min(i, col);  // the upper half of a diagonal tile mirrors the lower
+            const bool ok = hi < w && hi - lo <= bw;
+            const C x = (C)load_if<T>(ok, rs, ((unsigned)(c0 + lo) * ldu + (unsigned)(hi - lo)) * es);
+            acc[j][v] = (hi >= w && hi == lo) ? C(1) : x;
         }
     }
-    if (w2 <= 0) return;  // uniform: no second sub-panel
+    if (update) {
 #pragma unroll
-    for (int k = kNS; k < kNB; ++k) {
-        const bool ok = has_row && k < w && r >= k && r - k <= bw;
-        x[k] = load_if<T>(ok, rs, ((unsigned)(c0 + k) * ldu + (unsigned)(r - k)) * es);
+        for (int q = 0; q < kP; ++q) {
+            const int k = kUW * q + wv;
+            sh.panel[k * kNB + (lane ^ ((k & 3) << 4))] = (C)pv[q];
+        }
+        if (tid < kNB) sh.nd[tid] = -(C)dv;
+        lds_barrier();
+        C own[kNB / 4], nd[kNB / 4];
+#pragma unroll
+        for (int s = 0; s < kNB / 4; ++s) {
+            nd[s] = sh.nd[4 * s + lk];
+            own[s] = sh.panel[(4 * s + lk) * kNB + (i ^ (lk << 4))];
+        }
+        // wave 0 has the least of it and goes on to its diagonal tile while the others finish
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (j > wv) continue;
+#pragma unroll
+            for (int s = 0; s < kNB / 4; ++s)
+                acc[j] = M::run(nd[s] * sh.panel[(4 * s + lk) * kNB + ((kQ * j + li) ^ (lk << 4))], own[s], acc[j]);
+        }
     }
-    if (r < kNB) {
+    C lkeep[4] = {C(0), C(0), C(0), C(0)};
+    auto store_l = [&](int c, const C (&l)[4]) {
 #pragma unroll
-        for (int k = 0; k < kNS; ++k) lnext[r - kNS][k] = x[k];
-    }
-    __syncthreads();
-    // rank-32 update of the second part, x[32+j] -= S[r][j], S[r][j] = sum_k L[r][k] d_k L[32+j][k],
-    // on MFMA per wave (entries above the diagonal of rows 32..63 are updated too; never
-    // read).  The wave's rows go through its LDS region: row i of the wave holds L[r][k] d_k at
-    // xr[i*kXr + k], then S[r][j] at xr[i*kXr + j].  S^T tiles (16 j x 16 rows): A = L[32+j][k]
-    // from lnext, B = (L d)^T from the region, so that each value is read once per lane (a
-    // loop over rows with lnext broadcast to every lane costs 32 x 32 LDS broadcasts per wave).
-    {
-        C *reg = xr[wave];
-        const int lane = tid & 63, li = lane & 15, lg = lane >> 4;
+        for (int v = 0; v < 4; ++v) {
+            const int col = kQ * c + M::row(lane, v);
+            store_if<T>(i < w && i - col <= bw, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(i - col)) * es, (T)l[v]);
+        }
+    };
+    // acc[0] is the strip's tile in column c, acc[j] the one in column c + j: shifted down after every
+    // sub-block, so that the loop stays rolled (its code is fetched once, not four times)
+#pragma unroll 1
+    for (int c = 0; c < 4; ++c) {
+        C e[kQ], inv[4], dinv[4];
+        if (wv == c) {
 #pragma unroll
-        for (int k = 0; k < kNS; ++k) reg[lane * kXr + k] = x[k] * dval1[k];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-        C av[2][kNS / 4];
+            for (int v = 0; v < 4; ++v) sh.tr[M::row(lane, v) * (kQ + 1) + li] = acc[0][v];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 #pragma unroll
-        for (int jt = 0; jt < 2; ++jt)
+            for (int k = 0; k < kQ; ++k) e[k] = sh.tr[k * (kQ + 1) + li];
 #pragma unroll
-            for (int s = 0; s < kNS / 4; ++s) av[jt][s] = lnext[16 * jt + li][4 * s + lg];
-        const typename M::acc_t zero = {C(0), C(0), C(0), C(0)};
-        typename M::acc_t acc[2][4];
+            for (int q = 0; q < 4; ++q) {
+                inv[q] = M::row(lane, q) == li ? C(1) : C(0);
+                dinv[q] = C(0);
+            }
+            const C d0 = row_bcast<0>(e[0]);
+            eliminate<0, C>(e, inv, dinv, li, lk, neg_recip(d0, rcp_estimate(-d0)));
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
-            acc[0][rt] = zero;
-            acc[1][rt] = zero;
-#pragma unroll
-            for (int s = 0; s < kNS / 4; ++s) {
-                const C bv = reg[(16 * rt + li) * kXr + 4 * s + lg];
-                acc[0][rt] = M::run(av[0][s], bv, acc[0][rt]);
-                acc[1][rt] = M::run(av[1][s], bv, acc[1][rt]);
+            for (int q = 0; q < 4; ++q) {
+                sh.inv[q * 64 + lane] = inv[q];
+                sh.dinv[q * 64 + lane] = dinv[q];
+                if (li == 0) sh.dk[kQ * c + M::row(lane, q)] = dinv[q];
             }
         }
-        // lane holds S[16 rt + li][16 jt + row(lane, v)]: back to the row owners through the region
-        // (each row's B reads feed its own tiles, so they precede these writes)
+        lds_barrier();
+        acc_t x = {C(0), C(0), C(0), C(0)};
+        C lv[4];
+        if (wv > c) {
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+            for (int s = 0; s < 4; ++s) x = M::run(sh.inv[s * 64 + lane], acc[0][s], x);
 #pragma unroll
-            for (int jt = 0; jt < 2; ++jt)
+            for (int v = 0; v < 4; ++v) {
+                lv[v] = x[v] * sh.dinv[v * 64 + lane];
+                sh.l[wv][v * 64 + lane] = lv[v];
+            }
 #pragma unroll
-                for (int v = 0; v < 4; ++v) reg[(16 * rt + li) * kXr + 16 * jt + M::row(lane, v)] = acc[jt][rt][v];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            for (int j = 1; j < 4; ++j)
+                if (c + j == wv) {
 #pragma unroll
-        for (int j = 0; j < kNS; ++j) x[kNS + j] -= reg[lane * kXr + j];
+                    for (int s = 0; s < 4; ++s) acc[j] = M::run(-lv[s], x[s], acc[j]);
+                }
+        }
+        lds_barrier();
+        if (wv > c) {
+#pragma unroll
+            for (int j = 1; j < 4; ++j)
+                if (c + j < wv) {
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) acc[j] = M::run(-sh.l[c + j][s * 64 + lane], x[s], acc[j]);
+                }
+#pragma unroll
+            for (int j = 0; j < 3; ++j) acc[j] = acc[j + 1];
+            if (wv > c + 1) {
+                store_l(c, lv);
+            } else {  // its own sub-block is next: the stores follow it
+#pragma unroll
+                for (int v = 0; v < 4; ++v) lkeep[v] = lv[v];
+            }
+        } else if (wv == c) {
+            if (c > 0) store_l(c - 1, lkeep);
+            // off the chain: the factored tile and the row solves' operands to memory, the pivots' check; lane
+            // (li, lk) stores columns 4 lk .. 4 lk + 3 of its row
+            C sel[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const C lo = lk == 0 ? e[q] : e[4 + q], hi = lk == 2 ? e[8 + q] : e[12 + q];
+                sel[q] = lk < 2 ? lo : hi;
+            }
+            const int k0 = 4 * lk;
+            unsigned off = ((unsigned)(c0 + kQ * c + k0) * ldu + (unsigned)(li - k0)) * es;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int k = k0 + q;
+                const C val = k == li ? sel[q] : sel[q] * sh.dk[kQ * c + k];
+                store_if<T>(k <= li && i < w && li - k <= bw, rs, off, (T)val);
+                off += (ldu - 1) * es;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) work[(4 * c + q) * 64 + lane] = inv[q];
+            if (lane < kQ) work[kWorkInv + kQ * c + lane] = sh.dk[kQ * c + lane];
+            const C d01 = (li & 1) ? sel[1] : sel[0], d23 = (li & 1) ? sel[3] : sel[2];
+            const C dr = (li & 2) ? d23 : d01;  // the pivot of row li, in the lanes lk = li / 4
+            const bool bad = lk == (li >> 2) && i < w && (dr == C(0) || !isfinite(dr) || !isfinite((double)(T)dr));
+            const unsigned long long bm = __ballot(bad);
+            // (these lanes are in the order of their rows)
+            if (lane == 0 && bm != 0 && sh.bad == 0) sh.bad = c0 + kQ * c + ((__ffsll((long long)bm) - 1) & (kQ - 1)) + 1;
+        }
     }
-    // second diagonal block (rows 32..63) through LDS, unit pivots past w2
-    if (r < kNB) {
-        const int rr = r - kNS;
-#pragma unroll
-        for (int kk = 0; kk < kNS; ++kk)
-            blk2[kk * kNS + rr] = rr >= w2 ? (rr == kk ? C(1) : C(0)) : (kk <= rr ? x[kNS + kk] : C(0));
-    }
-    __syncthreads();
-    if (wave == 0) diag_factor<T, C>(blk2, dval2, dinv2, w2, c0 + kNS, d.info, false);
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) {
-        const int idx = tid + kPT * q, kk = idx / kNS, rr = idx % kNS;
-        const bool ok = rr >= kk && rr < w2 && rr - kk <= bw;
-        store_if<T>(ok, rs, ((unsigned)(c0 + kNS + kk) * ldu + (unsigned)(rr - kk)) * es, (T)blk2[idx]);
-    }
-    if (r < kNB) return;  // rows of the second diagonal block are done
-    // TRSM of the second sub-panel
-#pragma unroll
-    for (int kk = 0; kk < kNS; ++kk) {
-        const C tk = x[kNS + kk];
-#pragma unroll
-        for (int jj = kk + 1; jj < kNS; ++jj) x[kNS + jj] -= tk * blk2[kk * kNS + jj];
-        x[kNS + kk] = tk * dinv2[kk];
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    const int ro = opaque(r);
-#pragma unroll
-    for (int j = 0; j < kNS; ++j) {
-        const int col = kNS + j;
-        const bool ok = has_row && j < w2 && ro - col <= bw;
-        store_if<T>(ok, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(ro - col)) * es, (T)x[col]);
+    lds_barrier();  // sh.bad of every sub-block
+    if (tid == 0 && d.info) {
+        if (c0 == 0)
+            *d.info = sh.bad;
+        else if (sh.bad != 0 && *d.info == 0)
+            *d.info = sh.bad;
     }
 }
+
+// Row tile t of the panel at c0 (rows c0 + 64 + 16 t .. + 15, its 64 columns) against the factored
+// diagonal block, one wave: X = A L^-T by blocks of 16 columns (substitution between them, the 16 x 16
+// inverse within), L = X D^-1.  40 MFMAs in one chain; the operands of the diagonal block are read
+// from L2 by every wave, which spreads a band's rows over as many CUs as there are.
+template <typename T, typename C>
+__device__ __forceinline__ void solve_rows(const BandDesc &d, int c0, int t0, int ntile, const C *work)
+{
+    using M = Mfma16<C>;
+    using acc_t = typename M::acc_t;
+    const int n = d.n, bw = d.bw;
+    const int nr = min(n - c0, kNB + bw);  // panel rows (relative to c0); the panel is full: n > c0 + 64
+    if (n <= c0 + kNB || kNB + kQ * t0 >= nr) return;
+    const unsigned ldu = (unsigned)bw + 1;
+    constexpr unsigned es = sizeof(T);
+    const __amdgpu_buffer_rsrc_t rs = band_rsrc(d.fac, (unsigned)((size_t)n * ldu * es));
+    const int lane = threadIdx.x & 63, li = lane & 15;
+    C inv[4][4], dinv[4][4], l[4][4][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            inv[c][s] = work[(4 * c + s) * 64 + lane];
+            dinv[c][s] = work[kWorkInv + kQ * c + M::row(lane, s)];
+#pragma unroll
+            for (int e = 0; e < c; ++e) {  // L[16 c + li][16 e + krow]
+                const int row = kQ * c + li, col = kQ * e + M::row(lane, s);
+                l[c][e][s] = -(C)load_if<T>(row - col <= bw, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(row - col)) * es);
+            }
+        }
+    for (int t = t0; t < t0 + ntile; ++t) {
+        const int r = kNB + kQ * t + li;
+        if (kNB + kQ * t >= nr) break;  // uniform
+        acc_t a[4], x[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int col = kQ * c + M::row(lane, v);
+                a[c][v] = (C)load_if<T>(r < nr && r - col <= bw, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(r - col)) * es);
+            }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+#pragma unroll
+            for (int e = 0; e < c; ++e)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) a[c] = M::run(l[c][e][s], x[e][s], a[c]);
+            const acc_t zero = {C(0), C(0), C(0), C(0)};
+            x[c] = zero;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) x[c] = M::run(inv[c][s], a[c][s], x[c]);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int col = kQ * c + M::row(lane, v);
+                store_if<T>(r < nr && r - col <= bw, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(r - col)) * es,
+                            (T)(x[c][v] * dinv[c][v]));
+            }
+    }
+}
+
 
 // lower-triangle block index p -> (bi, bj), bj <= bi
 __device__ __forceinline__ void tri_decode(int p, int &bi, int &bj)
@@ -370,8 +370,15 @@ __device__ __forceinline__ void tri_decode(int p, int &bi, int &bj)
 }
 
 // Parts of a step's trailing update (32 x 32 blocks (bi, bj), bj <= bi, of the window):
-// kAll every block; kNext block columns 0 and 1 (the next panel's columns); kRest the others.
+// kAll every block; kNext block columns 0 and 1 (the next panel's columns); kRest the others.  The
+// three blocks of the next diagonal block, (0,0), (1,0) and (1,1), are left out of kAll and kNext:
+// the workgroup that factors it updates it (diag_panel).
 enum TrailPart { kAll = 0, kNext = 1, kRest = 2 };
+__host__ __device__ inline int trail_blocks(int nbk, int part)
+{
+    const int tail = nbk > 2 ? nbk - 2 : 0;  // block rows below the diagonal block
+    return part == kRest ? tail * (tail + 1) / 2 : part == kNext ? 2 * tail : tail * (tail + 1) / 2 + 2 * tail;
+}
 
 // Blocks p[0] < p[1] < ... of the given part (wave-uniform), computed together (independent
 // accumulators, the loads of all of them in flight at once): A[i][j] -= sum_k L[i][k] d_k L[j][k]
@@ -387,8 +394,7 @@ __device__ __forceinline__ void trailing_blocks(const BandDesc &d, int c0, int p
     if (c0 >= n) return;
     const int w = min(kNB, n - c0), nr = min(n - c0, w + bw);
     const int nbk = (nr - w + 31) / 32;
-    const int nblock = part == kAll ? nbk * (nbk + 1) / 2 : part == kNext ? min(nbk, 2) * nbk - (nbk >= 2 ? 1 : 0)
-                                                                          : (nbk > 2 ? (nbk - 2) * (nbk - 1) / 2 : 0);
+    const int nblock = trail_blocks(nbk, part);
     if (p[0] >= nblock) return;
     T *fac = (T *)d.fac;
     const unsigned ldu = (unsigned)bw + 1;
@@ -407,10 +413,10 @@ __device__ __forceinline__ void trailing_blocks(const BandDesc &d, int c0, int p
         const int q = valid[s] ? p[s] : p[0];
         int bi, bj;
         if (part == kNext) {
-            bj = q < nbk ? 0 : 1;
-            bi = bj == 0 ? q : q - nbk + 1;
+            bj = q < nbk - 2 ? 0 : 1;
+            bi = 2 + (bj == 0 ? q : q - (nbk - 2));
         } else {
-            tri_decode(q, bi, bj);
+            tri_decode(part == kAll ? q + 3 : q, bi, bj);
             if (part == kRest) {
                 bi += 2;
                 bj += 2;
@@ -470,15 +476,11 @@ __device__ __forceinline__ void trailing_blocks(const BandDesc &d, int c0, int p
                 for (int v = 0; v < 4; ++v) store_vs<T>(rs, off[s][a][b][v], 0, cur[s][a][b][v]);
 }
 
-// Panel step at c0 of every band in the grid (one workgroup per band).  kRows: the register-resident
-// form (band widths up to kPT - 32).
-template <typename T, bool kRows>
-__global__ __launch_bounds__(kPT) void k_band_panel(const BandDesc *descs, int c0)
+// Diagonal block at column 0 of every band (the later ones are factored by the trailing launches).
+template <typename T, typename C>
+__global__ __launch_bounds__(64 * kUW) void k_band_diag(const BandDesc *descs, void *work)
 {
-    if (kRows)
-        panel_rows<T>(descs[blockIdx.x], c0);
-    else
-        panel_general<T>(descs[blockIdx.x], c0);
+    diag_panel<T, C>(descs[blockIdx.x], 0, false, panel_work<C>(work, (int)blockIdx.x));
 }
 
 // XCD-aware assignment of a launch's workgroups to (band, index within the band).  Workgroups are
@@ -506,44 +508,59 @@ inline unsigned band_grid(int active, int wg)
     return (unsigned)(active < kXcds ? active * wg : ((active + kXcds - 1) / kXcds) * kXcds * wg);
 }
 
-// One part of the trailing update at c0, kUW blocks (one per wave) per workgroup
-template <typename T>
-__global__ __launch_bounds__(64 * kUW) void k_band_trailing(const BandDesc *descs, int c0, int wg_per_band, int part,
-                                                            int active)
+// Rows of the panel at c0, kUW waves per workgroup and `tiles` 16-row tiles per wave
+template <typename T, typename C>
+__global__ __launch_bounds__(64 * kUW) void k_band_rows(const BandDesc *descs, void *work, int c0, int wg_per_band, int tiles,
+                                                        int active)
 {
     int band, local;
     if (!band_of_workgroup((int)blockIdx.x, active, wg_per_band, band, local)) return;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    solve_rows<T, C>(descs[band], c0, (local * kUW + wave) * tiles, tiles, panel_work<C>(work, band));
+}
+
+// One part of the trailing update at c0, kUW blocks (one per wave) per workgroup; workgroups
+// [0, ndiag) update and factor the next diagonal block of their band.  They hold the step's longest
+// chain, so they are dispatched first.  (The update part starts at workgroup `pad`, ndiag rounded up to
+// a multiple of the XCD count, so that its XCD-aware mapping lines up with the first part's.)
+template <typename T, typename C>
+__global__ __launch_bounds__(64 * kUW) void k_band_trailing(const BandDesc *descs, void *work, int c0, int ndiag, int pad,
+                                                            int wg_per_band, int part, int active)
+{
+    const int b = (int)blockIdx.x;
+    if (b < ndiag) {
+        diag_panel<T, C>(descs[b], c0 + kNB, true, panel_work<C>(work, b));
+        return;
+    }
+    if (b < pad) return;
+    int band, local;
+    if (!band_of_workgroup(b - pad, active, wg_per_band, band, local)) return;
     const int p[1] = {__builtin_amdgcn_readfirstlane((int)(local * kUW + (threadIdx.x >> 6)))};
     trailing_blocks<T, 1>(descs[band], c0, part, p);
 }
 
-// Lookahead step: workgroups [0, npanel) factor the panel at c0 + NB of their band while the others
-// apply the rest of the trailing update at c0 (block columns 2 and up): AW waves of each of these
-// workgroups take NBLK blocks each, the other waves leave at once.  The two parts touch disjoint
-// columns: the panel reads and writes columns [c0 + NB, c0 + 2 NB), already updated by the kNext
-// part; the rest of the update reads the panel at c0 and writes columns from c0 + 2 NB on.
-// (The update part starts at workgroup `pad`, npanel rounded up to a multiple of the XCD count,
-// so that its XCD-aware mapping lines up with the panels' workgroups.)
-template <typename T, bool kRows, int AW, int NBLK>
-__global__ __launch_bounds__(kPT) void k_band_step(const BandDesc *descs, int c0, int npanel, int wg_per_band,
-                                                    int pad, int active)
+// Lookahead step: the first workgroups (nrow per band, padded to `pad`) solve the rows of the panel at
+// c0 + NB while the others apply the rest of the trailing update at c0 (block columns 2 and up), NBLK
+// blocks per wave.  The two parts touch disjoint columns: the rows read and write columns
+// [c0 + NB, c0 + 2 NB), already updated by the kNext part; the rest of the update reads the panel at
+// c0 and writes columns from c0 + 2 NB on.
+template <typename T, typename C, int NBLK>
+__global__ __launch_bounds__(kPT) void k_band_step(const BandDesc *descs, void *work, int c0, int nrow, int tiles, int np, int pad,
+                                                   int wg_per_band, int active)
 {
     const int b = (int)blockIdx.x;
-    if (b < npanel) {
-        if (kRows)
-            panel_rows<T>(descs[b], c0 + kNB);
-        else
-            panel_general<T>(descs[b], c0 + kNB);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    constexpr int kW = kPT / 64;
+    int band, local;
+    if (b < pad) {
+        if (!band_of_workgroup(b, np, nrow, band, local)) return;
+        solve_rows<T, C>(descs[band], c0 + kNB, (local * kW + wave) * tiles, tiles, panel_work<C>(work, band));
         return;
     }
-    if (b < pad) return;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    if (wave >= AW) return;
-    int band, local;
     if (!band_of_workgroup(b - pad, active, wg_per_band, band, local)) return;
     int p[NBLK];
 #pragma unroll
-    for (int s = 0; s < NBLK; ++s) p[s] = (local * NBLK + s) * AW + wave;
+    for (int s = 0; s < NBLK; ++s) p[s] = (local * NBLK + s) * kW + wave;
     trailing_blocks<T, NBLK>(descs[band], c0, kRest, p);
 }
 
@@ -593,13 +610,13 @@ __global__ __launch_bounds__(1024) void k_pivot_stats(const BandDesc *descs)
 }
 
 // Factor schedules (every one gives the same result bit for bit):
-//   0 plain: panel, then the whole trailing update, per step;
-//   1, 2 lookahead: per step the next panel's columns first (kNext), then the next panel together
-//   with the rest of the update (k_band_step) with AW waves x NBLK blocks per workgroup:
-//   1: 8 x 1, 2: 8 x 2 (more blocks in flight per wave).
-// The lookahead takes the rest of the update off the panel's critical path but runs it at the
-// panel kernel's register budget (2 waves per SIMD); which one is faster depends on the number
-// and shape of the bands, so the autotuner picks per shape bucket (KSH_LOOKAHEAD=k forces k).
+//   0 plain: per step the panel's rows, then the whole trailing update, whose first workgroups update
+//   and factor the next diagonal block;
+//   1, 2 lookahead: per step the next panel's columns (kNext, with the next diagonal block), then the
+//   next panel's rows together with the rest of the update (k_band_step), 1 or 2 blocks per wave.
+// Plain has the rest of the update beside the diagonal block's chain, lookahead beside the rows; which
+// one is faster depends on the number and shape of the bands, so the autotuner picks per shape
+// bucket (KSH_LOOKAHEAD=k forces k).
 constexpr int kSchedules = 3;
 
 int schedule_forced()
@@ -610,62 +627,86 @@ int schedule_forced()
     return v >= 0 && v < kSchedules ? v : -1;
 }
 
-template <typename T, bool kRows, int AW, int NBLK>
-void run_lookahead(hipStream_t s, const BandDesc *d_descs, const std::vector<int> &ns, int maxbw)
+// bands (orders descending) with a column c
+inline int active_at(const std::vector<int> &ns, int c)
 {
-    const int nbands = (int)ns.size();
-    const int nbk = (maxbw + 31) / 32;
-    auto active_at = [&](int c0) {
-        int a = nbands;
-        while (a > 0 && ns[a - 1] <= c0) --a;
-        return a;
-    };
-    const int wg1 = std::max(1, ((nbk >= 2 ? 2 * nbk - 1 : nbk) + kUW - 1) / kUW);
-    const int nrest = nbk > 2 ? (nbk - 2) * (nbk - 1) / 2 : 0;
-    const int wg2 = (nrest + AW * NBLK - 1) / (AW * NBLK);
-    hipLaunchKernelGGL((k_band_panel<T, kRows>), dim3((unsigned)nbands), dim3(kPT), 0, s, d_descs, 0);
-    for (int c0 = 0; c0 < ns[0]; c0 += kNB) {
-        const int active = active_at(c0), np = active_at(c0 + kNB);
-        hipLaunchKernelGGL(k_band_trailing<T>, dim3(band_grid(active, wg1)), dim3(64 * kUW), 0, s, d_descs, c0, wg1,
-                           (int)kNext, active);
-        const int pad = wg2 > 0 && active >= kXcds ? (np + kXcds - 1) / kXcds * kXcds : np;
-        const int grid = pad + (wg2 > 0 ? (int)band_grid(active, wg2) : 0);
+    int a = (int)ns.size();
+    while (a > 0 && ns[a - 1] <= c) --a;
+    return a;
+}
+
+// 16-row tiles per wave of the row solves: one while the tiles leave the chip room (the solve is one
+// chain of 40 MFMAs per tile), two when there are enough bands to fill it (the operands of the diagonal
+// block, 20 KB in FP64, are then read once for two tiles of 8 KB)
+inline int row_tiles(int active) { return active >= 32 ? 2 : 1; }
+
+template <typename T, typename C, int NBLK>
+void run_lookahead(hipStream_t s, const BandDesc *d_descs, void *work, const std::vector<int> &ns, int maxbw)
+{
+    constexpr int kW = kPT / 64;
+    const int nbk = (maxbw + 31) / 32, ntile = (maxbw + kQ - 1) / kQ;
+    const int wg1 = (trail_blocks(nbk, kNext) + kUW - 1) / kUW;
+    const int wg2 = (trail_blocks(nbk, kRest) + kW * NBLK - 1) / (kW * NBLK);
+    int np = active_at(ns, kNB);  // bands with rows below the current panel
+    if (np == 0) return;
+    {
+        const int tiles = row_tiles(np), wg = (ntile + kUW * tiles - 1) / (kUW * tiles);
+        if (wg > 0)
+            hipLaunchKernelGGL((k_band_rows<T, C>), dim3(band_grid(np, wg)), dim3(64 * kUW), 0, s, d_descs, work, 0, wg, tiles, np);
+    }
+    for (int c0 = 0; np > 0; c0 += kNB) {
+        const int pad1 = np >= kXcds ? (np + kXcds - 1) / kXcds * kXcds : np;
+        hipLaunchKernelGGL((k_band_trailing<T, C>), dim3((unsigned)pad1 + (wg1 > 0 ? band_grid(np, wg1) : 0u)), dim3(64 * kUW), 0, s,
+                           d_descs, work, c0, np, pad1, wg1, (int)kNext, np);
+        const int np1 = active_at(ns, c0 + 2 * kNB);
+        const int tiles = row_tiles(np1), nrow = (ntile + kW * tiles - 1) / (kW * tiles);
+        int pad = np1 > 0 && nrow > 0 ? (int)band_grid(np1, nrow) : 0;
+        if (np >= kXcds) pad = (pad + kXcds - 1) / kXcds * kXcds;
+        const unsigned grid = (unsigned)pad + (wg2 > 0 ? band_grid(np, wg2) : 0u);
         if (grid > 0)
-            hipLaunchKernelGGL((k_band_step<T, kRows, AW, NBLK>), dim3((unsigned)grid), dim3(kPT), 0, s, d_descs, c0, np,
-                               wg2, pad, active);
+            hipLaunchKernelGGL((k_band_step<T, C, NBLK>), dim3(grid), dim3(kPT), 0, s, d_descs, work, c0, nrow, tiles, np1, pad, wg2,
+                               np);
+        np = np1;
     }
 }
 
-template <typename T, bool kRows>
-void run_tiled_sched(hipStream_t s, const BandDesc *d_descs, const std::vector<int> &ns, int maxbw, int sched)
+template <typename T, typename C>
+void run_tiled_sched(hipStream_t s, const BandDesc *d_descs, void *work, const std::vector<int> &ns, int maxbw, int sched)
 {
     // ns: orders of the bands, descending (the device array is in the same order)
     const int nbands = (int)ns.size();
+    hipLaunchKernelGGL((k_band_diag<T, C>), dim3((unsigned)nbands), dim3(64 * kUW), 0, s, d_descs, work);
     if (sched == 0) {
-        const int nbk = (maxbw + 31) / 32;
-        const int wg = std::max(1, (nbk * (nbk + 1) / 2 + kUW - 1) / kUW);
-        int active = nbands;
-        for (int c0 = 0; c0 < ns[0]; c0 += kNB) {
-            while (active > 0 && ns[active - 1] <= c0) --active;
-            hipLaunchKernelGGL((k_band_panel<T, kRows>), dim3((unsigned)active), dim3(kPT), 0, s, d_descs, c0);
-            hipLaunchKernelGGL(k_band_trailing<T>, dim3(band_grid(active, wg)), dim3(64 * kUW), 0, s, d_descs, c0, wg,
-                               (int)kAll, active);
+        const int nbk = (maxbw + 31) / 32, ntile = (maxbw + kQ - 1) / kQ;
+        const int wg = (trail_blocks(nbk, kAll) + kUW - 1) / kUW;
+        int np;
+        for (int c0 = 0; (np = active_at(ns, c0 + kNB)) > 0; c0 += kNB) {
+            const int tiles = row_tiles(np), wgr = (ntile + kUW * tiles - 1) / (kUW * tiles);
+            if (wgr > 0)
+                hipLaunchKernelGGL((k_band_rows<T, C>), dim3(band_grid(np, wgr)), dim3(64 * kUW), 0, s, d_descs, work, c0, wgr, tiles, np);
+            const int pad = np >= kXcds ? (np + kXcds - 1) / kXcds * kXcds : np;
+            hipLaunchKernelGGL((k_band_trailing<T, C>), dim3((unsigned)pad + (wg > 0 ? band_grid(np, wg) : 0u)), dim3(64 * kUW), 0, s,
+                               d_descs, work, c0, np, pad, wg, (int)kAll, np);
         }
     } else if (sched == 1) {
-        run_lookahead<T, kRows, 8, 1>(s, d_descs, ns, maxbw);
+        run_lookahead<T, C, 1>(s, d_descs, work, ns, maxbw);
     } else {
-        run_lookahead<T, kRows, 8, 2>(s, d_descs, ns, maxbw);
+        run_lookahead<T, C, 2>(s, d_descs, work, ns, maxbw);
     }
     hipLaunchKernelGGL(k_pivot_stats<T>, dim3((unsigned)nbands), dim3(1024), 0, s, d_descs);
 }
 
+// Arithmetic of the panel (diagonal block and rows): the storage precision up to half-width kPanelBw; an
+// FP32 factor of a wider band has its panel in FP64 (longer sums per entry).
+constexpr int kPanelBw = 480;
 template <typename T>
 void run_tiled(hipStream_t s, const BandDesc *d_descs, const std::vector<int> &ns, int maxbw, int sched)
 {
-    if (maxbw + kNS <= kPT)
-        run_tiled_sched<T, true>(s, d_descs, ns, maxbw, sched);
+    void *work = (unsigned char *)const_cast<BandDesc *>(d_descs) + factor_desc_offset(ns.size());
+    if (maxbw <= kPanelBw)
+        run_tiled_sched<T, T>(s, d_descs, work, ns, maxbw, sched);
     else
-        run_tiled_sched<T, false>(s, d_descs, ns, maxbw, sched);
+        run_tiled_sched<T, double>(s, d_descs, work, ns, maxbw, sched);
 }
 
 // Captured launch sequences of factor calls (opt-in: KSH_GRAPHS=1).  A call's sequence (about

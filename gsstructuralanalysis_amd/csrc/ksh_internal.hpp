@@ -197,7 +197,8 @@ struct BandDesc {
 int band_factor_batch(hipStream_t s, void *d_descs, const std::vector<BandDescHost> &h, int prec,
                       const char *prof_name = nullptr);
 // factor of a batch of bands over the whole GPU (ksh_factor_tiled.hip): panel steps of two
-// launches covering every band still active; d_descs holds h.size() device BandDescs
+// launches covering every band still active; d_descs holds h.size() device BandDescs and, behind them,
+// the panel workspaces: factor_desc_bytes(h.size()) in all
 int band_factor_tiled_batch(hipStream_t s, void *d_descs, const std::vector<BandDescHost> &h, int prec);
 // batched refinement: r = b - K x with norms (||r||^2, ||b||^2), then x += r on active matrices
 struct RefDesc {
@@ -221,6 +222,10 @@ int ensure_fac64(Matrix &K);
 int ensure_rc64(Matrix &K);
 int band_solve_batch(hipStream_t s, void *d_descs, const std::vector<BandDescHost> &h, int prec);
 constexpr size_t kBandDescBytes = 48;
+// panel workspace of one band of a factor call (operands of the row solves), behind the descriptors
+constexpr size_t kBandWorkBytes = 8704;
+inline size_t factor_desc_offset(size_t n) { return (n * kBandDescBytes + 255) / 256 * 256; }
+inline size_t factor_desc_bytes(size_t n) { return factor_desc_offset(n) + n * kBandWorkBytes; }
 int band_solve(Matrix &K, const void *fac, int prec, double *x_dev);
 // solve of one large band over many workgroups (ksh_solve_tiled.hip); z: n doubles of workspace;
 // bar: 3 device unsigneds for the one-launch form's grid barrier (nullptr: stepped launches)
