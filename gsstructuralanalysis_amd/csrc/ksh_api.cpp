@@ -167,7 +167,7 @@ void destroy_matrix(Matrix *K)
         (void)hipEventDestroy(K->rc_done);
         K->rc_done = nullptr;
     }
-    void *ptrs[] = {K->ab, K->fac, K->fac64, K->rc64, K->u_at, K->work, K->flag, K->red, K->desc};
+    void *ptrs[] = {K->ab, K->fac, K->fac64, K->rc64, K->u_at, K->work, K->flag, K->red, K->desc, K->team_ws};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
 }

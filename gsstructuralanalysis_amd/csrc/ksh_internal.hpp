@@ -160,6 +160,7 @@ struct Matrix {
     int *flag = nullptr;           // small device int buffer
     void *desc = nullptr;          // device descriptor of this band for batched kernels (one BandDesc)
     double *red = nullptr;         // reduction scratch
+    void *team_ws = nullptr;       // team solve workspace (allocated by the first solve that uses it)
 };
 
 // kernels / launchers (ksh_assembly.hip, ksh_band.hip)
@@ -227,9 +228,19 @@ constexpr size_t kBandWorkBytes = 8704;
 inline size_t factor_desc_offset(size_t n) { return (n * kBandDescBytes + 255) / 256 * 256; }
 inline size_t factor_desc_bytes(size_t n) { return factor_desc_offset(n) + n * kBandWorkBytes; }
 int band_solve(Matrix &K, const void *fac, int prec, double *x_dev);
-// solve of one large band over many workgroups (ksh_solve_tiled.hip); z: n doubles of workspace;
-// bar: 3 device unsigneds for the one-launch form's grid barrier (nullptr: stepped launches)
-int band_solve_tiled(hipStream_t s, const void *fac, int prec, int n, int bw, double *x, double *z, unsigned *bar);
+// solve of one large band by stepped launches (ksh_solve_tiled.hip); z: n doubles of workspace
+int band_solve_tiled(hipStream_t s, const void *fac, int prec, int n, int bw, double *x, double *z);
+// solves by resident teams of workgroups (ksh_solve_team.hip); work: the sum of team_solve_bytes(n) over
+// the jobs, kept by the caller until the solve is done; d_descs: kTeamDescBytes a job (unused for one)
+struct TeamJob {
+    const void *fac;
+    int n, bw;
+    double *x;
+};
+constexpr size_t kTeamDescBytes = 80;
+size_t team_solve_bytes(int n);
+bool team_solve_takes(int n, int bw, int prec, int count);
+int team_solve(hipStream_t s, const std::vector<TeamJob> &jobs, int prec, void *work, void *d_descs);
 // path of a single-band factor / solve: 1 = multi-workgroup (tiled), 0 = one workgroup
 bool band_use_tiled_factor(int n, int bw, int prec);
 bool band_use_tiled_solve(int n, int bw, int prec);

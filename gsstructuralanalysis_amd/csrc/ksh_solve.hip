@@ -565,9 +565,10 @@ int band_solve_batch(hipStream_t s, void *d_descs, const std::vector<BandDescHos
     return KSH_SUCCESS;
 }
 
-// KSH_BAND_PATH=tiled / wg forces the multi-workgroup / one-workgroup path.  Otherwise bands
-// that the LDS-resident kernel takes stay on one workgroup; wider ones go multi-workgroup when
-// a step launch (~4 us for 64 rows) costs less than one CU streaming those rows' band entries.
+// KSH_BAND_PATH=tiled / wg forces the stepped / one-workgroup path.  Single bands that no team serves
+// (team_solve_takes, team_workspace) stay on one workgroup where the LDS-resident kernel takes them; wider
+// ones go stepped when a step launch (~4 us for 64 rows) costs less than one CU streaming those rows' band
+// entries.
 bool band_use_tiled_solve(int n, int bw, int prec)
 {
     const char *e = std::getenv("KSH_BAND_PATH");
@@ -578,14 +579,38 @@ bool band_use_tiled_solve(int n, int bw, int prec)
     return (double)(bw + 1) * es >= 3072.0;
 }
 
+// Workspace of K's team solves, allocated on first use; false where it cannot be (a capturing stream, no
+// memory left), and the other solve paths take the call
+static bool team_workspace(Matrix &K)
+{
+    if (K.team_ws) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(K.pb->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
+    if (hipMalloc(&K.team_ws, team_solve_bytes(K.n)) != hipSuccess) {
+        (void)hipGetLastError();
+        K.team_ws = nullptr;
+    }
+    return K.team_ws != nullptr;
+}
+
+static bool band_path_forced()
+{
+    const char *e = std::getenv("KSH_BAND_PATH");
+    return e && (std::strcmp(e, "tiled") == 0 || std::strcmp(e, "wg") == 0);
+}
+
 int band_solve(Matrix &K, const void *fac, int prec, double *x_dev)
 {
     Problem &pb = *K.pb;
+    if (!band_path_forced() && team_solve_takes(K.n, K.bw, prec, 1) && team_workspace(K)) {
+        ProfScope ps("band_solve", pb.stream);
+        ps.set_work(2.0 * K.n * (K.bw + 1.0) * (prec == KSH_FP64 ? 8.0 : 4.0) + 16.0 * K.n);
+        return team_solve(pb.stream, {TeamJob{fac, K.n, K.bw, x_dev}}, prec, K.team_ws, nullptr);
+    }
     if (band_use_tiled_solve(K.n, K.bw, prec)) {
         ProfScope ps("band_solve_tiled", pb.stream);
         ps.set_work(2.0 * K.n * (K.bw + 1.0) * (prec == KSH_FP64 ? 8.0 : 4.0) + 16.0 * K.n);
-        return band_solve_tiled(pb.stream, fac, prec, K.n, K.bw, x_dev, K.work + 4 * (size_t)K.n,
-                                reinterpret_cast<unsigned *>(K.flag + 1));
+        return band_solve_tiled(pb.stream, fac, prec, K.n, K.bw, x_dev, K.work + 4 * (size_t)K.n);
     }
     const size_t smem = solve_lds(K.n, K.bw, (size_t)K.n * K.ld * (prec == KSH_FP64 ? sizeof(double) : sizeof(float)), prec);
     ProfScope ps("band_solve", pb.stream);

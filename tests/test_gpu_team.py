@@ -1,0 +1,63 @@
+"""Team solves (a leader walking the chain of 64-row blocks, helpers forming the rest) at the sizes where
+they can go wrong: orders around the multiples of 64 (the smallest a team takes is 129), half-widths
+below one block, around one, two and three blocks, and wide; FP64 and FP32 factors.
+
+Checked by the backward error of the solve, ||b - K x|| <= c eps G ||x||: G, the largest entry of
+|L| |D| |L|^T of the oracle's factor, is what an unpivoted factor's solve is relative to, eps the factor's
+precision, and c = 8 bw + 64 + 512 covers one rounding per product along a band row, for the factor and
+the two sweeps, plus the 64-wide inverses and products of a block (eight of 64 terms).  And by the
+team's size changing nothing: every sum has one order, whoever forms it, so a leader alone, with one
+helper or with many gives the same bits."""
+import numpy as np
+import pytest
+
+from gsstructuralanalysis_amd import _lib as L
+from gsstructuralanalysis_amd import geometry as g
+from oracle import ok
+from oracle.ok import Oracle
+
+pytestmark = pytest.mark.gpu
+
+# (free dofs, half-width): 135 26, 180 26, 192 56, 234 65, 216 62, 255 110, 180 128, 429 128, 330 101, 432 155, 480 191,
+# 1287 869
+SHAPES = [(2, 1, 15), (2, 1, 20), (2, 6, 8), (3, 3, 12), (2, 7, 8), (2, 15, 5), (2, 18, 3), (3, 10, 10), (3, 7, 10), (3, 13, 8), (3, 17, 7),
+          (3, 140, 2)]
+
+
+def _growth(ref, n, bw):
+    """max_i sum_k L_ik^2 |d_k|, the largest entry of |L| |D| |L|^T."""
+    f = ref.ab.reshape(n, bw + 1)
+    out = np.abs(f[:, 0]).copy()
+    for k in range(n):
+        m = min(bw, n - 1 - k)
+        out[k + 1:k + 1 + m] += f[k, 1:1 + m] ** 2 * abs(f[k, 0])
+    return out.max()
+
+
+@pytest.mark.parametrize("p,nx,ny", SHAPES)
+@pytest.mark.parametrize("prec", [L.FP64, L.FP32_IR])
+def test_team_solve_at_block_edges(p, nx, ny, prec, ksh, monkeypatch):
+    from gsstructuralanalysis_amd.problem import BandMatrix, ShellProblem
+    pt = g.roof_problem(p=p, n=nx, ny=ny)
+    o = Oracle(pt)
+    print(f"[case] team solve roof p={p} {nx}x{ny} nfree={o.nfree} bw={o.bw} prec={prec}", flush=True)
+    assert o.nfree > 128
+    sp = ShellProblem(pt)
+    rng = np.random.default_rng(23)
+    Kb = o.tangent_band(rng.standard_normal(o.nfree) * 1e-4)
+    ref = ok.BandLDLT(Kb, o.nfree, o.bw)
+    A = BandMatrix(sp, precision=prec)
+    A.upload(Kb)
+    A.set_inertia_guard(0.0)
+    A.factor()
+    eps = np.finfo(np.float64 if prec == L.FP64 else np.float32).eps
+    bound = (8 * o.bw + 64 + 512) * eps * _growth(ref, o.nfree, o.bw)
+    for _ in range(2):
+        b = rng.standard_normal(o.nfree)
+        x = A.solve(b)
+        r = b - ok.band_symv(Kb, o.nfree, o.bw, x)
+        assert np.linalg.norm(r) <= bound * np.linalg.norm(x)
+        for size in ("1", "2", "5", "12"):
+            monkeypatch.setenv("KSH_TEAM", size)
+            assert np.array_equal(A.solve(b), x), size
+        monkeypatch.delenv("KSH_TEAM")
