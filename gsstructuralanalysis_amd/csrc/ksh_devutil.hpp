@@ -7,6 +7,15 @@ namespace ksh {
 
 typedef unsigned int ksh_u32x2 __attribute__((ext_vector_type(2)));
 
+// a wave-uniform pointer in scalar registers
+template <typename T>
+__device__ __forceinline__ T *uniform_ptr(T *p)
+{
+    const unsigned long long a = (unsigned long long)p;
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a), hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(a >> 32));
+    return (T *)(((unsigned long long)hi << 32) | lo);
+}
+
 // broadcast of lane `src`'s value (v_readlane: the result is wave-uniform)
 __device__ __forceinline__ double readlane_f64(double v, int src)
 {

@@ -21,11 +21,13 @@
 // The chain from one diagonal block to the next (rows of the next 64 columns, update, 64 pivots) is what
 // bounds a single band and small batches; the panel of one workgroup per band that these kernels
 // replace (diagonal blocks of 32 by v_readlane, rows by substitution) took 38 us a step in FP64 at
-// bw 326 and 107 us at bw 1166, against 16 + 6 us now, most of it the diagonal block's 12 us:
-// factors of a 32 x 32 roof 2.5 -> 1.3 ms, of the 128 x 128 plate 89 -> 17 ms.
+// bw 326 and 107 us at bw 1166, against 16 + 6 us in two launches and 14 us in one (fused schedule), most
+// of it the diagonal block's 12 us: factors of a 32 x 32 roof 2.5 -> 1.3 -> 0.8 ms, of the 128 x 128 plate
+// 89 -> 17 -> 11.8 ms.
 // Plain schedule: rows, then every block, per step.  Lookahead schedule: the blocks of the next panel's
 // columns first (k_band_trailing), then k_band_step, whose first workgroups solve the next panel's
-// rows while the others apply the remaining blocks.
+// rows while the others apply the remaining blocks.  Fused schedule: one launch a step, whose workgroups
+// solve the rows they need themselves (k_band_fused).
 // Bands are sorted by order, largest first, so a step's grids cover exactly the bands that are
 // still active.  Work per band: about n bw^2 multiply-adds; HBM traffic about 2 n bw^2 / NB
 // entries (the trailing window of a step, read and written).
@@ -99,24 +101,107 @@ __device__ __forceinline__ void eliminate(C (&e)[kQ], C (&w)[4], C (&dsel)[4], i
 // What the row solves of a panel need beside its factored block, per band: the operands of the four
 // 16 x 16 inverses (step s of sub-block c at [(4 c + s) * 64 + lane]), then 1 / d of the 64 columns.
 constexpr int kWorkInv = 4 * 4 * 64;
+// Three slots a band, by panel: in the fused schedule a launch writes the next panel's while it still reads
+// this one's and the last one's.
+constexpr size_t kWorkSlot = (kWorkInv + kNB) * sizeof(double);
 template <typename C>
-__device__ __forceinline__ C *panel_work(void *work, int band)
+__device__ __forceinline__ C *panel_work(void *work, int band, int c0)
 {
-    return (C *)((unsigned char *)work + (size_t)band * kBandWorkBytes);
+    return (C *)((unsigned char *)work + (size_t)band * kBandWorkBytes + (size_t)(c0 / kNB % 3) * kWorkSlot);
 }
-static_assert((kWorkInv + kNB) * sizeof(double) <= kBandWorkBytes, "factor workspace");
+static_assert(3 * kWorkSlot <= kBandWorkBytes, "factor workspace");
+
+// Row tiles of the panel at c0 (tile t: rows c0 + 64 + 16 t .. + 15, its 64 columns) against the factored
+// diagonal block, one wave: X = A L^-T by blocks of 16 columns (substitution between them, the 16 x 16
+// inverse within), L = X D^-1.  40 MFMAs in one chain; the operands of the diagonal block are read
+// from L2 by every wave, which spreads a band's rows over as many CUs as there are.  Tiles t0, t0 +
+// stride, ...: out(t, column, value) takes lane li's entry of row li of the tile.  Rows past the panel
+// are zero.
+template <typename T, typename C, typename F>
+__device__ __forceinline__ void solve_tiles(const BandDesc &d, int c0, int t0, int stride, int ntile, const C *work, F &&out)
+{
+    using M = Mfma16<C>;
+    using acc_t = typename M::acc_t;
+    const int n = d.n, bw = d.bw;
+    const int nr = min(n - c0, kNB + bw);  // panel rows (relative to c0); the panel is full: n > c0 + 64
+    const unsigned ldu = (unsigned)bw + 1;
+    constexpr unsigned es = sizeof(T);
+    const __amdgpu_buffer_rsrc_t rs = band_rsrc(d.fac, (unsigned)((size_t)n * ldu * es));
+    const int lane = threadIdx.x & 63, li = lane & 15;
+    C inv[4][4], dinv[4][4], l[4][4][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            inv[c][s] = work[(4 * c + s) * 64 + lane];
+            dinv[c][s] = work[kWorkInv + kQ * c + M::row(lane, s)];
+#pragma unroll
+            for (int e = 0; e < c; ++e) {  // L[16 c + li][16 e + krow]
+                const int row = kQ * c + li, col = kQ * e + M::row(lane, s);
+                l[c][e][s] = -(C)load_if<T>(row - col <= bw, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(row - col)) * es);
+            }
+        }
+    for (int q = 0; q < ntile; ++q) {
+        const int t = t0 + q * stride, r = kNB + kQ * t + li;
+        acc_t a[4], x[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int col = kQ * c + M::row(lane, v);
+                a[c][v] = (C)load_if<T>(r < nr && r - col <= bw, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(r - col)) * es);
+            }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+#pragma unroll
+            for (int e = 0; e < c; ++e)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) a[c] = M::run(l[c][e][s], x[e][s], a[c]);
+            const acc_t zero = {C(0), C(0), C(0), C(0)};
+            x[c] = zero;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) x[c] = M::run(inv[c][s], a[c][s], x[c]);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) out(t, kQ * c + M::row(lane, v), (T)(x[c][v] * dinv[c][v]));
+    }
+}
+
+// tiles t0 .. t0 + ntile - 1 of the panel at c0, back to the band
+template <typename T, typename C>
+__device__ __forceinline__ void solve_rows(const BandDesc &d, int c0, int t0, int ntile, const C *work)
+{
+    const int n = d.n, bw = d.bw, nr = min(n - c0, kNB + bw);
+    if (n <= c0 + kNB || kNB + kQ * t0 >= nr) return;
+    const unsigned ldu = (unsigned)bw + 1;
+    constexpr unsigned es = sizeof(T);
+    const __amdgpu_buffer_rsrc_t rs = band_rsrc(d.fac, (unsigned)((size_t)n * ldu * es));
+    const int li = threadIdx.x & 15;
+    const int left = (nr - kNB - kQ * t0 + kQ - 1) / kQ;
+    solve_tiles<T, C>(d, c0, t0, 1, min(ntile, left), work, [&](int t, int col, T v) {
+        const int r = kNB + kQ * t + li;
+        store_if<T>(r < nr && r - col <= bw, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(r - col)) * es, v);
+    });
+}
+
+// place of entry (row, k) of a 64 x 64 operand block in LDS: the 16 rows and 4 columns an MFMA operand
+// reads at once fall into different banks
+__device__ __forceinline__ int panel_at(int k, int row) { return k * kNB + (row ^ ((k & 3) << 4)); }
 
 // Diagonal block of the panel at c0 (64 columns, unit pivots past n): four waves, wave w owning the
-// 16-row strip w (tiles (w, 0..w)).  With `update`, the block first takes the rank-64 update of the
+// 16-row strip w (tiles (w, 0..w)).  With kUpdate, the block first takes the rank-64 update of the
 // panel at c0 - 64, whose 64 x 64 operand block goes through LDS (one memory latency for the whole
-// block).  Then for c = 0..3: wave c factors tile (c, c) by rows; the strips below solve their tile
+// block); with kSolve its rows there are still unsolved, and the workgroup solves these 64 first (`prev`:
+// that panel's workspace).  Then for c = 0..3: wave c factors tile (c, c) by rows; the strips below solve their tile
 // (i, c) against it (one product with the 16 x 16 inverse) and update their remaining tiles.  The
 // inverses are of 16 x 16 unit lower blocks only: between sub-blocks the solve is a substitution.
 // Bound by its chain: 64 pivots of about 100 cycles each (reciprocal and broadcasts), four LDS round
 // trips and product chains between the sub-blocks.
 template <typename C>
 struct DiagLds {
-    C panel[kNB * kNB];   // L[c0 + row][c0 - 64 + k] at k * 64 + (row ^ 16 (k % 4))
+    C panel[kNB * kNB];   // L[c0 + row][c0 - 64 + k] at panel_at(k, row)
     C nd[kNB];            // -d of the previous panel
     C tr[kQ * (kQ + 1)];  // a diagonal tile on its way to lane = row
     C inv[4 * 64];        // sub-block c: operands of the inverse
@@ -126,12 +211,12 @@ struct DiagLds {
     int bad;
 };
 
-template <typename T, typename C>
-__device__ __forceinline__ void diag_panel(const BandDesc &d, int c0, bool update, C *work)
+enum DiagMode { kFirst, kUpdate, kSolve };
+template <typename T, typename C, int kMode>
+__device__ __forceinline__ void diag_panel(const BandDesc &d, int c0, C *work, const C *prev, DiagLds<C> &sh)
 {
     using M = Mfma16<C>;
     using acc_t = typename M::acc_t;
-    __shared__ DiagLds<C> sh;
     const int n = d.n, bw = d.bw;
     if (c0 >= n) return;
     const unsigned ldu = (unsigned)bw + 1;
@@ -144,14 +229,14 @@ __device__ __forceinline__ void diag_panel(const BandDesc &d, int c0, bool updat
     const int i = kQ * wv + li;  // this lane's row
     constexpr int kP = kNB * kNB / (64 * kUW);
     T pv[kP], dv = T(0);
-    if (update) {  // panel operands: lanes along a column's rows
-        const int cp = c0 - kNB;
+    const int cp = c0 - kNB;
+    if constexpr (kMode != kFirst) dv = load_if<T>(tid < kNB, rs, (unsigned)(cp + lane) * ldu * es);
+    if constexpr (kMode == kUpdate) {  // panel operands: lanes along a column's rows
 #pragma unroll
         for (int q = 0; q < kP; ++q) {
             const int k = kUW * q + wv;
             pv[q] = load_if<T>(lane < w && lane + kNB - k <= bw, rs, ((unsigned)(cp + k) * ldu + (unsigned)(lane + kNB - k)) * es);
         }
-        dv = load_if<T>(tid < kNB, rs, (unsigned)(cp + lane) * ldu * es);
     }
     acc_t acc[4];
 #pragma unroll
@@ -166,11 +251,12 @@ __device__ __forceinline__ void diag_panel(const BandDesc &d, int c0, bool updat
             acc[j][v] = (hi >= w && hi == lo) ? C(1) : x;
         }
     }
-    if (update) {
+    if constexpr (kMode != kFirst) {
+        if constexpr (kMode == kUpdate) {
 #pragma unroll
-        for (int q = 0; q < kP; ++q) {
-            const int k = kUW * q + wv;
-            sh.panel[k * kNB + (lane ^ ((k & 3) << 4))] = (C)pv[q];
+            for (int q = 0; q < kP; ++q) sh.panel[panel_at(kUW * q + wv, lane)] = (C)pv[q];
+        } else {
+            solve_tiles<T, C>(d, cp, wv, 1, 1, prev, [&](int t, int k, T v) { sh.panel[panel_at(k, kQ * t + li)] = (C)v; });
         }
         if (tid < kNB) sh.nd[tid] = -(C)dv;
         lds_barrier();
@@ -178,7 +264,7 @@ __device__ __forceinline__ void diag_panel(const BandDesc &d, int c0, bool updat
 #pragma unroll
         for (int s = 0; s < kNB / 4; ++s) {
             nd[s] = sh.nd[4 * s + lk];
-            own[s] = sh.panel[(4 * s + lk) * kNB + (i ^ (lk << 4))];
+            own[s] = sh.panel[panel_at(4 * s + lk, i)];
         }
         // wave 0 has the least of it and goes on to its diagonal tile while the others finish
 #pragma unroll
@@ -186,7 +272,7 @@ __device__ __forceinline__ void diag_panel(const BandDesc &d, int c0, bool updat
             if (j > wv) continue;
 #pragma unroll
             for (int s = 0; s < kNB / 4; ++s)
-                acc[j] = M::run(nd[s] * sh.panel[(4 * s + lk) * kNB + ((kQ * j + li) ^ (lk << 4))], own[s], acc[j]);
+                acc[j] = M::run(nd[s] * sh.panel[panel_at(4 * s + lk, kQ * j + li)], own[s], acc[j]);
         }
     }
     C lkeep[4] = {C(0), C(0), C(0), C(0)};
@@ -295,69 +381,6 @@ __device__ __forceinline__ void diag_panel(const BandDesc &d, int c0, bool updat
             *d.info = sh.bad;
     }
 }
-
-// Row tile t of the panel at c0 (rows c0 + 64 + 16 t .. + 15, its 64 columns) against the factored
-// diagonal block, one wave: X = A L^-T by blocks of 16 columns (substitution between them, the 16 x 16
-// inverse within), L = X D^-1.  40 MFMAs in one chain; the operands of the diagonal block are read
-// from L2 by every wave, which spreads a band's rows over as many CUs as there are.
-template <typename T, typename C>
-__device__ __forceinline__ void solve_rows(const BandDesc &d, int c0, int t0, int ntile, const C *work)
-{
-    using M = Mfma16<C>;
-    using acc_t = typename M::acc_t;
-    const int n = d.n, bw = d.bw;
-    const int nr = min(n - c0, kNB + bw);  // panel rows (relative to c0); the panel is full: n > c0 + 64
-    if (n <= c0 + kNB || kNB + kQ * t0 >= nr) return;
-    const unsigned ldu = (unsigned)bw + 1;
-    constexpr unsigned es = sizeof(T);
-    const __amdgpu_buffer_rsrc_t rs = band_rsrc(d.fac, (unsigned)((size_t)n * ldu * es));
-    const int lane = threadIdx.x & 63, li = lane & 15;
-    C inv[4][4], dinv[4][4], l[4][4][4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            inv[c][s] = work[(4 * c + s) * 64 + lane];
-            dinv[c][s] = work[kWorkInv + kQ * c + M::row(lane, s)];
-#pragma unroll
-            for (int e = 0; e < c; ++e) {  // L[16 c + li][16 e + krow]
-                const int row = kQ * c + li, col = kQ * e + M::row(lane, s);
-                l[c][e][s] = -(C)load_if<T>(row - col <= bw, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(row - col)) * es);
-            }
-        }
-    for (int t = t0; t < t0 + ntile; ++t) {
-        const int r = kNB + kQ * t + li;
-        if (kNB + kQ * t >= nr) break;  // uniform
-        acc_t a[4], x[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int col = kQ * c + M::row(lane, v);
-                a[c][v] = (C)load_if<T>(r < nr && r - col <= bw, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(r - col)) * es);
-            }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-#pragma unroll
-            for (int e = 0; e < c; ++e)
-#pragma unroll
-                for (int s = 0; s < 4; ++s) a[c] = M::run(l[c][e][s], x[e][s], a[c]);
-            const acc_t zero = {C(0), C(0), C(0), C(0)};
-            x[c] = zero;
-#pragma unroll
-            for (int s = 0; s < 4; ++s) x[c] = M::run(inv[c][s], a[c][s], x[c]);
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int col = kQ * c + M::row(lane, v);
-                store_if<T>(r < nr && r - col <= bw, rs, ((unsigned)(c0 + col) * ldu + (unsigned)(r - col)) * es,
-                            (T)(x[c][v] * dinv[c][v]));
-            }
-    }
-}
-
 
 // lower-triangle block index p -> (bi, bj), bj <= bi
 __device__ __forceinline__ void tri_decode(int p, int &bi, int &bj)
@@ -476,11 +499,30 @@ __device__ __forceinline__ void trailing_blocks(const BandDesc &d, int c0, int p
                 for (int v = 0; v < 4; ++v) store_vs<T>(rs, off[s][a][b][v], 0, cur[s][a][b][v]);
 }
 
+// Descriptor of a workgroup's band in scalar registers.  The compiler takes a descriptor read behind a
+// division or a store for possibly divergent, and would then turn every buffer access through it into a loop
+// over the lanes' (equal) descriptors.
+__device__ __forceinline__ BandDesc uniform_desc(const BandDesc *descs, int band)
+{
+    const BandDesc &s = descs[__builtin_amdgcn_readfirstlane(band)];
+    BandDesc d;
+    d.fac = uniform_ptr(s.fac);
+    d.n = __builtin_amdgcn_readfirstlane(s.n);
+    d.bw = __builtin_amdgcn_readfirstlane(s.bw);
+    d.info = uniform_ptr(s.info);
+    d.stats = nullptr;
+    d.x = nullptr;
+    d.active = 1;
+    return d;
+}
+
 // Diagonal block at column 0 of every band (the later ones are factored by the trailing launches).
 template <typename T, typename C>
 __global__ __launch_bounds__(64 * kUW) void k_band_diag(const BandDesc *descs, void *work)
 {
-    diag_panel<T, C>(descs[blockIdx.x], 0, false, panel_work<C>(work, (int)blockIdx.x));
+    __shared__ DiagLds<C> sh;
+    const BandDesc d = uniform_desc(descs, (int)blockIdx.x);
+    diag_panel<T, C, kFirst>(d, 0, panel_work<C>(work, (int)blockIdx.x, 0), nullptr, sh);
 }
 
 // XCD-aware assignment of a launch's workgroups to (band, index within the band).  Workgroups are
@@ -501,6 +543,9 @@ __device__ __forceinline__ bool band_of_workgroup(int h, int active, int wg, int
         band = h % kXcds + kXcds * (s / wg);
         local = s % wg;
     }
+    // the divisions run on the vector unit: back to scalars
+    band = __builtin_amdgcn_readfirstlane(band);
+    local = __builtin_amdgcn_readfirstlane(local);
     return band < active;
 }
 inline unsigned band_grid(int active, int wg)
@@ -516,7 +561,8 @@ __global__ __launch_bounds__(64 * kUW) void k_band_rows(const BandDesc *descs, v
     int band, local;
     if (!band_of_workgroup((int)blockIdx.x, active, wg_per_band, band, local)) return;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    solve_rows<T, C>(descs[band], c0, (local * kUW + wave) * tiles, tiles, panel_work<C>(work, band));
+    const BandDesc d = uniform_desc(descs, band);
+    solve_rows<T, C>(d, c0, (local * kUW + wave) * tiles, tiles, panel_work<C>(work, band, c0));
 }
 
 // One part of the trailing update at c0, kUW blocks (one per wave) per workgroup; workgroups
@@ -529,14 +575,17 @@ __global__ __launch_bounds__(64 * kUW) void k_band_trailing(const BandDesc *desc
 {
     const int b = (int)blockIdx.x;
     if (b < ndiag) {
-        diag_panel<T, C>(descs[b], c0 + kNB, true, panel_work<C>(work, b));
+        __shared__ DiagLds<C> sh;
+        const BandDesc d = uniform_desc(descs, b);
+        diag_panel<T, C, kUpdate>(d, c0 + kNB, panel_work<C>(work, b, c0 + kNB), nullptr, sh);
         return;
     }
     if (b < pad) return;
     int band, local;
     if (!band_of_workgroup(b - pad, active, wg_per_band, band, local)) return;
     const int p[1] = {__builtin_amdgcn_readfirstlane((int)(local * kUW + (threadIdx.x >> 6)))};
-    trailing_blocks<T, 1>(descs[band], c0, part, p);
+    const BandDesc d = uniform_desc(descs, band);
+    trailing_blocks<T, 1>(d, c0, part, p);
 }
 
 // Lookahead step: the first workgroups (nrow per band, padded to `pad`) solve the rows of the panel at
@@ -554,14 +603,111 @@ __global__ __launch_bounds__(kPT) void k_band_step(const BandDesc *descs, void *
     int band, local;
     if (b < pad) {
         if (!band_of_workgroup(b, np, nrow, band, local)) return;
-        solve_rows<T, C>(descs[band], c0 + kNB, (local * kW + wave) * tiles, tiles, panel_work<C>(work, band));
+        const BandDesc d = uniform_desc(descs, band);
+        solve_rows<T, C>(d, c0 + kNB, (local * kW + wave) * tiles, tiles, panel_work<C>(work, band, c0 + kNB));
         return;
     }
     if (!band_of_workgroup(b - pad, active, wg_per_band, band, local)) return;
     int p[NBLK];
 #pragma unroll
     for (int s = 0; s < NBLK; ++s) p[s] = (local * NBLK + s) * kW + wave;
-    trailing_blocks<T, NBLK>(descs[band], c0, kRest, p);
+    const BandDesc d = uniform_desc(descs, band);
+    trailing_blocks<T, NBLK>(d, c0, kRest, p);
+}
+
+// 64 x 64 tile (I, J), J <= I, of the trailing window at c0 with the panel's rows still unsolved: the four
+// waves solve the 64 rows of I and of J into LDS, then take one 32 x 32 block each of the tile's update
+// (the same MFMA sequence per block as trailing_blocks).
+template <typename T>
+struct TileLds {
+    T pi[kNB * kNB], pj[kNB * kNB];  // L[window row][k] at panel_at(k, row)
+    T nd[kNB];
+};
+template <typename T, typename C>
+__device__ __forceinline__ void fused_tile(const BandDesc &d, int c0, int I, int J, const C *work, TileLds<T> &sh)
+{
+    using M = Mfma16<T>;
+    using acc_t = typename M::acc_t;
+    const int n = d.n, bw = d.bw;
+    const int nr = min(n - c0, kNB + bw);
+    const unsigned ldu = (unsigned)bw + 1;
+    constexpr unsigned es = sizeof(T);
+    const __amdgpu_buffer_rsrc_t rs = band_rsrc(d.fac, (unsigned)((size_t)n * ldu * es));
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ri = 32 * (wv >> 1), rj = 32 * (wv & 1);  // the wave's block in the tile
+    const bool mine = I != J || ri >= rj, diag = I == J && ri == rj;
+    const T dv = load_if<T>(tid < kNB, rs, (unsigned)(c0 + lane) * ldu * es);
+    acc_t cur[2][2];
+    unsigned off[2][2][4];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int i = kNB + kNB * I + ri + 16 * a + li, j = kNB + kNB * J + rj + 16 * b + M::row(lane, v);
+                const bool ok = mine && i < nr && i >= j;
+                off[a][b][v] = ok ? ((unsigned)c0 * ldu + (unsigned)j * (ldu - 1) + (unsigned)i) * es : kMaskedOff;
+                cur[a][b][v] = load_vs<T>(rs, off[a][b][v], 0);
+            }
+    solve_tiles<T, C>(d, c0, 4 * I + wv, 4 * (J - I), I == J ? 1 : 2, work, [&](int t, int k, T v) {
+        (t == 4 * I + wv ? sh.pi : sh.pj)[panel_at(k, kQ * wv + li)] = v;
+    });
+    if (tid < kNB) sh.nd[tid] = -dv;
+    lds_barrier();
+    if (!mine) return;
+    const T *pj = I == J ? sh.pi : sh.pj;
+#pragma unroll
+    for (int s = 0; s < kNB / 4; ++s) {
+        const int k = 4 * s + lk;
+        const T nd = sh.nd[k];
+        const T A0 = nd * pj[panel_at(k, rj + li)], A1 = nd * pj[panel_at(k, rj + 16 + li)];
+        const T B0 = sh.pi[panel_at(k, ri + li)], B1 = sh.pi[panel_at(k, ri + 16 + li)];
+        cur[0][0] = M::run(A0, B0, cur[0][0]);
+        cur[1][0] = M::run(A0, B1, cur[1][0]);
+        cur[1][1] = M::run(A1, B1, cur[1][1]);
+        if (!diag) cur[0][1] = M::run(A1, B0, cur[0][1]);
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) store_vs<T>(rs, off[a][b][v], 0, cur[a][b][v]);
+}
+
+// Fused step at c0, one launch a step: workgroup 0 of a band solves the next 64 rows, updates and factors
+// the next diagonal block; `ntile` workgroups apply the rest of the update, solving the rows they need
+// themselves (the panel at c0 is only read, so no workgroup waits for another); the last ones write the
+// solved rows of the panel before, which nothing in this launch reads.  Three times the update's
+// multiply-adds and one launch on the chain instead of two: for few bands.
+template <typename T, typename C>
+__global__ __launch_bounds__(64 * kUW) void k_band_fused(const BandDesc *descs, void *work, int c0, int ntile, int nrow)
+{
+    __shared__ union {
+        DiagLds<C> diag;
+        TileLds<T> tile;
+    } sh;
+    const int per = 1 + ntile + nrow;
+    const int band = __builtin_amdgcn_readfirstlane((int)blockIdx.x / per), g = (int)blockIdx.x - band * per;
+    const BandDesc d = uniform_desc(descs, band);
+    if (g > ntile) {
+        if (c0 == 0) return;
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        solve_rows<T, C>(d, c0 - kNB, (g - 1 - ntile) * kUW + wave, 1, panel_work<C>(work, band, c0 - kNB));
+        return;
+    }
+    if (d.n <= c0 + kNB) return;
+    const C *here = panel_work<C>(work, band, c0);
+    if (g == 0) {
+        diag_panel<T, C, kSolve>(d, c0 + kNB, panel_work<C>(work, band, c0 + kNB), here, sh.diag);
+        return;
+    }
+    int I, J;
+    tri_decode(g, I, J);  // tile 0, the next diagonal block, is workgroup 0's
+    if (kNB + kNB * I >= min(d.n - c0, kNB + d.bw)) return;
+    fused_tile<T, C>(d, c0, I, J, here, sh.tile);
 }
 
 // negatives, min d, max |d|, min |d| of each factored diagonal (one workgroup of 1024 threads per band)
@@ -612,11 +758,16 @@ __global__ __launch_bounds__(1024) void k_pivot_stats(const BandDesc *descs)
 // Factor schedules (every one gives the same result bit for bit):
 //   0 plain: per step the panel's rows, then the whole trailing update, whose first workgroups update
 //   and factor the next diagonal block;
-//   1, 2 lookahead: per step the next panel's columns (kNext, with the next diagonal block), then the
-//   next panel's rows together with the rest of the update (k_band_step), 1 or 2 blocks per wave.
-// Plain has the rest of the update beside the diagonal block's chain, lookahead beside the rows; which
-// one is faster depends on the number and shape of the bands, so the autotuner picks per shape
-// bucket (KSH_LOOKAHEAD=k forces k).
+//   1 lookahead: per step the next panel's columns (kNext, with the next diagonal block), then the
+//   next panel's rows together with the rest of the update (k_band_step);
+//   2 fused (k_band_fused), one launch a step, for up to kFusedBands bands; for more, lookahead with two
+//   blocks per wave.
+// Plain has the rest of the update beside the diagonal block's chain, lookahead beside the rows, fused the
+// shortest chain and the most arithmetic; which one is fastest depends on the number and shape of the
+// bands, so the autotuner picks per shape bucket (KSH_LOOKAHEAD=k forces k).
+// Fused up to 8 bands: a band's workgroups (22 at bw 326, 192 at bw 1166) then stay around the chip's 256
+// CUs; with more, the threefold arithmetic is what bounds the step.
+constexpr int kFusedBands = 8;
 constexpr int kSchedules = 3;
 
 int schedule_forced()
@@ -690,6 +841,16 @@ void run_tiled_sched(hipStream_t s, const BandDesc *d_descs, void *work, const s
         }
     } else if (sched == 1) {
         run_lookahead<T, C, 1>(s, d_descs, work, ns, maxbw);
+    } else if (nbands <= kFusedBands) {
+        const int nt = (maxbw + kNB - 1) / kNB, ntile = std::max(0, nt * (nt + 1) / 2 - 1);
+        const int nrow = ((maxbw + kQ - 1) / kQ + kUW - 1) / kUW;
+        int c0 = 0;
+        for (;; c0 += kNB) {  // the step past a band's last panel still writes that panel's rows
+            const int np = active_at(ns, c0);
+            if (np == 0) break;
+            hipLaunchKernelGGL((k_band_fused<T, C>), dim3((unsigned)(np * (1 + ntile + nrow))), dim3(64 * kUW), 0, s, d_descs, work, c0,
+                               ntile, nrow);
+        }
     } else {
         run_lookahead<T, C, 2>(s, d_descs, work, ns, maxbw);
     }

@@ -224,7 +224,7 @@ int ensure_rc64(Matrix &K);
 int band_solve_batch(hipStream_t s, void *d_descs, const std::vector<BandDescHost> &h, int prec);
 constexpr size_t kBandDescBytes = 48;
 // panel workspace of one band of a factor call (operands of the row solves), behind the descriptors
-constexpr size_t kBandWorkBytes = 8704;
+constexpr size_t kBandWorkBytes = 3 * 8704;
 inline size_t factor_desc_offset(size_t n) { return (n * kBandDescBytes + 255) / 256 * 256; }
 inline size_t factor_desc_bytes(size_t n) { return factor_desc_offset(n) + n * kBandWorkBytes; }
 int band_solve(Matrix &K, const void *fac, int prec, double *x_dev);
