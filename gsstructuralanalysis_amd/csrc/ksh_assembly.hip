@@ -17,8 +17,8 @@
 // no atomics).
 //
 // Every kernel runs over a batch of instances described by an InstDesc array (a single problem is
-// a batch of one): element kernels map blockIdx.x to (instance, element) and entry kernels map a
-// thread to (instance, dof / band slot) by binary search over the prefix offsets.
+// a batch of one).  A wave works for one instance, which it finds in the prefix offsets: an
+// instance's elements, dofs, Gauss points and band pairs each start at a wave of their own.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -41,147 +41,235 @@ using shell::ElemArgs;
 
 inline unsigned nblk(size_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
-template <typename Get>
-__device__ inline int find_inst(int n, long long key, Get get)
+// The descriptor of the instance that a wave works for: the last m with first(m) <= key (first is
+// non-decreasing over the n instances, first(0) = 0; key is the same in every lane and all 64
+// lanes are active).  The lanes test 64 instances at a time, so up to 64 instances take one read
+// and up to 4096 two, instead of one dependent read per halving.  The index is wave-uniform, and
+// the pointers are stated to be global: their loads are global_load / s_load.  Loaded from the
+// array by a per-lane index they were generic pointers in vector registers, and a flat access
+// waits for all memory and LDS accesses in flight, and every access by a buffer resource made
+// from one ran in a loop over the lanes' distinct values (147 such loops in k_band_gather).
+template <typename First>
+__device__ __forceinline__ InstDesc inst_desc(const InstDesc *__restrict__ descs, int n, long long key, First first)
 {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (get(mid) <= key) lo = mid;
-        else hi = mid - 1;
+    int lo = 0, end = n;
+    while (end - lo > 1) {
+        const int step = (end - lo + 63) >> 6, m = lo + (int)(threadIdx.x & 63) * step;
+        const bool at = m < end && first(descs[min(m, end - 1)]) <= key;
+        lo = __builtin_amdgcn_readfirstlane(lo + (__popcll(__ballot(at)) - 1) * step);
+        end = min(end, lo + step);
     }
-    return lo;
+    InstDesc d = descs[lo];
+    d.ctrl0 = global_ptr(d.ctrl0);
+    d.tabx = global_ptr(d.tabx);
+    d.taby = global_ptr(d.taby);
+    d.gpgeo = global_ptr(d.gpgeo);
+    d.F = global_ptr(d.F);
+    d.u_free = global_ptr(d.u_free);
+    d.free_idx = global_ptr(d.free_idx);
+    d.free2full = global_ptr(d.free2full);
+    d.u_full = global_ptr(d.u_full);
+    d.Fe = global_ptr(d.Fe);
+    d.R = global_ptr(d.R);
+    d.Ke = global_ptr(d.Ke);
+    d.ab = global_ptr(d.ab);
+    d.Hg = global_ptr(d.Hg);
+    d.P0 = global_ptr(d.P0);
+    return d;
+}
+
+// index of this wave in the launch
+__device__ __forceinline__ int wave_index()
+{
+    return __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)));
 }
 
 // ---------------------------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------------------------
-__global__ void k_construct_solution(const InstDesc *descs, int ninst, int total)
+__global__ __launch_bounds__(256) void k_construct_solution(const InstDesc *__restrict__ descs, int ninst)
 {
-    int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= total) return;
-    const InstDesc &d = descs[find_inst(ninst, gid, [&](int m) { return (long long)descs[m].full0; })];
-    int g = gid - d.full0;
-    int f = d.free_idx[g];
+    const int w = wave_index();
+    const InstDesc d = inst_desc(descs, ninst, w, [](const InstDesc &e) { return e.full0; });
+    const int g = (w - d.full0) * 64 + (int)(threadIdx.x & 63);
+    if (g >= d.ndof) return;
+    const int f = d.free_idx[g];
     d.u_full[g] = (f >= 0) ? d.u_free[f] : 0.0;
 }
 
-// deformed derivative vectors (a1, a2, a11, a22, a12) at one Gauss point of element (ex, ey)
-template <int P>
-__device__ __forceinline__ void gp_derivatives(const InstDesc &d, int ex, int ey, const double *tx, const double *ty,
-                                               double (&dv)[15])
+// deformed derivative vectors (a1, a2, a11, a22, a12) at one Gauss point from its basis tables
+// (value, first and second derivative, P1 entries each) and the element's control points x(ia,
+// ib, c).  Products and sums in the order of k_setup_geometry, so that the rounding of a_ab and of
+// the undeformed A_ab cancels in the strain: sums along x first and then along y take 204
+// operations instead of 320, and lost a digit of the residual.  kRows: the points of one ib are
+// read at a time (from LDS; from memory all of them are loaded at once)
+template <int P, bool kRows, typename X>
+__device__ __forceinline__ void gp_derivatives(const double *tx, const double *ty, X x, double (&dv)[15])
 {
-    constexpr int P1 = P + 1, NB = P1 * P1;
+    constexpr int P1 = P + 1, kUnroll = kRows ? 1 : P1;
+    double vx[3][P1];
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int a = 0; a < P1; ++a) vx[r][a] = tx[r * P1 + a];
 #pragma unroll
     for (int r = 0; r < 15; ++r) dv[r] = 0.0;
+#pragma unroll kUnroll
+    for (int ib = 0; ib < P1; ++ib) {
+        const double vy[3] = {ty[ib], ty[P1 + ib], ty[2 * P1 + ib]};
 #pragma unroll
-    for (int A = 0; A < NB; ++A) {
-        const int ia = A % P1, ib = A / P1, cp = (ex + ia) + d.mx * (ey + ib);
-        const double psi[5] = {tx[P1 + ia] * ty[ib], tx[ia] * ty[P1 + ib], tx[2 * P1 + ia] * ty[ib],
-                               tx[ia] * ty[2 * P1 + ib], tx[P1 + ia] * ty[P1 + ib]};
+        for (int ia = 0; ia < P1; ++ia) {
+            const double psi[5] = {vx[1][ia] * vy[0], vx[0][ia] * vy[1], vx[2][ia] * vy[0], vx[0][ia] * vy[2], vx[1][ia] * vy[1]};
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const double x = d.ctrl0[3 * cp + c] + d.u_full[3 * cp + c];
+            for (int c = 0; c < 3; ++c) {
+                const double xc = x(ia, ib, c);
 #pragma unroll
-            for (int a = 0; a < 5; ++a) dv[3 * a + c] += psi[a] * x;
+                for (int a = 0; a < 5; ++a) dv[3 * a + c] += psi[a] * xc;
+            }
         }
     }
 }
 
-// Residual, stage 1: one thread per Gauss point; its state and the 15 entries of f_g
-// (f_int_{A,i} = sum_g phi . f_g), stored entry-major in the H_g buffer (Fg[I * ngp + gp]).
-template <int P>
-__global__ __launch_bounds__(128) void k_residual_gp(const InstDesc *descs, int ninst, int total)
-{
-    constexpr int P1 = P + 1, NQ = P1, NG = NQ * NQ;
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= total) return;
-    const InstDesc &d = descs[find_inst(ninst, gid, [&](int m) { return (long long)descs[m].elem0 * NG; })];
-    const int gp = gid - d.elem0 * NG;
-    const int e = gp / NG, g = gp % NG, ex = e % d.nx, ey = e / d.nx, qx = g % NQ, qy = g / NQ;
-    const double *tx = d.tabx + ((size_t)(ex * NQ + qx) * 3) * P1;
-    const double *ty = d.taby + ((size_t)(ey * NQ + qy) * 3) * P1;
-    double dv[15];
-    gp_derivatives<P>(d, ex, ey, tx, ty, dv);
-    double st[shell::kState];
-    shell::gp_state(dv, d.gpgeo + (size_t)gp * kGeoStride, d.t, st);
-    const size_t stride = (size_t)d.nel * NG;
-#pragma unroll
-    for (int I = 0; I < kFq; ++I) d.Hg[(size_t)I * stride + gp] = shell::f_entry(st, I);
-    if (d.pressure != 0.0) {  // -p w (a1 x a2) on the deformed surface: the follower load, as a force on the residual's side
-        double n[3];
-        shell::cross3(dv, dv + 3, n);
-        const double s = -d.pressure * d.gpgeo[(size_t)gp * kGeoStride + 13];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) d.Hg[(size_t)(kFq + i) * stride + gp] = s * n[i];
-    }
-}
+// elements of a wave of k_residual_elem: one Gauss point per lane
+constexpr int res_elements(int p) { return p == 2 ? 64 / 9 : 64 / 16; }
 
-// Residual, stage 2: one wave per element; lane (A, i) sums Fe[3A+i] = sum_g sum_a
-// Psi_g[a][A] f_g[3a+i] (g outer, a inner).  The wave first stages its element's Gauss-point
-// resultants (kFq or, with a follower pressure, kFqP rows of NG contiguous values) and its two
-// basis tables (NQ x 3 x P1 values each, contiguous per element column / row) in LDS, every load
-// in flight at once; the sums then read LDS only.  (Reading them inside the sum cost one memory
-// latency per Gauss point.)
+// Residual: a wave takes EW consecutive elements of one instance, a Gauss point per lane and then
+// an element dof per lane.
+//   stage: the elements' deformed control points and their two basis tables into LDS, every load
+//     in flight at once;
+//   points: the lane's state and its f_g (f_int_{A,i} = sum_g phi . f_g; 15 entries, and the
+//     follower pressure's 3) into LDS;
+//   sums: Fe[3A+i] = sum_g sum_a Psi_g[a][A] f_g[3a+i] as a product of two short sums, over qx at
+//     each qy for the three factors N, N', N'' along y, then over qy: 32 multiply-adds per dof
+//     at degree 3 instead of 80, and half the LDS reads.
+// Undeformed geometry (128 bytes a point) is all that has to come from memory.  With the f_g
+// written to memory by one kernel and read by another (2 x 120 bytes a point, and the control
+// points read once per point), the 64 roofs of 16..48 elements a side took 186 us;
+// 48 us like this.
 template <int P>
-__global__ __launch_bounds__(256) void k_residual_tiles(const InstDesc *descs, int ninst, int total_el)
+__global__ __launch_bounds__(64, 3) void k_residual_elem(const InstDesc *__restrict__ descs, int ninst)
 {
-    constexpr int P1 = P + 1, NB = P1 * P1, NQ = P1, NG = NQ * NQ, NT = NQ * 3 * P1;
-    constexpr int FL = (kFqP * NG + 63) / 64, TL = (2 * NT + 63) / 64;  // loads per lane
-    __shared__ double sF[4][kFqP * NG];
-    __shared__ double sT[4][2 * NT];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int eg = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + w));
-    if (eg >= total_el) return;
-    const InstDesc &d = descs[find_inst(ninst, eg, [&](int m) { return (long long)descs[m].elem0; })];
-    const int e = eg - d.elem0, ex = e % d.nx, ey = e / d.nx;
+    constexpr int P1 = P + 1, NB = P1 * P1, NQ = P1, NG = NQ * NQ, NT = NQ * 3 * P1, NL = 3 * NB;
+    constexpr int EW = res_elements(P), NGP = NG | 1;  // an odd pitch: rows of f_g on different banks
+    constexpr int XL = (EW * NL + 63) / 64, TL = (EW * 2 * NT + 63) / 64;
+    // control points, then f_g, then the sums over qx: each is read into registers before the next
+    // is written
+    __shared__ double sF[EW][kFqP * NGP];
+    __shared__ double sT[EW][2 * NT];
+    const int w = (int)blockIdx.x, lane = (int)threadIdx.x;
+    const InstDesc d = inst_desc(descs, ninst, w, [](const InstDesc &e) { return e.res0; });
+    const int e0 = (w - d.res0) * EW, ne = min(EW, d.nel - e0);
+    // LDS accesses of one wave complete in order; the fence keeps the compiler from moving them
+    auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    {
+        double vx[XL], vu[XL], vt[TL];
+#pragma unroll
+        for (int q = 0; q < XL; ++q) {
+            const int idx = lane + 64 * q, el = idx / NL, r = idx % NL, A = r / 3;
+            const int e = e0 + min(el, ne - 1), cp = (e % d.nx + A % P1) + d.mx * (e / d.nx + A / P1);
+            vx[q] = d.ctrl0[3 * cp + r % 3];
+            vu[q] = d.u_full[3 * cp + r % 3];
+        }
+#pragma unroll
+        for (int q = 0; q < TL; ++q) {
+            const int idx = lane + 64 * q, el = idx / (2 * NT), r = idx % (2 * NT);
+            const int e = e0 + min(el, ne - 1);
+            const double *tab = r < NT ? d.tabx + (size_t)(e % d.nx) * NT + r : d.taby + (size_t)(e / d.nx) * NT + (r - NT);
+            vt[q] = *tab;
+        }
+#pragma unroll
+        for (int q = 0; q < XL; ++q) {
+            const int idx = lane + 64 * q;
+            if (idx < EW * NL) sF[idx / NL][idx % NL] = vx[q] + vu[q];
+        }
+#pragma unroll
+        for (int q = 0; q < TL; ++q) {
+            const int idx = lane + 64 * q;
+            if (idx < EW * 2 * NT) sT[idx / (2 * NT)][idx % (2 * NT)] = vt[q];
+        }
+    }
+    wave_sync();
     const bool prs = d.pressure != 0.0;
-    const int nf = (prs ? kFqP : kFq) * NG;
-    const size_t stride = (size_t)d.nel * NG;
-    const double *Fg = d.Hg + (size_t)e * NG;
-    double vf[FL], vt[TL];
+    {
+        const int lp = opaque(lane), el = min(lp / NG, ne - 1), g = lp % NG, qx = g % NQ, qy = g / NQ;
+        const double *geo = d.gpgeo + ((size_t)(e0 + el) * NG + g) * kGeoStride;
+        double gl[14];
 #pragma unroll
-    for (int q = 0; q < FL; ++q) {
-        const int idx = lane + 64 * q;
-        vf[q] = idx < nf ? Fg[(size_t)(idx / NG) * stride + idx % NG] : 0.0;
+        for (int r = 0; r < 14; ++r) gl[r] = geo[r];
+        double dv[15], f[kFq];
+        const double *xs = sF[el];
+        gp_derivatives<P, true>(sT[el] + qx * 3 * P1, sT[el] + NT + qy * 3 * P1,
+                          [&](int ia, int ib, int c) { return xs[3 * (ia + P1 * ib) + c]; }, dv);
+        __builtin_amdgcn_sched_barrier(0);
+        shell::gp_forces(dv, gl, d.t, f);
+        wave_sync();
+        if (lp / NG < EW) {  // a lane past the last element repeats it and writes rows nobody reads
+            double *F = sF[lp / NG] + g;
+#pragma unroll
+            for (int I = 0; I < kFq; ++I) F[I * NGP] = f[I];
+            if (prs) {  // -p w (a1 x a2) on the deformed surface: the follower load, as a force on the residual's side
+                double n[3];
+                shell::cross3(dv, dv + 3, n);
+                const double s = -d.pressure * gl[13];
+#pragma unroll
+                for (int i = 0; i < 3; ++i) F[(kFq + i) * NGP] = s * n[i];
+            }
+        }
     }
+    wave_sync();
+    // over qx: entry (el, r = (qy, ia, i)), the factors N, N', N'' along y
+    const int ls = opaque(lane);  // index arithmetic is repeated here instead of kept in registers
+    double t[XL][3];
 #pragma unroll
-    for (int q = 0; q < TL; ++q) {
-        const int idx = lane + 64 * q;
-        vt[q] = idx < NT ? d.tabx[(size_t)ex * NT + idx] : idx < 2 * NT ? d.taby[(size_t)ey * NT + idx - NT] : 0.0;
+    for (int q = 0; q < XL; ++q) {
+        __builtin_amdgcn_sched_barrier(0);
+        const int idx = min(ls + 64 * q, EW * NL - 1), el = idx / NL, r = idx % NL;
+        const int i = r % 3, ia = r / 3 % P1, qy = r / (3 * P1);
+        t[q][0] = t[q][1] = t[q][2] = 0.0;
+#pragma unroll
+        for (int qx = 0; qx < NQ; ++qx) {
+            const double *tx = sT[el] + qx * 3 * P1 + ia, *F = sF[el] + i * NGP + qx + NQ * qy;
+            t[q][0] += tx[P1] * F[0];
+            t[q][0] += tx[2 * P1] * F[6 * NGP];
+            t[q][1] += tx[0] * F[3 * NGP];
+            t[q][1] += tx[P1] * F[12 * NGP];
+            t[q][2] += tx[0] * F[9 * NGP];
+        }
+        if (prs) {
+#pragma unroll
+            for (int qx = 0; qx < NQ; ++qx) t[q][0] += sT[el][qx * 3 * P1 + ia] * sF[el][(kFq + i) * NGP + qx + NQ * qy];
+        }
     }
+    wave_sync();
 #pragma unroll
-    for (int q = 0; q < FL; ++q)
-        if (lane + 64 * q < kFqP * NG) sF[w][lane + 64 * q] = vf[q];
+    for (int q = 0; q < XL; ++q) {
+        const int idx = ls + 64 * q;
+        if (idx < EW * NL) {
 #pragma unroll
-    for (int q = 0; q < TL; ++q)
-        if (lane + 64 * q < 2 * NT) sT[w][lane + 64 * q] = vt[q];
-    // the wave reads what its other lanes wrote: LDS accesses of one wave complete in order, and
-    // the fence keeps the compiler from moving the reads above the writes
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-    if (lane >= 3 * NB) return;
-    const int A = lane / 3, i = lane % 3, ia = A % P1, ib = A / P1;
-    const double *F = sF[w];
-    // the follower-pressure term is a separate instantiation of the loop, so that the loop without
-    // it keeps no branch
-    auto sum = [&](auto with_pressure) {
+            for (int k = 0; k < 3; ++k) sF[idx / NL][k * NL + idx % NL] = t[q][k];
+        }
+    }
+    wave_sync();
+    const int lo = opaque(lane);
+#pragma unroll
+    for (int q = 0; q < XL; ++q) {
+        const int idx = lo + 64 * q, el = idx / NL, r = idx % NL;
+        if (el >= ne) break;
+        const int i = r % 3, A = r / 3, ia = A % P1, ib = A / P1;
         double acc = 0.0;
 #pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const int qx = g % NQ, qy = g / NQ;
-            const double *tx = sT[w] + qx * 3 * P1;
-            const double *ty = sT[w] + NT + qy * 3 * P1;
-            const double psi[5] = {tx[P1 + ia] * ty[ib], tx[ia] * ty[P1 + ib], tx[2 * P1 + ia] * ty[ib],
-                                   tx[ia] * ty[2 * P1 + ib], tx[P1 + ia] * ty[P1 + ib]};
+        for (int qy = 0; qy < NQ; ++qy) {
+            const double *ty = sT[el] + NT + qy * 3 * P1 + ib, *T = sF[el] + 3 * (ia + P1 * qy) + i;
 #pragma unroll
-            for (int a = 0; a < 5; ++a) acc += psi[a] * F[(3 * a + i) * NG + g];
-            if constexpr (decltype(with_pressure)::value) acc += tx[ia] * ty[ib] * F[(kFq + i) * NG + g];
+            for (int k = 0; k < 3; ++k) acc += ty[k * P1] * T[k * NL];
         }
-        return acc;
-    };
-    d.Fe[(size_t)e * 3 * NB + lane] = prs ? sum(std::true_type{}) : sum(std::false_type{});
+        d.Fe[(size_t)e0 * NL + idx] = acc;
+    }
 }
 
 // Tangent, stage 1: one thread per Gauss point.  Derivative vectors of the deformed surface,
@@ -189,18 +277,21 @@ __global__ __launch_bounds__(256) void k_residual_tiles(const InstDesc *descs, i
 // stored entry-major (Hg[q * ngp + gp]) so that a wave's stores are contiguous.  All indices
 // into the state are compile-time constants after unrolling, so it lives in registers.
 template <int P>
-__global__ __launch_bounds__(128) void k_tangent_gp(const InstDesc *descs, int ninst, int total)
+__global__ __launch_bounds__(128) void k_tangent_gp(const InstDesc *__restrict__ descs, int ninst)
 {
     constexpr int P1 = P + 1, NQ = P1, NG = NQ * NQ;
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= total) return;
-    const InstDesc &d = descs[find_inst(ninst, gid, [&](int m) { return (long long)descs[m].elem0 * NG; })];
-    const int gp = gid - d.elem0 * NG;
+    const int w = wave_index();
+    const InstDesc d = inst_desc(descs, ninst, w, [](const InstDesc &e) { return e.gp0; });
+    const int gp = (w - d.gp0) * 64 + (int)(threadIdx.x & 63);
+    if (gp >= d.nel * NG) return;
     const int e = gp / NG, g = gp % NG, ex = e % d.nx, ey = e / d.nx, qx = g % NQ, qy = g / NQ;
     const double *tx = d.tabx + ((size_t)(ex * NQ + qx) * 3) * P1;
     const double *ty = d.taby + ((size_t)(ey * NQ + qy) * 3) * P1;
     double dv[15];
-    gp_derivatives<P>(d, ex, ey, tx, ty, dv);
+    gp_derivatives<P, false>(tx, ty, [&](int ia, int ib, int c) {
+        const int cp = (ex + ia) + d.mx * (ey + ib);
+        return d.ctrl0[3 * cp + c] + d.u_full[3 * cp + c];
+    }, dv);
     double st[shell::kState];
     shell::gp_state(dv, d.gpgeo + (size_t)gp * kGeoStride, d.t, st);
     const size_t stride = (size_t)d.nel * NG;
@@ -226,13 +317,13 @@ __device__ __forceinline__ int hq_index(int I, int J)
 // it, from H_g (LDS broadcasts) and basis values (tables, L1).  The six tiles i <= k are
 // computed, and K_e's lower triangle is stored from them (the tiles i > k as transposes).
 template <int P, typename T, int E>
-__global__ __launch_bounds__(64 * E) void k_tangent_tiles(const InstDesc *descs, int ninst, int total_el)
+__global__ __launch_bounds__(64 * E) void k_tangent_tiles(const InstDesc *__restrict__ descs, int ninst, int total_el)
 {
     constexpr int P1 = P + 1, NB = P1 * P1, NQ = P1, NG = NQ * NQ, NKK = ((5 * NG + 3) / 4) * 4;
     using M = Mfma16<T>;
     const int eg = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * E + (threadIdx.x >> 6)));
     if (eg >= total_el) return;
-    const InstDesc &d = descs[find_inst(ninst, eg, [&](int m) { return (long long)descs[m].elem0; })];
+    const InstDesc d = inst_desc(descs, ninst, eg, [](const InstDesc &e) { return e.elem0; });
     const int e = eg - d.elem0, ex = e % d.nx, ey = e / d.nx;
     const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
     const int ia = li % P1, ib = li / P1;
@@ -243,9 +334,20 @@ __global__ __launch_bounds__(64 * E) void k_tangent_tiles(const InstDesc *descs,
     double(*sHw)[kHs] = sH[threadIdx.x >> 6];
     {
         const double *Hb = d.Hg + (size_t)e * NG;
-        for (int idx = lane; idx < NG * kHq; idx += 64) {
-            const int q = idx / NG, g = idx % NG;  // NG consecutive points of one entry: contiguous
-            sHw[g][q] = Hb[(size_t)q * stride + g];
+        constexpr int NLD = (NG * kHq + 63) / 64, kGrp = 10;  // loads per lane, in flight at a time
+#pragma unroll
+        for (int n0 = 0; n0 < NLD; n0 += kGrp) {
+            double v[kGrp];
+#pragma unroll
+            for (int n = 0; n < kGrp; ++n) {
+                const int idx = lane + 64 * (n0 + n), q = idx / NG, g = idx % NG;  // NG consecutive points of one entry: contiguous
+                if (n0 + n < NLD) v[n] = idx < NG * kHq ? Hb[(size_t)q * stride + g] : 0.0;
+            }
+#pragma unroll
+            for (int n = 0; n < kGrp; ++n) {
+                const int idx = lane + 64 * (n0 + n), q = idx / NG, g = idx % NG;
+                if (n0 + n < NLD && idx < NG * kHq) sHw[g][q] = v[n];
+            }
         }
         // the wave reads what its own lanes wrote: the LDS writes must be complete
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -349,12 +451,12 @@ __device__ __forceinline__ double ek_cross(int k, const double *a, int i)
 // matrix reads.  One wave per element, lane r = 3A + i; the element's Gauss-point data (a1, a2,
 // p w, N, N,1, N,2) staged in LDS.
 template <int P, typename T>
-__global__ __launch_bounds__(64) void k_pressure_tiles(const InstDesc *descs, int ninst, int total_el)
+__global__ __launch_bounds__(64) void k_pressure_tiles(const InstDesc *__restrict__ descs, int ninst, int total_el)
 {
     constexpr int P1 = P + 1, NB = P1 * P1, NQ = P1, NG = NQ * NQ;
     const int eg = (int)blockIdx.x;
     if (eg >= total_el) return;
-    const InstDesc &d = descs[find_inst(ninst, eg, [&](int m) { return (long long)descs[m].elem0; })];
+    const InstDesc d = inst_desc(descs, ninst, eg, [](const InstDesc &e) { return e.elem0; });
     if (d.pressure == 0.0) return;
     const int e = eg - d.elem0, ex = e % d.nx, ey = e / d.nx;
     const int lane = (int)threadIdx.x;
@@ -403,12 +505,12 @@ __global__ __launch_bounds__(64) void k_pressure_tiles(const InstDesc *descs, in
 
 // consistent mass tiles: M_e^{ii}[A][B] = sum_g rho t N_A N_B wdA
 template <int P, typename T>
-__global__ __launch_bounds__(256) void k_mass_elem(const InstDesc *descs, int ninst)
+__global__ __launch_bounds__(256) void k_mass_elem(const InstDesc *__restrict__ descs, int ninst)
 {
     constexpr int P1 = P + 1, NB = P1 * P1, NQ = P1, NG = NQ * NQ;
     __shared__ double sN[NG][16];
     __shared__ double sW[NG];
-    const InstDesc &d = descs[find_inst(ninst, blockIdx.x, [&](int m) { return (long long)descs[m].elem0; })];
+    const InstDesc d = inst_desc(descs, ninst, blockIdx.x, [](const InstDesc &e) { return e.elem0; });
     const int e = blockIdx.x - d.elem0, ex = e % d.nx, ey = e / d.nx;
     for (int idx = threadIdx.x; idx < NG * 16; idx += blockDim.x) {
         int g = idx / 16, A = idx % 16;
@@ -507,21 +609,31 @@ __global__ void k_setup_geometry(ElemArgs ar, const double *wq, double E, double
 // mode 3: R = -sum.  With a follower pressure the element sums hold F_int(u) - P(u), and the ALM
 // form adds P(0) (r = F_int - lambda F - (P(u) - P(0)), the reference's Force - lambda Force -
 // rhs(u) with Force = F_ext(0)); the static form is its negative.
-__global__ void k_vector_gather(const InstDesc *descs, int ninst, int total)
+template <int P>
+__global__ __launch_bounds__(256) void k_vector_gather(const InstDesc *__restrict__ descs, int ninst)
 {
-    int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= total) return;
-    const InstDesc &d = descs[find_inst(ninst, gid, [&](int m) { return (long long)descs[m].dof0; })];
-    int I = gid - d.dof0;
-    int p = d.p, P1 = p + 1, NB = P1 * P1;
-    int g = d.free2full[I], cp = g / 3, c = g % 3, i = cp % d.mx, j = cp / d.mx;
-    int exlo = max(i - p, 0), exhi = min(i, d.nx - 1), eylo = max(j - p, 0), eyhi = min(j, d.ny - 1);
-    double acc = 0.0;
-    for (int ey = eylo; ey <= eyhi; ++ey)
-        for (int ex = exlo; ex <= exhi; ++ex) {
-            int e = ex + d.nx * ey, A = (i - ex) + P1 * (j - ey);
-            acc += d.Fe[(size_t)e * 3 * NB + 3 * A + c];
+    constexpr int P1 = P + 1, NB = P1 * P1;
+    const int w = wave_index();
+    const InstDesc d = inst_desc(descs, ninst, w, [](const InstDesc &e) { return e.dof0; });
+    const int I = (w - d.dof0) * 64 + (int)(threadIdx.x & 63);
+    if (I >= d.nfree) return;
+    const int g = d.free2full[I], cp = g / 3, c = g % 3, i = cp % d.mx, j = cp / d.mx;
+    // every element's value is loaded before the first is added: one memory latency instead of
+    // one per element
+    double v[P1][P1];
+#pragma unroll
+    for (int b = 0; b < P1; ++b)
+#pragma unroll
+        for (int a = 0; a < P1; ++a) {
+            const int ex = i - P + a, ey = j - P + b;
+            const bool in = ex >= 0 && ex < d.nx && ey >= 0 && ey < d.ny;
+            v[b][a] = in ? d.Fe[(size_t)(ex + d.nx * ey) * 3 * NB + 3 * ((P - a) + P1 * (P - b)) + c] : 0.0;
         }
+    double acc = 0.0;
+#pragma unroll
+    for (int b = 0; b < P1; ++b)
+#pragma unroll
+        for (int a = 0; a < P1; ++a) acc += v[b][a];
     const double p0 = d.P0 ? d.P0[I] : 0.0;
     if (d.mode == 1) acc = acc - d.lambda * d.F[I] + p0;
     else if (d.mode == 2) acc = d.lambda * d.F[I] - acc - p0;
@@ -539,11 +651,11 @@ __global__ void k_vector_gather(const InstDesc *descs, int ninst, int total)
 // of its free dofs.  Slots no element reaches are never written: the band must hold 0 there (a
 // fresh band, or one zeroed by the launcher).  Reads each stored element entry once.
 template <int P, typename T>
-__global__ __launch_bounds__(256) void k_band_gather(const InstDesc *descs, int ninst)
+__global__ __launch_bounds__(256, 3) void k_band_gather(const InstDesc *__restrict__ descs, int ninst)
 {
     constexpr int P1 = P + 1, NPAIR = P1 + P * (2 * P + 1);
-    const long long chunk = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const InstDesc &d = descs[find_inst(ninst, chunk, [&](int m) { return descs[m].chunk0; })];
+    const int chunk = wave_index();
+    const InstDesc d = inst_desc(descs, ninst, chunk, [](const InstDesc &e) { return e.chunk0; });
     const long long t = (chunk - d.chunk0) * 64 + (threadIdx.x & 63);
     const int my = d.ny + P, ncp = d.mx * my;
     if (t >= (long long)ncp * NPAIR) return;
@@ -573,7 +685,9 @@ __global__ __launch_bounds__(256) void k_band_gather(const InstDesc *descs, int 
     for (int cJ = 0; cJ < 3; ++cJ)
 #pragma unroll
         for (int cI = 0; cI < 3; ++cI) acc[cJ][cI] = 0.0;
-#pragma unroll
+    // one row of elements (9 P1 loads) in flight at a time; all rows at once took 306 registers and
+    // left one wave per SIMD
+#pragma unroll 1
     for (int ty = 0; ty < P1; ++ty)
 #pragma unroll
         for (int tx = 0; tx < P1; ++tx) {
@@ -636,8 +750,9 @@ ElemArgs host_elem_args(const Problem &pb)
     return a;
 }
 
+// elements of the batch, and waves of its per-dof, per-Gauss-point and band-pair kernels
 struct Totals {
-    long long nel = 0, nfree = 0, ndof = 0, slots = 0, chunks = 0;
+    long long nel = 0, wfree = 0, wdof = 0, wgp = 0, wres = 0, slots = 0, chunks = 0;
 };
 
 // prefix offsets of a batch
@@ -645,15 +760,20 @@ Totals prefix(std::vector<InstDesc> &h)
 {
     Totals t;
     for (auto &d : h) {
+        const long long ngp = (long long)d.nel * (d.p + 1) * (d.p + 1);
         d.elem0 = (int)t.nel;
-        d.dof0 = (int)t.nfree;
-        d.full0 = (int)t.ndof;
+        d.dof0 = (int)t.wfree;
+        d.full0 = (int)t.wdof;
+        d.gp0 = (int)t.wgp;
+        d.res0 = (int)t.wres;
         const long long npair = (long long)(d.nx + d.p) * (d.ny + d.p) * ((d.p + 1) + d.p * (2 * d.p + 1));
         d.chunk0 = t.chunks;
         t.chunks += (npair + 63) / 64;
         t.nel += d.nel;
-        t.nfree += d.nfree;
-        t.ndof += d.ndof;
+        t.wfree += (d.nfree + 63) / 64;
+        t.wdof += (d.ndof + 63) / 64;
+        t.wgp += (ngp + 63) / 64;
+        t.wres += (d.nel + res_elements(d.p) - 1) / res_elements(d.p);
         t.slots += (long long)d.nfree * (d.bw + 1);
     }
     return t;
@@ -669,11 +789,21 @@ int check_batch(const std::vector<InstDesc> &h, bool band)
 {
     if (h.empty()) return fail(KSH_OTHER_ERROR, "empty batch");
     for (auto &d : h) {
+        if (d.p != 2 && d.p != 3) return fail(KSH_OTHER_ERROR, "spline degree is neither 2 nor 3");
         if (d.p != h[0].p) return fail(KSH_OTHER_ERROR, "batch mixes spline degrees");
         if (band && d.sprec != h[0].sprec) return fail(KSH_OTHER_ERROR, "batch mixes band precisions");
         if (band && (size_t)d.nel * kKeTile * sizeof(double) >= 0x80000000ull)
             return fail(KSH_OTHER_ERROR, "element matrices of 2 GiB or more: beyond the gather's 32-bit offsets");
     }
+    return KSH_SUCCESS;
+}
+
+int launch_vector_gather(hipStream_t s, const InstDesc *d_desc, const std::vector<InstDesc> &h, const Totals &t)
+{
+    const dim3 g(nblk(t.wfree, 4)), b(256);
+    if (h[0].p == 2) hipLaunchKernelGGL(k_vector_gather<2>, g, b, 0, s, d_desc, (int)h.size());
+    else hipLaunchKernelGGL(k_vector_gather<3>, g, b, 0, s, d_desc, (int)h.size());
+    KSH_HIP(hipGetLastError());
     return KSH_SUCCESS;
 }
 
@@ -685,25 +815,17 @@ int run_residual(hipStream_t s, InstDesc *d_desc, std::vector<InstDesc> &h, bool
     const int n = (int)h.size();
     if ((rc = upload_descs(s, d_desc, h))) return rc;
     if (construct)
-        hipLaunchKernelGGL(k_construct_solution, dim3(nblk(t.ndof, 256)), dim3(256), 0, s, d_desc, n, (int)t.ndof);
+        hipLaunchKernelGGL(k_construct_solution, dim3(nblk(t.wdof, 4)), dim3(256), 0, s, d_desc, n);
     {
         ProfScope ps("residual_elem", s);
         const long long ng = (h[0].p + 1LL) * (h[0].p + 1LL), ngp = t.nel * ng;
         if (ngp >= (1LL << 31)) return fail(KSH_OTHER_ERROR, "batch has 2^31 or more Gauss points");
-        const dim3 gg(nblk(ngp, 128)), ge(nblk(t.nel, 4));
-        if (h[0].p == 2) {
-            hipLaunchKernelGGL(k_residual_gp<2>, gg, dim3(128), 0, s, d_desc, n, (int)ngp);
-            hipLaunchKernelGGL(k_residual_tiles<2>, ge, dim3(256), 0, s, d_desc, n, (int)t.nel);
-        } else {
-            hipLaunchKernelGGL(k_residual_gp<3>, gg, dim3(128), 0, s, d_desc, n, (int)ngp);
-            hipLaunchKernelGGL(k_residual_tiles<3>, ge, dim3(256), 0, s, d_desc, n, (int)t.nel);
-        }
+        if (h[0].p == 2) hipLaunchKernelGGL(k_residual_elem<2>, dim3((unsigned)t.wres), dim3(64), 0, s, d_desc, n);
+        else hipLaunchKernelGGL(k_residual_elem<3>, dim3((unsigned)t.wres), dim3(64), 0, s, d_desc, n);
     }
     KSH_HIP(hipGetLastError());
     ProfScope ps("vector_gather", s);
-    hipLaunchKernelGGL(k_vector_gather, dim3(nblk(t.nfree, 256)), dim3(256), 0, s, d_desc, n, (int)t.nfree);
-    KSH_HIP(hipGetLastError());
-    return KSH_SUCCESS;
+    return launch_vector_gather(s, d_desc, h, t);
 }
 
 int run_tangent(hipStream_t s, InstDesc *d_desc, std::vector<InstDesc> &h, bool construct, bool mass)
@@ -714,7 +836,7 @@ int run_tangent(hipStream_t s, InstDesc *d_desc, std::vector<InstDesc> &h, bool 
     const int n = (int)h.size();
     if ((rc = upload_descs(s, d_desc, h))) return rc;
     if (construct)
-        hipLaunchKernelGGL(k_construct_solution, dim3(nblk(t.ndof, 256)), dim3(256), 0, s, d_desc, n, (int)t.ndof);
+        hipLaunchKernelGGL(k_construct_solution, dim3(nblk(t.wdof, 4)), dim3(256), 0, s, d_desc, n);
     const bool f64 = h[0].sprec == KSH_FP64, p2 = h[0].p == 2;
     const dim3 g((unsigned)t.nel), b(256);
     if (mass) {
@@ -728,8 +850,8 @@ int run_tangent(hipStream_t s, InstDesc *d_desc, std::vector<InstDesc> &h, bool 
         {
             ProfScope ps("tangent_gp", s);
             ps.set_work((double)ngp * (kHq + kGeoStride) * 8.0);  // H_g written, undeformed geometry read (bytes)
-            if (p2) hipLaunchKernelGGL(k_tangent_gp<2>, dim3(nblk(ngp, 128)), dim3(128), 0, s, d_desc, n, (int)ngp);
-            else hipLaunchKernelGGL(k_tangent_gp<3>, dim3(nblk(ngp, 128)), dim3(128), 0, s, d_desc, n, (int)ngp);
+            if (p2) hipLaunchKernelGGL(k_tangent_gp<2>, dim3(nblk(t.wgp, 2)), dim3(128), 0, s, d_desc, n);
+            else hipLaunchKernelGGL(k_tangent_gp<3>, dim3(nblk(t.wgp, 2)), dim3(128), 0, s, d_desc, n);
         }
         ProfScope ps("tangent_elem", s);
         double work = 0.0;  // B^T D B count per element and Gauss point: 72 n_e + 12 n_e^2
@@ -830,7 +952,7 @@ int batch_construct(hipStream_t s, InstDesc *d_desc, const std::vector<InstDesc>
     Totals t = prefix(h);
     int rc;
     if ((rc = upload_descs(s, d_desc, h))) return rc;
-    hipLaunchKernelGGL(k_construct_solution, dim3(nblk(t.ndof, 256)), dim3(256), 0, s, d_desc, (int)h.size(), (int)t.ndof);
+    hipLaunchKernelGGL(k_construct_solution, dim3(nblk(t.wdof, 4)), dim3(256), 0, s, d_desc, (int)h.size());
     KSH_HIP(hipGetLastError());
     return KSH_SUCCESS;
 }
@@ -883,15 +1005,13 @@ int launch_residual(Problem &pb, double lambda, int conv, double *R_dev)
     return run_residual(pb.stream, pb.d_desc, h, false);
 }
 
-// residual with caller-chosen partial-result storage (u_full: ndof, Hg: kFq ngp, or kFqP ngp with a follower
-// pressure, Fe: 3 nb nel doubles)
+// residual with caller-chosen partial-result storage (u_full: ndof, Fe: 3 nb nel doubles)
 int run_residual_into(Problem &pb, const double *u_free_dev, double lambda, int conv, double *R_dev, double *u_full,
-                      double *Hg, double *Fe)
+                      double *Fe)
 {
     InstDesc d = make_desc(pb);
     d.u_free = u_free_dev;
     d.u_full = u_full;
-    d.Hg = Hg;
     d.Fe = Fe;
     d.lambda = lambda;
     d.mode = (conv == KSH_RES_ALM) ? 1 : 2;
@@ -942,11 +1062,10 @@ int launch_external_force(Problem &pb)
         d.mode = 0;
         d.R = pb.F;
         std::vector<InstDesc> h = {d};
-        prefix(h);
+        const Totals t = prefix(h);
         int rc;
         if ((rc = upload_descs(pb.stream, pb.d_desc, h))) return rc;
-        hipLaunchKernelGGL(k_vector_gather, dim3(nblk(pb.nfree, 256)), dim3(256), 0, pb.stream, pb.d_desc, 1, pb.nfree);
-        KSH_HIP(hipGetLastError());
+        if ((rc = launch_vector_gather(pb.stream, pb.d_desc, h, t))) return rc;
     }
     if (pb.npoint > 0) {
         hipLaunchKernelGGL(k_point_loads, dim3(1), dim3(1), 0, pb.stream, pb.npoint, pb.p, pb.mx, pb.free_idx, pb.pl_N,

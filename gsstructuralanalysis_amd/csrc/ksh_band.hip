@@ -12,6 +12,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "ksh_devutil.hpp"
 #include "ksh_internal.hpp"
 #include "ksh_mfma.hpp"
 #include "ksh_profile.hpp"
@@ -82,7 +83,7 @@ __global__ void k_convert(TD *dst, const TS *src, size_t count)
 // binary search over the chunk offsets.  The conversion is the same per entry either way.
 constexpr int kCopyPer = 8, kCopyBlk = 256 * kCopyPer;
 
-__global__ __launch_bounds__(256) void k_copy_batched(const CopyDesc *descs, int nband)
+__global__ __launch_bounds__(256) void k_copy_batched(const CopyDesc *__restrict__ descs, int nband)
 {
     const long long blk = blockIdx.x;
     int lo = 0, hi = nband - 1;
@@ -91,7 +92,9 @@ __global__ __launch_bounds__(256) void k_copy_batched(const CopyDesc *descs, int
         if (descs[mid].blk0 <= blk) lo = mid;
         else hi = mid - 1;
     }
-    const CopyDesc &d = descs[lo];
+    CopyDesc d = descs[lo];
+    d.src = global_ptr(d.src);
+    d.dst = global_ptr(d.dst);
     const size_t i0 = (size_t)(blk - d.blk0) * kCopyBlk + (size_t)threadIdx.x * kCopyPer;
     if (i0 >= d.count) return;
     const bool f64s = d.src_prec == KSH_FP64, f64d = d.dst_prec == KSH_FP64;

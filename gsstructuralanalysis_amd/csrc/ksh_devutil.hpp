@@ -16,6 +16,15 @@ __device__ __forceinline__ T *uniform_ptr(T *p)
     return (T *)(((unsigned long long)hi << 32) | lo);
 }
 
+// the same pointer, stated to be one to global memory (a pointer read from memory is a generic one
+// to the compiler, and a flat access waits for every memory and LDS access in flight); by way of an
+// integer, since a pair of pointer casts is folded away
+template <typename T>
+__device__ __forceinline__ T *global_ptr(T *p)
+{
+    return (T *)(__attribute__((address_space(1))) T *)(unsigned long long)p;
+}
+
 // broadcast of lane `src`'s value (v_readlane: the result is wave-uniform)
 __device__ __forceinline__ double readlane_f64(double v, int src)
 {

@@ -49,8 +49,8 @@ int fail(int code, const std::string &msg);
 struct InstDesc {
     int p, nx, ny, mx, nel, nfree, bw, ndof;
     int elem0;              // first element of this instance in the launch
-    int dof0;               // first free dof
-    int full0;              // first full dof
+    int dof0, full0;        // first wave of its free dofs and of its full dofs, 64 a wave
+    int gp0, res0;          // first wave of its Gauss points, 64 a wave, and of k_residual_elem
     int skip_zero;          // 1: band slots no element reaches already hold 0 in ab and are not stored
     long long chunk0;       // band gather: first 64-thread chunk of this instance
     double t, rho, lambda;
@@ -59,7 +59,7 @@ struct InstDesc {
     const int *free_idx, *free2full;
     double *u_full, *Fe, *R;
     void *Ke, *ab;
-    double *Hg;             // per-Gauss-point H_g (upper triangle, kHq entries), entry-major
+    double *Hg;             // per-Gauss-point H_g (upper triangle, kHq entries), entry-major (tangent)
     double pressure;        // follower pressure along a1 x a2 (0: none)
     const double *P0;       // its load on the undeformed surface (free dofs; with a pressure)
 };

@@ -1,7 +1,7 @@
 // ksh_noalloc.hip -- ksh_assemble_residual_dev_noalloc: the residual of ksh_assemble_residual_dev
 // for callers that cannot allocate device memory (code under HIP graph capture, tight serving
-// loops).  Its partial results -- the full control-net displacement, the per-Gauss-point stress
-// resultants and the element force vectors -- go to a fixed device array of this library, one per
+// loops).  Its partial results -- the full control-net displacement and the element force vectors
+// (the per-Gauss-point stress resultants stay on chip) -- go to a fixed device array of this library, one per
 // GPU, instead of the problem's own workspace; nothing is allocated or freed per call.
 //
 // `scratch` is a file-scope device array: its host-side name is only a stand-in, so its address on
@@ -20,7 +20,7 @@
 namespace ksh {
 
 int run_residual_into(Problem &pb, const double *u_free_dev, double lambda, int conv, double *R_dev, double *u_full,
-                      double *Hg, double *Fe);
+                      double *Fe);
 
 namespace {
 
@@ -53,11 +53,11 @@ int scratch_ptr(int device, double **out)
 
 }  // namespace
 
-// resultants per Gauss point of one residual evaluation (three more with a follower pressure)
+// resultants per Gauss point (three more with a follower pressure)
 size_t noalloc_fq(const Problem &pb) { return pb.pressure != 0.0 ? (size_t)kFqP : (size_t)kFq; }
 
-// scratch doubles one residual evaluation of `pb` needs: u_full, the resultants per Gauss point,
-// element force vectors
+// the size by which a problem is accepted: u_full, element force vectors and, though no longer
+// stored, the resultants per Gauss point, so that the accepted problems stay what they were
 size_t noalloc_residual_doubles(const Problem &pb)
 {
     return (size_t)pb.ndof + noalloc_fq(pb) * (size_t)pb.ngp + 3ull * (size_t)pb.nb * (size_t)pb.nel + 3 * 32;
@@ -82,8 +82,7 @@ extern "C" int ksh_assemble_residual_dev_noalloc(ksh_problem *pb, const double *
     // 256-byte aligned sub-arrays
     auto align = [](size_t n) { return (n + 31) & ~size_t(31); };
     double *u_full = base;
-    double *Hg = u_full + align((size_t)pb->ndof);
-    double *Fe = Hg + align(noalloc_fq(*pb) * (size_t)pb->ngp);
-    if ((rc = run_residual_into(*pb, u_free_dev, lambda, conv, R_out_dev, u_full, Hg, Fe))) return fail(KSH_ASSEMBLY_ERROR, ksh_last_error());
+    double *Fe = u_full + align((size_t)pb->ndof);
+    if ((rc = run_residual_into(*pb, u_free_dev, lambda, conv, R_out_dev, u_full, Fe))) return fail(KSH_ASSEMBLY_ERROR, ksh_last_error());
     return KSH_SUCCESS;
 }

@@ -5,7 +5,7 @@
 // kappa = b_ab - B_ab with respect to a control-point displacement u_{A,i} is linear in the
 // 15-vector phi_{A,i} = (N_A,1 e_i, N_A,2 e_i, N_A,11 e_i, N_A,22 e_i, N_A,12 e_i); every second
 // variation is a bilinear form in two of them.  gp_state() gathers the per-point quantities,
-// h_entry() gives H_g[I][J] (K_{(A,i),(B,k)} = phi^T H_g phi) and f_entry() gives f_g[I]
+// h_entry() gives H_g[I][J] (K_{(A,i),(B,k)} = phi^T H_g phi) and gp_forces() gives f_g
 // (f_int_{A,i} = phi . f_g).  Formulation: Kiendl et al. 2009, CMAME 198:3902.
 #pragma once
 
@@ -194,12 +194,39 @@ __device__ double h_entry(const double *s, int I, int J)
     return h;
 }
 
-__device__ inline double f_entry(const double *s, int I)
+// f_g alone, without the state: with n^, m^ the stress resultants, mh = m11 a11 + m22 a22 +
+// 2 m12 a12 and q = (mh - (mh . a3) a3) / j, the variation of a3 contracts to cross products,
+// mh . d a3 = q . (d a1 x a2 + a1 x d a2), so that
+//   f = (n11 a1 + n12 a2 + a2 x q, n12 a1 + n22 a2 + q x a1, m11 a3, m22 a3, 2 m12 a3)
+__device__ __forceinline__ void gp_forces(const double *dv, const double *geo, double t, double *f)
 {
-    double m[3], b[3];
-    bcol(s, I, m, b);
-    return m[0] * s[S_NV] + m[1] * s[S_NV + 1] + m[2] * s[S_NV + 2] + b[0] * s[S_MV] + b[1] * s[S_MV + 1] +
-           b[2] * s[S_MV + 2];
+    const double *a1 = dv, *a2 = dv + 3, *a11 = dv + 6, *a22 = dv + 9, *a12 = dv + 12, *C = geo + 1;
+    double a3[3];
+    cross3(a1, a2, a3);
+    const double j = sqrt(dot3(a3, a3));
+    for (int i = 0; i < 3; ++i) a3[i] /= j;  // as the undeformed a3 was formed: their rounding cancels in the strains
+    const double ev[3] = {0.5 * (dot3(a1, a1) - geo[7]), 0.5 * (dot3(a2, a2) - geo[8]), dot3(a1, a2) - geo[9]};
+    const double kv[3] = {dot3(a11, a3) - geo[10], dot3(a22, a3) - geo[11], 2.0 * (dot3(a12, a3) - geo[12])};
+    const double fm = t * geo[0], fb = t * t * t / 12.0 * geo[0];
+    double nv[3], mu[3];
+    for (int r = 0; r < 3; ++r) {
+        nv[r] = fm * (sym3(C, r, 0) * ev[0] + sym3(C, r, 1) * ev[1] + sym3(C, r, 2) * ev[2]);
+        mu[r] = fb * (sym3(C, r, 0) * kv[0] + sym3(C, r, 1) * kv[1] + sym3(C, r, 2) * kv[2]);
+    }
+    mu[2] *= 2.0;
+    double q[3], x1[3], x2[3];
+    for (int i = 0; i < 3; ++i) q[i] = mu[0] * a11[i] + mu[1] * a22[i] + mu[2] * a12[i];
+    const double ma = dot3(q, a3);
+    for (int i = 0; i < 3; ++i) q[i] = (q[i] - ma * a3[i]) / j;
+    cross3(a2, q, x1);
+    cross3(q, a1, x2);
+    for (int i = 0; i < 3; ++i) {
+        f[i] = nv[0] * a1[i] + nv[2] * a2[i] + x1[i];
+        f[3 + i] = nv[1] * a2[i] + nv[2] * a1[i] + x2[i];
+        f[6 + i] = mu[0] * a3[i];
+        f[9 + i] = mu[1] * a3[i];
+        f[12 + i] = mu[2] * a3[i];
+    }
 }
 
 struct ElemArgs {

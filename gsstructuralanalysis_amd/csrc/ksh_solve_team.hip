@@ -205,8 +205,16 @@ __global__ __launch_bounds__(256) void k_team_prep(TeamDesc one, const TeamDesc 
     __shared__ double ns[kB][kB + 1];  // L_{k,k-1}
     __shared__ double ms[kB][kB + 1];  // M_k
     __shared__ double op[4][4 * 64];   // inverse of 16 x 16 block c as an MFMA operand
-    const TeamDesc d = many ? many[blockIdx.y] : one;
-    const int n = d.n, bw = d.bw, nblk = (n + kB - 1) / kB, k = (int)blockIdx.x;
+    TeamDesc d = many ? many[blockIdx.y] : one;
+    d.fac = uniform_ptr(d.fac);  // else the band is read in loops over distinct resources
+    d.y = global_ptr(d.y);
+    d.xo = global_ptr(d.xo);
+    d.cf = global_ptr(d.cf);
+    d.cb = global_ptr(d.cb);
+    d.ctl = global_ptr(d.ctl);
+    d.mat = global_ptr(uniform_ptr(d.mat));
+    const int n = __builtin_amdgcn_readfirstlane(d.n), bw = __builtin_amdgcn_readfirstlane(d.bw);
+    const int nblk = (n + kB - 1) / kB, k = (int)blockIdx.x;
     if (k >= nblk) return;
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -13,6 +13,7 @@
 // block order (deterministic).
 #include <hip/hip_runtime.h>
 
+#include "ksh_devutil.hpp"
 #include "ksh_internal.hpp"
 #include "ksh_profile.hpp"
 
@@ -106,7 +107,8 @@ __global__ __launch_bounds__(kT) void k_symv_rows(const T *ab, int n, int bw, co
     if (threadIdx.x < kRows && i0 + threadIdx.x < n) y[i0 + threadIdx.x] = v[0];
 }
 
-__device__ inline int find_block(const RefDesc *d, int n, int blk)
+// the descriptor that row block blk belongs to, its pointers stated to be global memory
+__device__ inline RefDesc find_block(const RefDesc *d, int n, int blk)
 {
     int lo = 0, hi = n - 1;
     while (lo < hi) {
@@ -114,7 +116,17 @@ __device__ inline int find_block(const RefDesc *d, int n, int blk)
         if (d[mid].blk0 <= blk) lo = mid;
         else hi = mid - 1;
     }
-    return lo;
+    RefDesc r = d[lo];
+    r.ab = global_ptr(r.ab);
+    r.b = global_ptr(r.b);
+    r.x = global_ptr(r.x);
+    r.r = global_ptr(r.r);
+    r.part = global_ptr(r.part);
+    r.b2 = global_ptr(r.b2);
+    r.x2 = global_ptr(r.x2);
+    r.r2 = global_ptr(r.r2);
+    r.part2 = global_ptr(r.part2);
+    return r;
 }
 
 // r = b - K x on one row block of one matrix (and r2 = b2 - K x2 with the same band loads when the
@@ -156,9 +168,9 @@ __device__ __forceinline__ void refine_rows(const RefDesc &d, int lb)
     }
 }
 
-__global__ __launch_bounds__(kT) void k_refine_rows_batched(const RefDesc *descs, int ninst)
+__global__ __launch_bounds__(kT) void k_refine_rows_batched(const RefDesc *__restrict__ descs, int ninst)
 {
-    const RefDesc &d = descs[find_block(descs, ninst, blockIdx.x)];
+    const RefDesc d = find_block(descs, ninst, blockIdx.x);
     if (!d.active) return;
     const int lb = blockIdx.x - d.blk0;
     if (d.x2)
@@ -173,22 +185,33 @@ __global__ __launch_bounds__(64) void k_refine_norms_batched(const RefDesc *desc
     const RefDesc &d = descs[blockIdx.x];
     if (!d.active) return;
     if (threadIdx.x < 2) {
-        const double *part = threadIdx.x == 0 ? d.part : d.part2;
-        double *norms = threadIdx.x == 0 ? d.norms : d.norms2;
+        const double *part = global_ptr(threadIdx.x == 0 ? d.part : d.part2);
+        double *norms = global_ptr(threadIdx.x == 0 ? d.norms : d.norms2);
         if (!part) return;
         double rr = 0.0, bb = 0.0;
-        for (int k = 0; k < d.nblk; ++k) {
-            rr += part[2 * k];
-            bb += part[2 * k + 1];
+        const int last = d.nblk - 1;
+        for (int k0 = 0; k0 <= last; k0 += kU) {  // kU blocks' loads in flight, added in block order
+            double v[kU], w[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                v[u] = part[2 * min(k0 + u, last)];
+                w[u] = part[2 * min(k0 + u, last) + 1];
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (k0 + u <= last) {
+                    rr += v[u];
+                    bb += w[u];
+                }
         }
         norms[0] = rr;
         norms[1] = bb;
     }
 }
 
-__global__ __launch_bounds__(kT) void k_refine_update_batched(const RefDesc *descs, int ninst)
+__global__ __launch_bounds__(kT) void k_refine_update_batched(const RefDesc *__restrict__ descs, int ninst)
 {
-    const RefDesc &d = descs[find_block(descs, ninst, blockIdx.x)];
+    const RefDesc d = find_block(descs, ninst, blockIdx.x);
     if (!d.active) return;
     const int i = (blockIdx.x - d.blk0) * kRows + threadIdx.x;
     if (threadIdx.x < kRows && i < d.n) d.x[i] += d.r[i];

@@ -3,7 +3,7 @@
 //
 // Every vector of every instance of a batch lives in device memory; the engine's host logic only
 // ever sees scalars.  One launch serves all instances of a round:
-//   k_dots      one workgroup per instance, up to kMaxDots dot products of length n in one pass;
+//   k_dots      one workgroup per instance and dot product of length n (up to kMaxDots);
 //               lanes stride over the entries, then a fixed-order reduction (wave shuffles, then
 //               the four wave sums in order), so results are bit-reproducible run to run;
 //   k_vecops    per instance a short program of 3-term combinations dst = a x + b y + c z,
@@ -17,6 +17,9 @@
 // All are HBM / latency bound and tiny next to the assembly and the factor.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
+#include "ksh_devutil.hpp"
 #include "ksh_internal.hpp"
 #include "ksh_vec.hpp"
 
@@ -33,34 +36,40 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
+// Latency bound: a workgroup holds kDots entries a lane in flight, and every product has its own
+// workgroup: 18 us for the up to ten products of 256 roofs of 16..48 elements a side, 61 us with all
+// of an instance's products in one workgroup, one entry a lane at a time.
+constexpr int kDots = 8;
+
 __global__ __launch_bounds__(kT) void k_dots(const DotDesc *__restrict__ descs)
 {
     const DotDesc &D = descs[blockIdx.x];
-    const int np = D.npairs;
-    double acc[kMaxDots];
+    const int k = blockIdx.y, n = D.n;
+    if (k >= D.npairs) return;
+    const double *a = global_ptr(D.a[k]), *b = global_ptr(D.b[k]);
+    double acc = 0.0;
+    for (int i0 = threadIdx.x; i0 < n; i0 += kDots * kT) {
+        double va[kDots], vb[kDots];
 #pragma unroll
-    for (int k = 0; k < kMaxDots; ++k) acc[k] = 0.0;
-    for (int i = threadIdx.x; i < D.n; i += kT) {
-#pragma unroll
-        for (int k = 0; k < kMaxDots; ++k)
-            if (k < np) acc[k] += D.a[k][i] * D.b[k][i];
-    }
-    __shared__ double part[kMaxDots][kT / 64];
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-#pragma unroll
-    for (int k = 0; k < kMaxDots; ++k) {
-        if (k < np) {
-            const double s = wave_sum(acc[k]);
-            if (lane == 0) part[k][wave] = s;
+        for (int q = 0; q < kDots; ++q) {
+            const int i = min(i0 + q * kT, n - 1);
+            va[q] = a[i];
+            vb[q] = b[i];
         }
+#pragma unroll
+        for (int q = 0; q < kDots; ++q)
+            if (i0 + q * kT < n) acc += va[q] * vb[q];
     }
+    __shared__ double part[kT / 64];
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    acc = wave_sum(acc);
+    if (lane == 0) part[wave] = acc;
     __syncthreads();
-    if (threadIdx.x < np) {
-        const int k = threadIdx.x;
+    if (threadIdx.x == 0) {
         double s = 0.0;
 #pragma unroll
-        for (int w = 0; w < kT / 64; ++w) s += part[k][w];
-        D.out[k] = s;
+        for (int w = 0; w < kT / 64; ++w) s += part[w];
+        global_ptr(D.out)[k] = s;
     }
 }
 
@@ -70,12 +79,12 @@ __global__ __launch_bounds__(kT) void k_vecops(const VecDesc *__restrict__ descs
     const int i = blockIdx.x * kT + threadIdx.x;
     if (i >= D.n) return;
     for (int k = 0; k < D.nops; ++k) {
-        const VecOp &o = D.op[k];
+        const VecOp o = D.op[k];
         double v = 0.0;
-        if (o.x) v = o.a * o.x[i];
-        if (o.y) v += o.b * o.y[i];
-        if (o.z) v += o.c * o.z[i];
-        o.dst[i] = v;
+        if (o.x) v = o.a * global_ptr(o.x)[i];
+        if (o.y) v += o.b * global_ptr(o.y)[i];
+        if (o.z) v += o.c * global_ptr(o.z)[i];
+        global_ptr(o.dst)[i] = v;
     }
 }
 
@@ -83,7 +92,11 @@ constexpr int kChunk = 2048;  // control points staged in LDS per pass
 
 __global__ __launch_bounds__(kT) void k_features(const FeatDesc *__restrict__ descs)
 {
-    const FeatDesc &D = descs[blockIdx.x];
+    FeatDesc D = descs[blockIdx.x];
+    D.P = global_ptr(D.P);
+    D.zfree = global_ptr(D.zfree);
+    D.U = global_ptr(D.U);
+    D.out = global_ptr(D.out);
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     __shared__ double z[kChunk];
     __shared__ double red[kT / 64];
@@ -129,7 +142,11 @@ __global__ __launch_bounds__(kT) void k_features(const FeatDesc *__restrict__ de
 
 __global__ __launch_bounds__(kT) void k_decode(const DecDesc *__restrict__ descs)
 {
-    const DecDesc &D = descs[blockIdx.y];
+    DecDesc D = descs[blockIdx.y];
+    D.Phi = global_ptr(D.Phi);
+    D.zfree = global_ptr(D.zfree);
+    D.coef = global_ptr(D.coef);
+    D.dU = global_ptr(D.dU);
     const int c = blockIdx.x * kT + threadIdx.x;
     if (c >= D.ncp) return;
     const int f = D.zfree[c];
@@ -141,36 +158,61 @@ __global__ __launch_bounds__(kT) void k_decode(const DecDesc *__restrict__ descs
     D.dU[f] += D.scale * s;
 }
 
+// One workgroup per instance (its norms need no second launch), so the largest instance's chain of
+// memory latencies is its time: each lane has kDr entries of every vector in flight.  Over 64 roofs
+// of 16..48 elements a side, one entry at a time took 51 us; 14 us.
+constexpr int kDr = 8;
+
 __global__ __launch_bounds__(kT) void k_dr(const DrDesc *__restrict__ descs)
 {
-    const DrDesc &D = descs[blockIdx.x];
+    const DrDesc D = descs[blockIdx.x];
+    const double *R = global_ptr(D.R), *m = global_ptr(D.m), *minv = global_ptr(D.minv), *damp = global_ptr(D.damp);
+    const double *U = global_ptr(D.U);
+    double *gv = global_ptr(D.v), *gdU = global_ptr(D.dU), *gDU = global_ptr(D.DU), *X = global_ptr(D.X);
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     __shared__ double red[4][kT / 64];
     const double dt = D.dt;
     double s[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int i = threadIdx.x; i < D.n; i += kT) {
-        double r = D.R[i], v = D.v[i], du;
-        if (D.mode == 0) {
-            du = 0.5 * dt * dt * D.minv[i] * r;
-            v = du / dt;
-        } else if (D.mode == 1) {
-            r -= D.damp[i] * v;
-            v += dt * D.minv[i] * r;
-            du = dt * v;
-        } else {
-            r -= D.damp[i] * v;
-            du = -1.5 * dt * v + 0.5 * dt * dt * D.minv[i] * r;
-            v = 0.0;
+    for (int i0 = threadIdx.x; i0 < D.n; i0 += kDr * kT) {
+        double lr[kDr], lv[kDr], lmi[kDr], lm[kDr], ld[kDr], lU[kDr], lD[kDr];
+#pragma unroll
+        for (int q = 0; q < kDr; ++q) {
+            const int i = min(i0 + q * kT, D.n - 1);
+            lr[q] = R[i];
+            lv[q] = gv[i];
+            lmi[q] = minv[i];
+            lm[q] = m[i];
+            ld[q] = D.mode != 0 ? damp[i] : 0.0;
+            lU[q] = U[i];
+            lD[q] = gDU[i];
         }
-        const double DU = D.DU[i] + du;
-        D.v[i] = v;
-        D.dU[i] = du;
-        D.DU[i] = DU;
-        D.X[i] = D.U[i] + DU;
-        s[0] += r * r;
-        s[1] += v * (D.m[i] * v);
-        s[2] += du * du;
-        s[3] += DU * DU;
+#pragma unroll
+        for (int q = 0; q < kDr; ++q) {
+            const int i = i0 + q * kT;
+            if (i >= D.n) break;
+            double r = lr[q], v = lv[q], du;
+            if (D.mode == 0) {
+                du = 0.5 * dt * dt * lmi[q] * r;
+                v = du / dt;
+            } else if (D.mode == 1) {
+                r -= ld[q] * v;
+                v += dt * lmi[q] * r;
+                du = dt * v;
+            } else {
+                r -= ld[q] * v;
+                du = -1.5 * dt * v + 0.5 * dt * dt * lmi[q] * r;
+                v = 0.0;
+            }
+            const double DU = lD[q] + du;
+            gv[i] = v;
+            gdU[i] = du;
+            gDU[i] = DU;
+            X[i] = lU[q] + DU;
+            s[0] += r * r;
+            s[1] += v * (lm[q] * v);
+            s[2] += du * du;
+            s[3] += DU * DU;
+        }
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -181,7 +223,7 @@ __global__ __launch_bounds__(kT) void k_dr(const DrDesc *__restrict__ descs)
     if (threadIdx.x < 4) {
         double t = 0.0;
         for (int w = 0; w < kT / 64; ++w) t += red[threadIdx.x][w];
-        D.out[threadIdx.x] = t;
+        global_ptr(D.out)[threadIdx.x] = t;
     }
 }
 
@@ -219,7 +261,9 @@ int batch_dots(hipStream_t s, DevScratch &desc_buf, const std::vector<DotDesc> &
         if (d.npairs < 0 || d.npairs > kMaxDots || d.n < 0 || !d.out) return fail(KSH_OTHER_ERROR, "dot descriptor");
     int rc;
     if ((rc = upload_descs(s, desc_buf, h))) return rc;
-    hipLaunchKernelGGL(k_dots, dim3((unsigned)h.size()), dim3(kT), 0, s, (const DotDesc *)desc_buf.p);
+    int most = 1;
+    for (const DotDesc &d : h) most = std::max(most, d.npairs);
+    hipLaunchKernelGGL(k_dots, dim3((unsigned)h.size(), (unsigned)most), dim3(kT), 0, s, (const DotDesc *)desc_buf.p);
     KSH_HIP(hipGetLastError());
     return KSH_SUCCESS;
 }
