@@ -49,19 +49,29 @@ constexpr int kBandMax = 512;    // widest band of the LDS-resident kernel
 // block).  Backward: wave w owns NK of the block's columns, one near row chunk (the next block's
 // rows) and BK far row chunks each.  FC: far registers consumed and refilled per scheduling
 // group; RC: diagonal-block entries per recurrence register run.
+//
+// What bounds it is the rate at which one CU takes a band from memory, about 20 bytes a cycle (4.0 us a
+// block and sweep at half-width 326 in FP64, 5.0 us at 470), or HBM where every CU has a band; below
+// that, the instructions of a block.  So the body is compiled for NC = 1 .. kClasses groups of far
+// columns (and the far row chunks that the widest such band has), and a workgroup takes the
+// narrowest that covers its band: loads beyond the band read nothing, but cost their issue slots.
+// The entries left out are zeros of every sum, so the class does not show in the result.  One
+// solve at n 900, half-width 115 in FP64 took 131 us with every load issued, 68 us by class; at 3,465 and
+// 326, 562 and 449 us.  (A wave of its own for the recurrence, and the recurrence by DPP instead of
+// v_readlane, gained 5% and less: the band's loads hide it.)
 template <typename T>
 struct SolveCfg {
     static constexpr int NT = sizeof(T) == 8 ? 512 : 1024;
     static constexpr int W = NT / 64;
     static constexpr int NK = kRB / W;
-    static constexpr int FK = (kBandMax - kRB) / W;
-    static constexpr int BK = kBandMax / kRB - 1;
     static constexpr int DQ = kRB * kRB / NT;
     static constexpr int FC = 7;
     static constexpr int RC = sizeof(T) == 8 ? 8 : 16;
+    static constexpr int kClasses = (kBandMax - kRB) / (W * FC);
+    static constexpr int width(int nc) { return kRB + W * FC * nc; }  // widest band of class nc
 };
-static_assert(SolveCfg<float>::FK % SolveCfg<float>::FC == 0 && SolveCfg<double>::FK % SolveCfg<double>::FC == 0, "far chunks");
-static_assert(kRB + SolveCfg<float>::W * SolveCfg<float>::FK == kBandMax, "far cover");
+static_assert(SolveCfg<float>::width(SolveCfg<float>::kClasses) == kBandMax &&
+                  SolveCfg<double>::width(SolveCfg<double>::kClasses) == kBandMax, "far cover");
 
 // Zeros around the vector in LDS, so that the row and column indices of the band products need no
 // clamping: forward columns reach back to r0 + 64 - 514 >= -512, backward rows up to
@@ -150,11 +160,12 @@ __device__ __forceinline__ void band_run(T *dst, __amdgpu_buffer_rsrc_t rs, int 
     }
 }
 
-template <typename T>
-__device__ __forceinline__ void band_solve_lds(const T *__restrict__ fac, int n, int bw, double *__restrict__ xg, unsigned char *smem)
+template <typename T, int NC>
+__device__ __forceinline__ void band_solve_class(const T *__restrict__ fac, int n, int bw, double *__restrict__ xg, unsigned char *smem)
 {
     using C = SolveCfg<T>;
-    constexpr int NT = C::NT, W = C::W, NK = C::NK, FK = C::FK, BK = C::BK, DQ = C::DQ, FC = C::FC, RC = C::RC;
+    constexpr int NT = C::NT, W = C::W, NK = C::NK, DQ = C::DQ, FC = C::FC, RC = C::RC;
+    constexpr int FK = FC * NC, BK = (C::width(NC) - 1) / kRB;  // far row chunk k starts 64 k + 1 rows below a column at the least
     const unsigned ldu = (unsigned)bw + 1;  // n * ld * sizeof(T) < 2 GiB (checked by the launcher)
     const int ld = bw + 1;
     const __amdgpu_buffer_rsrc_t rs = band_rsrc(fac, (unsigned)((size_t)n * ldu * sizeof(T)));
@@ -343,6 +354,15 @@ __device__ __forceinline__ void band_solve_lds(const T *__restrict__ fac, int n,
     for (int i = tid; i < n; i += NT) xg[i] = xs[i];
 }
 
+template <typename T, int NC = 1>
+__device__ __forceinline__ void band_solve_lds(const T *fac, int n, int bw, double *x, unsigned char *smem)
+{
+    if constexpr (NC < SolveCfg<T>::kClasses) {
+        if (bw > SolveCfg<T>::width(NC)) return band_solve_lds<T, NC + 1>(fac, n, bw, x, smem);
+    }
+    band_solve_class<T, NC>(fac, n, bw, x, smem);
+}
+
 template <typename T>
 __global__ __launch_bounds__(SolveCfg<T>::NT) void k_band_solve_lds(const T *fac, int n, int bw, double *x)
 {
@@ -354,9 +374,9 @@ template <typename T>
 __global__ __launch_bounds__(SolveCfg<T>::NT) void k_band_solve_lds_batched(const BandDesc *descs)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    const BandDesc &d = descs[blockIdx.x];
+    const BandDesc d = descs[blockIdx.x];
     if (!d.active) return;
-    band_solve_lds<T>((const T *)d.fac, d.n, d.bw, d.x, smem);
+    band_solve_lds<T>(global_ptr((const T *)d.fac), d.n, d.bw, global_ptr(d.x), smem);
 }
 
 // ---- streaming kernel (vector in HBM; any n) ----
