@@ -239,7 +239,7 @@ int BatchDevice::products(std::vector<ProductJob> &jobs, std::vector<double> &rr
                        const_cast<double *>(jobs[i].x), jobs[i].r, (double *)m_norms.p + 2 * i, (double *)m_ppart.p + po, 0, 0};
         po += 2 * (((size_t)K.n + 63) / 64);
     }
-    if ((rc = refine_residual_batch(m_stream, (RefDesc *)m_rdesc.p, h))) return rc;
+    if ((rc = refine_residual_batch(m_stream, (RefDesc *)m_rdesc.p, h, m_prod))) return rc;
     std::vector<double> nr(2 * nj);
     KSH_HIP(hipMemcpyAsync(nr.data(), m_norms.p, sizeof(double) * nr.size(), hipMemcpyDeviceToHost, m_stream));
     KSH_HIP(hipStreamSynchronize(m_stream));
@@ -693,7 +693,7 @@ int BatchDevice::solve(std::vector<SolveJob> &jobs)
                            const_cast<double *>(x[i]), r[i], (double *)m_norms.p + 2 * i, (double *)m_part.p + poff[i], 0, 0};
         }
         int rc2;
-        if ((rc2 = refine_residual_batch(m_stream, (RefDesc *)m_rdesc.p, h))) return rc2;
+        if ((rc2 = refine_residual_batch(m_stream, (RefDesc *)m_rdesc.p, h, m_prod))) return rc2;
         KSH_HIP(hipMemcpyAsync(nr.data(), m_norms.p, sizeof(double) * nr.size(), hipMemcpyDeviceToHost, m_stream));
         KSH_HIP(hipStreamSynchronize(m_stream));
         return KSH_SUCCESS;

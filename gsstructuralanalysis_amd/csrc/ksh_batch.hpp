@@ -131,7 +131,7 @@ private:
     std::vector<std::unique_ptr<RecountBatch>> m_rcb;
     hipStream_t m_rc_stream = nullptr;
     hipEvent_t m_ev_rc_ready = nullptr;
-    DevScratch m_desc, m_bdesc, m_cdesc, m_rdesc, m_stats, m_info, m_norms, m_part, m_r, m_dotdesc, m_vecdesc, m_dotout;
+    DevScratch m_desc, m_bdesc, m_cdesc, m_rdesc, m_prod, m_stats, m_info, m_norms, m_part, m_r, m_dotdesc, m_vecdesc, m_dotout;
     DevScratch m_zero, m_ppart, m_pw, m_start;
     size_t m_start_n = 0;
     size_t m_zero_n = 0;

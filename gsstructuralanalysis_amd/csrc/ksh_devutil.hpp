@@ -39,6 +39,46 @@ __device__ __forceinline__ float readlane_f32(float v, int src)
 __device__ __forceinline__ double bcast(double v, int src) { return readlane_f64(v, src); }
 __device__ __forceinline__ float bcast(float v, int src) { return readlane_f32(v, src); }
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+constexpr int kRor8 = 0x128, kHalfMirror = 0x141, kQuadSwap = 0xB1, kQuadCross = 0x4E;
+
+// (a, b) -> a of the lower 32 lanes beside b's lower, plus the same of the upper: lanes < 32 get
+// a[l] + a[l + 32], lanes >= 32 get b[l - 32] + b[l]; likewise for the 16-lane rows
+__device__ __forceinline__ double swap_add32(double a, double b)
+{
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double swap_add16(double a, double b)
+{
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+// sums over the 64 lanes of sixteen values: lane l gets the total of value l / 4
+__device__ __forceinline__ double sum_lanes(const double (&a)[16], int lane)
+{
+    double v[8], w[4], y[2];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = swap_add32(a[q], a[q + 8]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[q] = swap_add16(v[q], v[q + 4]);
+    const bool up8 = (lane & 8) != 0, up4 = (lane & 4) != 0;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) y[q] = (up8 ? w[q + 2] : w[q]) + dpp_move<kRor8>(up8 ? w[q] : w[q + 2]);
+    double s = (up4 ? y[1] : y[0]) + dpp_move<kHalfMirror>(up4 ? y[0] : y[1]);
+    s += dpp_move<kQuadSwap>(s);
+    s += dpp_move<kQuadCross>(s);
+    return s;
+}
+
 // workgroup barrier that orders LDS only: global loads in flight (register prefetches private to
 // their thread) are not waited for
 __device__ __forceinline__ void lds_barrier()

@@ -212,8 +212,10 @@ struct RefDesc {
     // a second vector on the same matrix (set by the launcher when two jobs share ab; else null)
     const double *b2;
     double *x2, *r2, *norms2, *part2;
+    double *prod, *prod2;  // products by column blocks (set by the launcher)
 };
-int refine_residual_batch(hipStream_t s, RefDesc *d_descs, const std::vector<RefDesc> &h);
+struct DevScratch;
+int refine_residual_batch(hipStream_t s, RefDesc *d_descs, const std::vector<RefDesc> &h, DevScratch &prod);
 int refine_update_batch(hipStream_t s, RefDesc *d_descs, const std::vector<RefDesc> &h);
 // FP64 refactorization of K's assembled values into fac64 (K.use64 = true afterwards)
 int refactor_fp64(Matrix &K);

@@ -1,21 +1,25 @@
 // ksh_spmv.hip -- symmetric band mat-vec y = K x and batched refinement residuals r = b - K x.
 //
-// K is stored as its lower band, column major: ab[j*ld + (i-j)], ld = bw+1.  A workgroup of 256
-// threads owns a block of 64 consecutive rows of one matrix (a launch covers all row blocks of all
-// matrices of a batch):
+// K is stored as its lower band, column major: ab[j*ld + (i-j)], ld = bw+1.  The single mat-vec goes by
+// rows: a workgroup of 256 threads owns a block of 64 consecutive rows:
 //   lower part  sum_{j<=i} K[i][j] x[j]: lanes = the block's rows, so each band column contributes
 //               one contiguous 64-entry run (coalesced); the four waves take every fourth column and
 //               issue 8 independent loads per lane before accumulating;
 //   upper part  sum_{j>i} K[j][i] x[j] = sum_d ab[i*ld + d] x[i+d]: one wave per 16 rows, lanes along
 //               the contiguous column of row i, wave reductions.
-// Every band entry is read twice (once for each triangle); the mat-vec is HBM bound at
-// 2 n (bw+1) sizeof(T) bytes.  Refinement residual norms are reduced per block, then per matrix in
-// block order (deterministic).
+// Every band entry is read twice (once for each triangle), one launch, no scratch.  The batched
+// residuals go by columns (below), each entry read once; their norms are reduced per block, then
+// per matrix in block order (deterministic).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <utility>
+#include <vector>
 
 #include "ksh_devutil.hpp"
 #include "ksh_internal.hpp"
 #include "ksh_profile.hpp"
+#include "ksh_vec.hpp"
 
 namespace ksh {
 
@@ -126,57 +130,147 @@ __device__ inline RefDesc find_block(const RefDesc *d, int n, int blk)
     r.x2 = global_ptr(r.x2);
     r.r2 = global_ptr(r.r2);
     r.part2 = global_ptr(r.part2);
+    r.prod = global_ptr(r.prod);
+    r.prod2 = global_ptr(r.prod2);
     return r;
 }
 
-// r = b - K x on one row block of one matrix (and r2 = b2 - K x2 with the same band loads when the
-// descriptor carries a second vector); block partial norms (||r||^2, ||b||^2) -> part (part2)
-template <int NR>
-__device__ __forceinline__ void refine_rows(const RefDesc &d, int lb)
+// ---- K x by column blocks, for the refinement residuals ----
+// A workgroup takes 64 columns of one matrix, wave w columns 16 w .. 16 w + 15, and walks down their band
+// by chunks of 64 rows (lane = row: every load is a contiguous run of one column).  An entry K[i][j] is
+// read once for both of its products: K[i][j] x_j goes to the chunk's partial sum of rows i, summed over
+// the block's columns and stored (prod: per column block its chunks' 64 sums), and K[i][j] x_i to
+// column j's own sum, complete at the end of the walk (prod's first n entries).  k_refine_sum then adds a
+// row's at most bw / 64 + 2 partial sums, in the order of the column blocks.  The band is read once
+// instead of twice and the partial sums are 1 / 32 of it: HBM bound.  256 bands of half-width 182..470 in
+// FP64 (3.1 GB), two vectors each: 1.61 ms by rows (every entry read for its row and again for its
+// column), 0.72 ms by columns (4.4 TB/s) and 0.04 ms for the sums.
+constexpr int kCols = kRows / 4;
+
+// chunks of 64 rows that a block of 64 columns of half-width bw reaches
+__host__ __device__ inline int col_chunks(int bw) { return (bw + 2 * kRows - 1) / kRows; }
+__host__ __device__ inline size_t prod_doubles(int n, int bw)
 {
-    const int i0 = lb * kRows;
-    const double *xs[NR];
-    xs[0] = d.x;
-    if constexpr (NR > 1) xs[1] = d.x2;
-    double kx[NR];
-    if (d.sprec == KSH_FP64)
-        symv_row_block<double, NR>((const double *)d.ab, d.n, d.bw, xs, i0, kx);
-    else
-        symv_row_block<float, NR>((const float *)d.ab, d.n, d.bw, xs, i0, kx);
-    if (threadIdx.x < 64) {
-        const int i = i0 + threadIdx.x;
+    const size_t nblk = ((size_t)n + kRows - 1) / kRows;
+    return nblk * kRows * (1 + (size_t)col_chunks(bw));
+}
+
+template <typename T, int NR>
+__device__ __forceinline__ void column_block(const RefDesc &d, int lb)
+{
+    __shared__ double red[2][NR][4][kRows];
+    const int n = d.n, bw = d.bw, j0 = lb * kRows, lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), jw = j0 + kCols * wv;
+    const size_t ld = (size_t)bw + 1;
+    const T *ab = (const T *)d.ab;
+    const double *x[NR];
+    double *prod[NR];
+    x[0] = d.x;
+    prod[0] = d.prod;
+    if constexpr (NR > 1) {
+        x[1] = d.x2;
+        prod[1] = d.prod2;
+    }
+    double xj[NR][kCols], up[NR][kCols];
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+#pragma unroll
+        for (int u = 0; u < kCols; ++u) {
+            xj[q][u] = jw + u < n ? x[q][jw + u] : 0.0;
+            up[q][u] = 0.0;
+        }
+    const int nch = (min(n - j0, kRows + bw) + kRows - 1) / kRows;
+    for (int c = 0; c < nch; ++c) {
+        const int i = j0 + kRows * c + lane;
+        double v[kCols], xi[NR], low[NR];
+#pragma unroll
+        for (int u = 0; u < kCols; ++u) {
+            const int j = jw + u, o = i - j;
+            const bool in = o >= 0 && o <= bw && i < n;
+            const T e = ab[in ? (size_t)j * ld + (unsigned)o : 0];
+            v[u] = in ? (double)e : 0.0;
+        }
 #pragma unroll
         for (int q = 0; q < NR; ++q) {
-            const double *b = q == 0 ? d.b : d.b2;
-            double *r = q == 0 ? d.r : d.r2, *part = q == 0 ? d.part : d.part2;
-            double ri = 0.0, bi = 0.0;
-            if (i < d.n) {
-                bi = b[i];
-                ri = bi - kx[q];
-                r[i] = ri;
-            }
-            double rr = ri * ri, bb = bi * bi;
-            for (int off = 32; off > 0; off >>= 1) {
-                rr += __shfl_xor(rr, off);
-                bb += __shfl_xor(bb, off);
-            }
-            if (threadIdx.x == 0) {
-                part[2 * lb] = rr;
-                part[2 * lb + 1] = bb;
-            }
+            xi[q] = i < n ? x[q][i] : 0.0;
+            low[q] = 0.0;
         }
+#pragma unroll
+        for (int u = 0; u < kCols; ++u)
+#pragma unroll
+            for (int q = 0; q < NR; ++q) {
+                low[q] += v[u] * xj[q][u];
+                up[q][u] += (i == jw + u ? 0.0 : v[u]) * xi[q];
+            }
+#pragma unroll
+        for (int q = 0; q < NR; ++q) red[c & 1][q][wv][lane] = low[q];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NR; ++q)
+            if (wv == ((c + q) & 3))
+                prod[q][((size_t)d.nblk + (size_t)lb * col_chunks(bw) + c) * kRows + lane] =
+                    (red[c & 1][q][0][lane] + red[c & 1][q][1][lane]) + (red[c & 1][q][2][lane] + red[c & 1][q][3][lane]);
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+        const double t = sum_lanes(up[q], lane);
+        if ((lane & 3) == 0) prod[q][jw + (lane >> 2)] = t;
     }
 }
 
-__global__ __launch_bounds__(kT) void k_refine_rows_batched(const RefDesc *__restrict__ descs, int ninst)
+__global__ __launch_bounds__(kT) void k_refine_cols(const RefDesc *__restrict__ descs, int ninst)
 {
     const RefDesc d = find_block(descs, ninst, blockIdx.x);
     if (!d.active) return;
     const int lb = blockIdx.x - d.blk0;
-    if (d.x2)
-        refine_rows<2>(d, lb);
-    else
-        refine_rows<1>(d, lb);
+    if (d.sprec == KSH_FP64) {
+        if (d.x2) column_block<double, 2>(d, lb);
+        else column_block<double, 1>(d, lb);
+    } else {
+        if (d.x2) column_block<float, 2>(d, lb);
+        else column_block<float, 1>(d, lb);
+    }
+}
+
+// r = b - K x on one block of 64 rows, K x from the column blocks' sums, and the block's partial norms
+// (||r||^2, ||b||^2); workgroup y: the first or the second vector of the descriptor
+__global__ __launch_bounds__(64) void k_refine_sum(const RefDesc *__restrict__ descs, int ninst)
+{
+    const RefDesc d = find_block(descs, ninst, blockIdx.x);
+    const bool second = blockIdx.y != 0;
+    if (!d.active || (second && !d.x2)) return;
+    const double *prod = second ? d.prod2 : d.prod, *b = second ? d.b2 : d.b;
+    double *r = second ? d.r2 : d.r, *part = second ? d.part2 : d.part;
+    const int lb = blockIdx.x - d.blk0, lane = (int)threadIdx.x, i = lb * kRows + lane;
+    const int nch = col_chunks(d.bw), first = max(0, lb - nch + 1);
+    const double own = prod[i];
+    double y = 0.0;
+    for (int J0 = first; J0 <= lb; J0 += kU) {
+        double v[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const int J = min(J0 + u, lb);
+            v[u] = prod[((size_t)d.nblk + (size_t)J * nch + (lb - J)) * kRows + lane];
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+            if (J0 + u <= lb) y += v[u];
+    }
+    double ri = 0.0, bi = 0.0;
+    if (i < d.n) {
+        bi = b[i];
+        ri = bi - (y + own);
+        r[i] = ri;
+    }
+    double rr = ri * ri, bb = bi * bi;
+    for (int off = 32; off > 0; off >>= 1) {
+        rr += __shfl_xor(rr, off);
+        bb += __shfl_xor(bb, off);
+    }
+    if (lane == 0) {
+        part[2 * lb] = rr;
+        part[2 * lb + 1] = bb;
+    }
 }
 
 // per-matrix norms from the block partials (block order), one workgroup per matrix
@@ -247,7 +341,11 @@ int band_symv(const Matrix &K, const double *x_dev, double *y_dev)
     return KSH_SUCCESS;
 }
 
-int refine_residual_batch(hipStream_t s, RefDesc *d_descs, const std::vector<RefDesc> &hin)
+// most of the products' scratch that one launch uses; larger batches go by several launches, one after
+// the other on the stream, over the same scratch
+constexpr size_t kProdBytes = 512ull << 20;
+
+int refine_residual_batch(hipStream_t s, RefDesc *d_descs, const std::vector<RefDesc> &hin, DevScratch &prod)
 {
     if (hin.empty()) return KSH_SUCCESS;
     // two active jobs on the same matrix (the arc-length solves' two right-hand sides) share one
@@ -274,15 +372,50 @@ int refine_residual_batch(hipStream_t s, RefDesc *d_descs, const std::vector<Ref
             }
         h.push_back(d);
     }
-    int tot = prefix_blocks(h);
+    // groups of descriptors [g0, g1) with their own offsets into the scratch and launch blocks
+    std::vector<std::pair<size_t, size_t>> groups;
+    std::vector<size_t> off(h.size());
+    size_t most = 0;
+    for (size_t g0 = 0; g0 < h.size();) {
+        size_t used = 0, g1 = g0;
+        for (; g1 < h.size(); ++g1) {
+            const size_t w = h[g1].active ? prod_doubles(h[g1].n, h[g1].bw) * (h[g1].x2 ? 2 : 1) * sizeof(double) : 0;
+            if (g1 > g0 && used + w > kProdBytes) break;
+            off[g1] = used;
+            used += w;
+        }
+        most = std::max(most, used);
+        groups.push_back({g0, g1});
+        g0 = g1;
+    }
+    int rc;
+    if ((rc = prod.ensure(most))) return rc;
+    std::vector<int> tot;
+    for (const auto &g : groups) {
+        int t = 0;
+        for (size_t i = g.first; i < g.second; ++i) {
+            RefDesc &d = h[i];
+            d.blk0 = t;
+            d.nblk = (int)nblocks(d.n);
+            t += d.nblk;
+            d.prod = (double *)((char *)prod.p + off[i]);
+            d.prod2 = d.x2 ? d.prod + prod_doubles(d.n, d.bw) : nullptr;
+        }
+        tot.push_back(t);
+    }
     KSH_HIP(hipMemcpyAsync(d_descs, h.data(), sizeof(RefDesc) * h.size(), hipMemcpyHostToDevice, s));
     {
         ProfScope ps("refine_residual_batch", s);
-        double work = 0.0;  // K read as a full band (2b+1 per row), x and b read, r written (per vector)
+        double work = 0.0;  // the band read once, x and b read, r written (per vector)
         for (const auto &d : h)
-            if (d.active) work += d.n * (2.0 * d.bw + 1.0) * (d.sprec == KSH_FP64 ? 8.0 : 4.0) + (d.x2 ? 48.0 : 24.0) * d.n;
+            if (d.active) work += d.n * (d.bw + 1.0) * (d.sprec == KSH_FP64 ? 8.0 : 4.0) + (d.x2 ? 48.0 : 24.0) * d.n;
         ps.set_work(work);
-        hipLaunchKernelGGL(k_refine_rows_batched, dim3((unsigned)tot), dim3(kT), 0, s, (const RefDesc *)d_descs, (int)h.size());
+        for (size_t g = 0; g < groups.size(); ++g) {
+            const RefDesc *dd = (const RefDesc *)d_descs + groups[g].first;
+            const int cnt = (int)(groups[g].second - groups[g].first);
+            hipLaunchKernelGGL(k_refine_cols, dim3((unsigned)tot[g]), dim3(kT), 0, s, dd, cnt);
+            hipLaunchKernelGGL(k_refine_sum, dim3((unsigned)tot[g], 2), dim3(64), 0, s, dd, cnt);
+        }
     }
     KSH_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_refine_norms_batched, dim3((unsigned)h.size()), dim3(64), 0, s, (const RefDesc *)d_descs);
