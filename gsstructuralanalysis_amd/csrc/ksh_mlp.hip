@@ -8,12 +8,12 @@
 //
 // One GEMM kernel serves the forward layer (Y = act(X W + b)), the input gradient
 // (dX = dY W^T) and the weight gradient (dW = X^T dY): operands are addressed through strides,
-// so a transposed operand is just other strides.  Workgroup tile 64 x 64 (four waves of 32 x 32
-// = 2 x 2 MFMA tiles), K in steps of 16 staged in LDS as BF16.
+// so a transposed operand is just other strides.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstring>
 #include <random>
 #include <vector>
@@ -34,77 +34,125 @@ __device__ __forceinline__ unsigned short bf16_rne(float x)
     return (unsigned short)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
 
-constexpr int kTM = 64, kTN = 64, kTK = 16;
-
 // C(m, n) = act(sum_k A(m, k) B(k, n) + bias[n]), A(m, k) = A[m sam + k sak], B(k, n) = B[k sbk + n sbn]
-// act: 0 identity, 1 GELU (the pre-activation goes to Z when Z != null)
-__global__ __launch_bounds__(256) void k_gemm_bf16(int M, int N, int K, const float *__restrict__ A, int sam, int sak,
-                                                   const float *__restrict__ B, int sbk, int sbn,
-                                                   const float *__restrict__ bias, int act, float *__restrict__ C, int ldc,
-                                                   float *__restrict__ Z)
+// act: 0 identity, 1 GELU (the pre-activation goes to Z when Z != null), 2 times GELU'(Z),
+// GELU'(z) = Phi(z) + z phi(z)
+//
+// The products are small (256 x 256 x 264 at a minibatch of 256: 0.4 MB, 35 MFLOP) and bound by memory
+// latency, so what counts is how many loads are in flight and how few rounds there are.  A workgroup of
+// eight waves takes a 32 x 32 tile of C (72 workgroups at that size) and splits K over the waves by steps of
+// 16; each wave loads the operands of kAhead steps straight into MFMA fragments (no LDS, no barrier), so
+// that up to K = 384 is one round trip, and the eight partial tiles meet in LDS in the order of the waves (the
+// sum depends on K alone, not on the batch).  64 x 64 tiles by 20 workgroups with K in barriered steps of 16
+// took 28.6 us a product on average, 6.5 us like this.
+// entries k .. k + 3 of a row at p with stride sk, zeros from K on or if !ok
+template <bool kVec>
+__device__ __forceinline__ void load_four(float (&v)[4], const float *p, int sk, int k, int K, bool ok)
 {
-    __shared__ unsigned short sA[kTM][kTK + 4];  // [m][k]
-    __shared__ unsigned short sB[kTN][kTK + 4];  // [n][k]
-    const int m0 = blockIdx.y * kTM, n0 = blockIdx.x * kTN;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    if constexpr (kVec) {
+        const float4 x = *reinterpret_cast<const float4 *>(p + min(k, K - 4));
+        const bool in = ok && k < K;
+        v[0] = in ? x.x : 0.f;
+        v[1] = in ? x.y : 0.f;
+        v[2] = in ? x.z : 0.f;
+        v[3] = in ? x.w : 0.f;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float x = p[(size_t)min(k + j, K - 1) * sk];
+            v[j] = ok && k + j < K ? x : 0.f;
+        }
+    }
+}
+
+constexpr int kGT = 32, kGW = 8, kAhead = 3, kPitch = kGT + 4;
+
+// VA / VB: A's rows / B's columns are contiguous in k, 16-byte aligned and K is a multiple of 4, so that a
+// lane's four entries are one load: as four loads of 64 scattered words each they are what bounds the
+// product (9.3 us).
+template <bool VA, bool VB>
+__global__ __launch_bounds__(64 * kGW) void k_gemm_bf16(int M, int N, int K, const float *__restrict__ A, int sam, int sak,
+                                                        const float *__restrict__ B, int sbk, int sbn,
+                                                        const float *__restrict__ bias, int act, float *__restrict__ C, int ldc,
+                                                        float *__restrict__ Z)
+{
+    __shared__ float red[kGW][kGT * kPitch];
+    const int m0 = blockIdx.x * kGT, n0 = blockIdx.y * kGT;
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kq = 4 * (lane >> 4);
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int steps = (K + 15) / 16;
+    // lane supplies A[row = lane % 16][k = 4 (lane / 16) .. +3] and B[k = same][col = lane % 16]
+    const float *pa[2], *pb[2];
+    bool oka[2], okb[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        const int m = m0 + 16 * a + li, n = n0 + 16 * a + li;
+        oka[a] = m < M;
+        okb[a] = n < N;
+        pa[a] = A + (size_t)min(m, M - 1) * sam;
+        pb[a] = B + (size_t)min(n, N - 1) * sbn;
+    }
     v4f acc[2][2];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < K; k0 += kTK) {
-        // stage 64 x 16 of A and 16 x 64 of B (4 entries per thread each), rounded to BF16
+    for (int c0 = wv; c0 < steps; c0 += kGW * kAhead) {
+        float va[kAhead][2][4], vb[kAhead][2][4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int idx = tid + 256 * q, r = idx >> 4, k = idx & 15;
-            const int m = m0 + r, n = n0 + r, kk = k0 + k;
-            sA[r][k] = bf16_rne((m < M && kk < K) ? A[(size_t)m * sam + (size_t)kk * sak] : 0.f);
-            sB[r][k] = bf16_rne((n < N && kk < K) ? B[(size_t)kk * sbk + (size_t)n * sbn] : 0.f);
+        for (int t = 0; t < kAhead; ++t) {
+            const int k = 16 * (c0 + kGW * t) + kq;
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                load_four<VA>(va[t][a], pa[a], sak, k, K, oka[a]);
+                load_four<VB>(vb[t][a], pb[a], sbk, k, K, okb[a]);
+            }
         }
-        __syncthreads();
-        // lane supplies A[row = lane % 16][k = 4 (lane / 16) .. +3] and B[k = same][col = lane % 16]
-        const int r = lane & 15, kq = 4 * (lane >> 4);
-        v4s fa[2], fb[2];
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+        for (int t = 0; t < kAhead; ++t) {
+            if (c0 + kGW * t >= steps) break;
+            v4s fa[2], fb[2];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) fa[a][j] = (short)sA[wm + 16 * a + r][kq + j];
+            for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+                for (int j = 0; j < 4; ++j) {
+                    fa[a][j] = (short)bf16_rne(va[t][a][j]);
+                    fb[a][j] = (short)bf16_rne(vb[t][a][j]);
+                }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) fb[b][j] = (short)sB[wn + 16 * b + r][kq + j];
+            for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa[a], fb[b], acc[a][b], 0, 0, 0);
-        __syncthreads();
+                for (int b = 0; b < 2; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa[a], fb[b], acc[a][b], 0, 0, 0);
+        }
     }
-    // result: lane holds D[4 (lane / 16) + v][lane % 16]
+    // lane holds D[4 (lane / 16) + v][lane % 16]
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int m = m0 + wm + 16 * a + 4 * (lane >> 4) + v, n = n0 + wn + 16 * b + (lane & 15);
-                if (m >= M || n >= N) continue;
-                float z = acc[a][b][v] + (bias ? bias[n] : 0.f);
-                if (Z) Z[(size_t)m * ldc + n] = z;
-                if (act == 1) z = 0.5f * z * (1.f + erff(z * 0.70710678118654752f));
-                C[(size_t)m * ldc + n] = z;
-            }
-}
-
-// dZ = dH * GELU'(Z), GELU'(z) = Phi(z) + z phi(z)
-__global__ void k_gelu_back(int count, const float *Z, const float *dH, float *dZ)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    const float z = Z[i];
-    const float cdf = 0.5f * (1.f + erff(z * 0.70710678118654752f));
-    const float pdf = 0.39894228040143268f * expf(-0.5f * z * z);
-    dZ[i] = dH[i] * (cdf + z * pdf);
+            for (int v = 0; v < 4; ++v) red[wv][(16 * a + kq + v) * kPitch + 16 * b + li] = acc[a][b][v];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kGT * kGT / (64 * kGW); ++q) {
+        const int idx = tid + 64 * kGW * q, r = idx / kGT, c = idx % kGT, m = m0 + r, n = n0 + c;
+        if (m >= M || n >= N) continue;
+        float z = 0.f;
+#pragma unroll
+        for (int w = 0; w < kGW; ++w) z += red[w][r * kPitch + c];
+        if (bias) z += bias[n];
+        if (act == 2) {
+            const float u = Z[(size_t)m * ldc + n];
+            const float cdf = 0.5f * (1.f + erff(u * 0.70710678118654752f));
+            const float pdf = 0.39894228040143268f * expf(-0.5f * u * u);
+            z *= cdf + u * pdf;
+        } else if (Z) {
+            Z[(size_t)m * ldc + n] = z;
+        }
+        if (act == 1) z = 0.5f * z * (1.f + erff(z * 0.70710678118654752f));
+        C[(size_t)m * ldc + n] = z;
+    }
 }
 
 // dY = 2 (Y - T) / (rows cols); loss partial sums per block into part[]
@@ -126,20 +174,28 @@ __global__ __launch_bounds__(256) void k_mse(int count, float scale, const float
     if (threadIdx.x == 0) part[blockIdx.x] = s[0] * scale;
 }
 
-// db[n] = sum_m dZ[m][n]: a workgroup of 4 waves per 64 columns, lanes along the columns (coalesced
-// rows), wave w summing rows w, w + 4, ... in order, then the four partial sums in wave order
-// (a fixed order, so the result is reproducible)
-__global__ __launch_bounds__(256) void k_colsum(int M, int N, const float *dZ, float *db)
+// db[n] = sum_m dZ[m][n]: a workgroup of kSumW waves per 64 columns, lanes along the columns (coalesced
+// rows), wave w summing rows w, w + kSumW, ... in order, then the partial sums in wave order (a fixed
+// order, so the result is reproducible).  Latency bound: 16 waves instead of 4, 8.0 us -> 2.4 us at 256 rows
+constexpr int kSumW = 16;
+__global__ __launch_bounds__(64 * kSumW) void k_colsum(int M, int N, const float *__restrict__ dZ, float *__restrict__ db)
 {
-    __shared__ float part[4][64];
+    __shared__ float part[kSumW][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = blockIdx.x * 64 + lane;
     float s = 0.f;
-    if (n < N)
-        for (int m = wave; m < M; m += 4) s += dZ[(size_t)m * N + n];
+    if (n < N) {
+#pragma unroll 8
+        for (int m = wave; m < M; m += kSumW) s += dZ[(size_t)m * N + n];
+    }
     part[wave][lane] = s;
     __syncthreads();
-    if (wave == 0 && n < N) db[n] = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
+    if (wave == 0 && n < N) {
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < kSumW; ++w) t += part[w][lane];
+        db[n] = t;
+    }
 }
 
 __global__ void k_adam(int count, float *w, const float *g, float *mo, float *ve, float lr, float b1, float b2, float eps,
@@ -176,8 +232,8 @@ struct Mlp {
     float *param = nullptr, *grad = nullptr, *m1 = nullptr, *m2 = nullptr;  // all weights then biases
     size_t nparam = 0;
     size_t woff[kLayers], boff[kLayers];
-    // activations: H[0] = input, H[l] layer outputs; Z[l] pre-activations; dH / dZ gradients
-    float *H[kLayers + 1] = {}, *Zp[kLayers] = {}, *dH[kLayers + 1] = {}, *dZ[kLayers] = {};
+    // activations: H[0] = input, H[l] layer outputs; Z[l] pre-activations; dZ their gradients
+    float *H[kLayers + 1] = {}, *Zp[kLayers] = {}, *dZ[kLayers] = {};
     float *target = nullptr, *loss_part = nullptr;
     int *idx = nullptr;
     float *data_x = nullptr, *data_y = nullptr;
@@ -196,9 +252,7 @@ struct Mlp {
         if (B <= batch_cap) return KSH_SUCCESS;
         for (int l = 0; l <= kLayers; ++l) {
             (void)hipFree(H[l]);
-            (void)hipFree(dH[l]);
             KSH_HIP(hipMalloc(&H[l], sizeof(float) * (size_t)B * width[l]));
-            KSH_HIP(hipMalloc(&dH[l], sizeof(float) * (size_t)B * width[l]));
         }
         for (int l = 0; l < kLayers; ++l) {
             (void)hipFree(Zp[l]);
@@ -217,8 +271,13 @@ struct Mlp {
     int gemm(int M, int N, int K, const float *A, int sam, int sak, const float *Bm, int sbk, int sbn, const float *bias,
              int act, float *C, int ldc, float *Z)
     {
-        dim3 g(nb(N, kTN), nb(M, kTM));
-        hipLaunchKernelGGL(k_gemm_bf16, g, dim3(256), 0, s, M, N, K, A, sam, sak, Bm, sbk, sbn, bias, act, C, ldc, Z);
+        dim3 g(nb(M, kGT), nb(N, kGT));
+        const auto vec = [&](const float *p, int sk, int srow) {
+            return sk == 1 && srow % 4 == 0 && K % 4 == 0 && ((uintptr_t)p & 15) == 0;
+        };
+        const bool va = vec(A, sak, sam), vb = vec(Bm, sbk, sbn);
+        auto *kern = va ? (vb ? k_gemm_bf16<true, true> : k_gemm_bf16<true, false>) : (vb ? k_gemm_bf16<false, true> : k_gemm_bf16<false, false>);
+        hipLaunchKernelGGL(kern, g, dim3(64 * kGW), 0, s, M, N, K, A, sam, sak, Bm, sbk, sbn, bias, act, C, ldc, Z);
         KSH_HIP(hipGetLastError());
         return KSH_SUCCESS;
     }
@@ -251,14 +310,11 @@ struct Mlp {
             const int K = width[l], N = width[l + 1];
             // dW = H[l]^T dZ[l]   (K x N, reduction over the batch)
             if ((rc = gemm(K, N, B, H[l], 1, K, dZ[l], N, 1, nullptr, 0, gW(l), N, nullptr))) return rc;
-            hipLaunchKernelGGL(k_colsum, dim3(nb(N, 64)), dim3(256), 0, s, B, N, dZ[l], gb(l));
+            hipLaunchKernelGGL(k_colsum, dim3(nb(N, 64)), dim3(64 * kSumW), 0, s, B, N, dZ[l], gb(l));
             KSH_HIP(hipGetLastError());
             if (l > 0) {
-                // dH[l] = dZ[l] W^T, then through GELU of layer l-1
-                if ((rc = gemm(B, K, N, dZ[l], N, 1, W(l), 1, N, nullptr, 0, dH[l], K, nullptr))) return rc;
-                hipLaunchKernelGGL(k_gelu_back, dim3(nb((size_t)B * K, 256)), dim3(256), 0, s, B * K, Zp[l - 1], dH[l],
-                                   dZ[l - 1]);
-                KSH_HIP(hipGetLastError());
+                // dZ[l-1] = (dZ[l] W^T) GELU'(Z of layer l-1)
+                if ((rc = gemm(B, K, N, dZ[l], N, 1, W(l), 1, N, nullptr, 2, dZ[l - 1], K, Zp[l - 1]))) return rc;
             }
         }
         if (loss) {
@@ -342,7 +398,6 @@ int ksh_mlp_destroy(ksh_mlp *m)
     for (float *p : {m->param, m->grad, m->m1, m->m2, m->target, m->loss_part, m->data_x, m->data_y}) (void)hipFree(p);
     for (int l = 0; l <= Mlp::kLayers; ++l) {
         (void)hipFree(m->H[l]);
-        (void)hipFree(m->dH[l]);
     }
     for (int l = 0; l < Mlp::kLayers; ++l) {
         (void)hipFree(m->Zp[l]);
