@@ -50,9 +50,9 @@ constexpr int kBandMax = 512;    // widest band of the LDS-resident kernel
 // rows) and BK far row chunks each.  FC: far registers consumed and refilled per scheduling
 // group; RC: diagonal-block entries per recurrence register run.
 //
-// What bounds it is the rate at which one CU takes a band from memory, about 20 bytes a cycle (4.0 us a
-// block and sweep at half-width 326 in FP64, 5.0 us at 470), or HBM where every CU has a band; below
-// that, the instructions of a block.  So the body is compiled for NC = 1 .. kClasses groups of far
+// What bounds it is the rate at which one workgroup takes a band from memory, about 20 bytes a cycle
+// in either precision (4.0 us a block and sweep at half-width 326 in FP64, 5.0 us at 470), or HBM where
+// every CU has a band; at small widths, the instructions of a block.  So the body is compiled for NC = 1 .. kClasses groups of far
 // columns (and the far row chunks that the widest such band has), and a workgroup takes the
 // narrowest that covers its band: loads beyond the band read nothing, but cost their issue slots.
 // The entries left out are zeros of every sum, so the class does not show in the result.  One
