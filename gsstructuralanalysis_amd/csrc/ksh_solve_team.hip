@@ -38,6 +38,7 @@
 #include "ksh_internal.hpp"
 #include "ksh_mfma.hpp"
 #include "ksh_profile.hpp"
+#include "ksh_team_order.hpp"
 
 namespace ksh {
 
@@ -309,7 +310,7 @@ __device__ __forceinline__ void load_cols(const Band<T> &B, int ib, int jb, bool
 struct TeamLds {
     double far[kTW][kB];   // partial sums of the helper's exchanges
     double part[kTW][kB];
-    double lead[2][kTW][kB];  // of the leader's (by parity: one barrier a step)
+    double lead[kLeadBuffers][kTW][kB];  // of the leader's, by lead_buffer (one barrier a step, in and between the sweeps)
     double vec[kTW][kU];
     unsigned team, rank;
 };
@@ -477,11 +478,10 @@ __device__ __forceinline__ void lead(const Band<T> &B, const TeamMem &d, TeamLds
         load_mat(d, k, kFwd ? kMq : kMp, wv, lane, q.w);
     };
     double v = 0.0;  // solution of the block before, entry 16 wv + lane % 16
-    int par = 0;
     auto step = [&](Regs &q, int s) {
-        const int k = block(s);
+        const int k = block(s), buf = lead_buffer(lead_step(kFwd, B.nblk, s));
         const double c = q.c;
-        sh.lead[par][wv][lane] = dot_bcast(0.0, v, q.w);
+        sh.lead[buf][wv][lane] = dot_bcast(0.0, v, q.w);
         if constexpr (kAlone) {
             if (kFwd)
                 help_forward<T>(B, d, sh, k, 1, k + 1, gone);
@@ -489,8 +489,7 @@ __device__ __forceinline__ void lead(const Band<T> &B, const TeamMem &d, TeamLds
                 help_backward<T>(B, d, sh, k, 1, k, gone);
         }
         lds_barrier();
-        const double sum = sum_groups(sh.lead[par][lane >> 4][jl]);
-        par ^= 1;
+        const double sum = sum_groups(sh.lead[buf][lane >> 4][jl]);
         v = slot_wait(cs + kB * k + jl, c, gone) - sum;
         if (lane < kU) {
             slot_store(vs + kB * k + jl, v);
