@@ -24,7 +24,9 @@
 // Progress.  Nothing waits for a workgroup that is not running: workgroups register as they start, the
 // leader (the first) waits a bounded time for S of them and closes the team with those it has, and
 // later ones leave at once.  A leader without helpers forms the c_k itself.  Every poll is bounded
-// all the same; past the bound a workgroup stops waiting and its NaNs reach the result.
+// all the same.  Past the bound a workgroup goes on with NaN, which reaches every later block of the chain:
+// a leader that ends with NaN does the whole solve again without helpers, over slots of its own: later,
+// and with the same bits (or with the NaN that the right-hand side or the factor holds).
 //
 // Replaces SimplicialLDLT::solve (src/gsALMSolvers/gsALMBase.hpp:200-211,
 // src/gsStaticSolvers/gsStaticNewton.hpp:215-240, src/gsEigenSolvers/gsEigenProblemBase.hpp:152-216).
@@ -52,7 +54,7 @@ constexpr int kU = kB / kTW;         // columns of a block per wave
 constexpr int kAhead = 4;            // blocks a helper loads ahead
 constexpr int kLead = 3;             // blocks the leader loads ahead
 constexpr unsigned long long kSentinel = 0x7FF7A5A5A5A5A5A5ull;
-constexpr unsigned kPollLimit = 1u << 16;  // polls of one slot (tens of ms), then the workgroup stops waiting
+constexpr unsigned kPollLimit = 1u << 16;  // polls of one slot (tens of ms), then its reader stops waiting
 constexpr unsigned kFormLimit = 64;        // polls of the team's forming (tens of us)
 
 struct TeamDesc {
@@ -60,7 +62,9 @@ struct TeamDesc {
     double *x;                   // right-hand side in, solution out
     int n, bw;
     unsigned *ctl;               // [0] registered workgroups, [1] team size once closed
-    double *y, *xo, *cf, *cb;    // forward solution, solution, forward and backward c_k (slots, padded to 64)
+    // vectors padded to 64: the right-hand side; then the team's slots of the forward solution, the solution,
+    // the forward and the backward c_k; then the same four of a leader without helpers
+    double *b;
     double *mat;                 // per block four 64 x 64: M_k, M_k^T, Q_k, P_k (see mat_at)
 };
 constexpr int kM = 0, kMt = 1, kMq = 2, kMp = 3;
@@ -76,11 +80,18 @@ typedef __attribute__((address_space(1))) const unsigned long long cgu64;
 typedef __attribute__((address_space(1))) unsigned gu32;
 typedef __attribute__((address_space(1))) const ksh_f64x2 cgf64x2;
 
+constexpr int kSlotVecs = 8;
+__host__ __device__ constexpr size_t pad_rows(int n) { return ((size_t)n + kB - 1) / kB * kB; }
+
 struct TeamMem {
-    gdouble *x, *y, *xo, *cf, *cb, *mat;
-    __device__ explicit TeamMem(const TeamDesc &d)
-        : x((gdouble *)d.x), y((gdouble *)d.y), xo((gdouble *)d.xo), cf((gdouble *)d.cf), cb((gdouble *)d.cb), mat((gdouble *)d.mat)
+    gdouble *x, *b, *y, *xo, *cf, *cb, *mat;
+    __device__ TeamMem(const TeamDesc &d, bool alone) : x((gdouble *)d.x), b((gdouble *)d.b), mat((gdouble *)d.mat)
     {
+        const size_t np = pad_rows(d.n);
+        y = b + np * (alone ? 5 : 1);
+        xo = y + np;
+        cf = xo + np;
+        cb = cf + np;
     }
 };
 
@@ -95,22 +106,27 @@ __device__ __forceinline__ void slot_store(gdouble *p, double v)
     if (b == kSentinel) b = 0x7FF8000000000000ull;
     __hip_atomic_store((gu64 *)p, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// v, a value of *p read before, once it is there (whole wave); `gone` ends all later waits of the wave.  The
+// A wave's waits: `gone`, once a slot did not come within `limit` polls, ends all later ones after one poll.
+struct Poll {
+    unsigned limit;
+    bool gone;
+};
+// v, a value of *p read before, once it is there (whole wave), else NaN.  The
 // first look is outside the polling loop: inside it every wait is for the loop's own load, which would
 // drain the band entries loaded ahead.
-__device__ __forceinline__ double slot_spin(cgdouble *p, bool &gone)
+__device__ __forceinline__ double slot_spin(cgdouble *p, Poll &poll)
 {
     double v;
     unsigned it = 0;
     do {
         v = slot_load(p);
-        gone = gone || ++it > kPollLimit;
-    } while (__any(slot_empty(v)) && !gone);
+        poll.gone = poll.gone || ++it > poll.limit;
+    } while (__any(slot_empty(v)) && !poll.gone);
     return slot_empty(v) ? __builtin_nan("") : v;
 }
-__device__ __forceinline__ double slot_wait(cgdouble *p, double v, bool &gone)
+__device__ __forceinline__ double slot_wait(cgdouble *p, double v, Poll &poll)
 {
-    if (__any(slot_empty(v))) v = slot_spin(p, gone);
+    if (__any(slot_empty(v))) v = slot_spin(p, poll);
     return v;
 }
 
@@ -169,10 +185,8 @@ __global__ __launch_bounds__(256) void k_team_prep(TeamDesc one, const TeamDesc 
     __shared__ double op[4][4 * 64];   // inverse of 16 x 16 block c as an MFMA operand
     TeamDesc d = many ? many[blockIdx.y] : one;
     d.fac = uniform_ptr(d.fac);  // else the band is read in loops over distinct resources
-    d.y = global_ptr(d.y);
-    d.xo = global_ptr(d.xo);
-    d.cf = global_ptr(d.cf);
-    d.cb = global_ptr(d.cb);
+    d.x = global_ptr(d.x);
+    d.b = global_ptr(d.b);
     d.ctl = global_ptr(d.ctl);
     d.mat = global_ptr(uniform_ptr(d.mat));
     const int n = __builtin_amdgcn_readfirstlane(d.n), bw = __builtin_amdgcn_readfirstlane(d.bw);
@@ -196,10 +210,10 @@ __global__ __launch_bounds__(256) void k_team_prep(TeamDesc one, const TeamDesc 
     }
     if (tid < kB) {
         const double empty = __builtin_bit_cast(double, kSentinel);
-        d.y[r0 + tid] = empty;
-        d.xo[r0 + tid] = empty;
-        d.cf[r0 + tid] = empty;
-        d.cb[r0 + tid] = empty;
+        double *p = d.b + r0 + tid;
+        *p = r0 + tid < n ? d.x[r0 + tid] : 0.0;
+#pragma unroll
+        for (int q = 0; q < kSlotVecs; ++q) *(p += pad_rows(n)) = empty;
         if (k == 0 && tid < 2) d.ctl[tid] = 0;
     }
 #pragma unroll
@@ -312,7 +326,7 @@ struct TeamLds {
     double part[kTW][kB];
     double lead[kLeadBuffers][kTW][kB];  // of the leader's, by lead_buffer (one barrier a step, in and between the sweeps)
     double vec[kTW][kU];
-    unsigned team, rank;
+    unsigned team, rank, nan;
 };
 
 // sixteen columns of one of block k's matrices: entries [lane][16 wv + u]
@@ -329,13 +343,13 @@ __device__ __forceinline__ void load_mat(const TeamMem &d, int k, int which, int
 
 // c_k of the forward sweep for blocks k0, k0 + step, ... < k1
 template <typename T>
-__device__ __forceinline__ void help_forward(const Band<T> &B, const TeamMem &d, TeamLds &sh, int k0, int step, int k1, bool &gone)
+__device__ __forceinline__ void help_forward(const Band<T> &B, const TeamMem &d, TeamLds &sh, int k0, int step, int k1, Poll &poll)
 {
     const int lane = B.lane, wv = B.wv, jl = kU * wv + (lane & 15);
     double m[kU], rhs = 0.0;
     auto begin = [&](int k) {  // what the block needs at its end
         load_mat(d, k, kM, wv, lane, m);
-        rhs = kB * k + jl < B.n ? d.x[kB * k + jl] : 0.0;
+        rhs = d.b[kB * k + jl];
     };
     auto finish = [&](int k, double acc) {
         sh.far[wv][lane] = acc;
@@ -373,7 +387,7 @@ __device__ __forceinline__ void help_forward(const Band<T> &B, const TeamMem &d,
     for (;;) {
 #pragma unroll
         for (int p = 0; p < kAhead; ++p) {
-            acc = dot_bcast(acc, slot_wait(d.y + kB * j + jl, yv[p], gone), l[p]);
+            acc = dot_bcast(acc, slot_wait(d.y + kB * j + jl, yv[p], poll), l[p]);
             if (++j > k - 2) {
                 finish(k, acc);
                 acc = 0.0;
@@ -389,7 +403,7 @@ __device__ __forceinline__ void help_forward(const Band<T> &B, const TeamMem &d,
 
 // c_k of the backward sweep for blocks k0, k0 - step, ... >= k1
 template <typename T>
-__device__ __forceinline__ void help_backward(const Band<T> &B, const TeamMem &d, TeamLds &sh, int k0, int step, int k1, bool &gone)
+__device__ __forceinline__ void help_backward(const Band<T> &B, const TeamMem &d, TeamLds &sh, int k0, int step, int k1, Poll &poll)
 {
     const int lane = B.lane, wv = B.wv, jl = kU * wv + (lane >> 2);
     double m[kU], y = 0.0;
@@ -402,7 +416,7 @@ __device__ __forceinline__ void help_backward(const Band<T> &B, const TeamMem &d
     };
     auto finish = [&](int k, const double (&acc)[kU]) {
         const int j = kB * k + jl;
-        const double z = slot_wait(d.y + j, y, gone) / (double)piv;
+        const double z = slot_wait(d.y + j, y, poll) / (double)piv;
         const double t = (j < B.n ? z : 0.0) - sum_lanes(acc, lane);
         // the wave's 16 entries: from one per four lanes to one per lane of each 16-lane row
         if ((lane & 3) == 0) sh.vec[wv][lane >> 2] = t;
@@ -444,7 +458,7 @@ __device__ __forceinline__ void help_backward(const Band<T> &B, const TeamMem &d
     for (;;) {
 #pragma unroll
         for (int p = 0; p < kAhead; ++p) {
-            const double x = slot_wait(d.xo + kB * i + lane, xv[p], gone);
+            const double x = slot_wait(d.xo + kB * i + lane, xv[p], poll);
 #pragma unroll
             for (int u = 0; u < kU; ++u) acc[u] += (double)l[p][u] * x;
             if (--i < k + 2) {
@@ -461,9 +475,9 @@ __device__ __forceinline__ void help_backward(const Band<T> &B, const TeamMem &d
     }
 }
 
-// The chain of one sweep: v_k = c_k - W_k v_prev with W = Q (forward, v = y) or P (backward, v = x)
+// The chain of one sweep: v_k = c_k - W_k v_prev with W = Q (forward, v = y) or P (backward, v = x).
 template <typename T, bool kFwd, bool kAlone>
-__device__ __forceinline__ void lead(const Band<T> &B, const TeamMem &d, TeamLds &sh, bool &gone)
+__device__ __forceinline__ void lead(const Band<T> &B, const TeamMem &d, TeamLds &sh, Poll &poll)
 {
     const int lane = B.lane, wv = B.wv, jl = kU * wv + (lane & 15);
     cgdouble *cs = kFwd ? d.cf : d.cb;
@@ -484,13 +498,13 @@ __device__ __forceinline__ void lead(const Band<T> &B, const TeamMem &d, TeamLds
         sh.lead[buf][wv][lane] = dot_bcast(0.0, v, q.w);
         if constexpr (kAlone) {
             if (kFwd)
-                help_forward<T>(B, d, sh, k, 1, k + 1, gone);
+                help_forward<T>(B, d, sh, k, 1, k + 1, poll);
             else
-                help_backward<T>(B, d, sh, k, 1, k, gone);
+                help_backward<T>(B, d, sh, k, 1, k, poll);
         }
         lds_barrier();
         const double sum = sum_groups(sh.lead[buf][lane >> 4][jl]);
-        v = slot_wait(cs + kB * k + jl, c, gone) - sum;
+        v = slot_wait(cs + kB * k + jl, c, poll) - sum;
         if (lane < kU) {
             slot_store(vs + kB * k + jl, v);
             if (!kFwd && kB * k + jl < B.n) d.x[kB * k + jl] = v;
@@ -513,13 +527,12 @@ __device__ __forceinline__ void lead(const Band<T> &B, const TeamMem &d, TeamLds
 // Teams of `size` workgroups: workgroup id 8 m + c serves band c + 8 (m / size) (workgroups go to the XCDs
 // round robin, so a team's share one)
 template <typename T>
-__global__ __launch_bounds__(64 * kTW) void k_team_solve(TeamDesc one, const TeamDesc *many, int nb, int size)
+__global__ __launch_bounds__(64 * kTW) void k_team_solve(TeamDesc one, const TeamDesc *many, int nb, int size, unsigned polls)
 {
     __shared__ TeamLds sh;
     const int id = (int)blockIdx.x, band = (id & 7) + 8 * ((id >> 3) / size);
     if (band >= nb) return;
     const TeamDesc desc = many ? many[band] : one;
-    const TeamMem d(desc);
     if (threadIdx.x == 0) {
         gu32 *ctl = (gu32 *)desc.ctl;
         const unsigned rank = __hip_atomic_fetch_add(&ctl[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -530,10 +543,11 @@ __global__ __launch_bounds__(64 * kTW) void k_team_solve(TeamDesc one, const Tea
             } while (team < (unsigned)size && ++it < kFormLimit);
             __hip_atomic_store(&ctl[1], team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
-            while (!(team = __hip_atomic_load(&ctl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) && ++it < kPollLimit) {}
+            while (!(team = __hip_atomic_load(&ctl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) && ++it < polls) {}
         }
         sh.team = team;
         sh.rank = rank;
+        sh.nan = 0;
     }
     __syncthreads();
     const int team = __builtin_amdgcn_readfirstlane((int)sh.team), rank = __builtin_amdgcn_readfirstlane((int)sh.rank);
@@ -545,28 +559,36 @@ __global__ __launch_bounds__(64 * kTW) void k_team_solve(TeamDesc one, const Tea
     B.lane = threadIdx.x & 63;
     B.wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     B.rs = band_rsrc(desc.fac, (unsigned)((size_t)desc.n * ((unsigned)desc.bw + 1) * sizeof(T)));
-    bool gone = false;
-    if (rank == 0) {
-        if (team == 1) {
-            lead<T, true, true>(B, d, sh, gone);
-            lead<T, false, true>(B, d, sh, gone);
-        } else {
-            lead<T, true, false>(B, d, sh, gone);
-            lead<T, false, false>(B, d, sh, gone);
-        }
-    } else {
+    Poll poll{polls, false};
+    if (rank > 0) {
+        const TeamMem d(desc, false);
         const int h = rank - 1, H = team - 1;
-        help_forward<T>(B, d, sh, h, H, B.nblk, gone);
-        help_backward<T>(B, d, sh, B.nblk - 1 - h, H, 0, gone);
+        help_forward<T>(B, d, sh, h, H, B.nblk, poll);
+        help_backward<T>(B, d, sh, B.nblk - 1 - h, H, 0, poll);
+        return;
     }
+    if (team > 1) {
+        const TeamMem d(desc, false);
+        lead<T, true, false>(B, d, sh, poll);
+        lead<T, false, false>(B, d, sh, poll);
+        // the chain's last block, read back: kept from the loop, it costs the steps 4% (other waits there)
+        Poll own{kPollLimit, false};
+        cgdouble *last = d.xo + kU * B.wv + (B.lane & 15);
+        const double v = slot_wait(last, slot_load(last), own);
+        if (__any(v != v)) __hip_atomic_store(&sh.nan, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane((int)sh.nan) == 0) return;
+    }
+    const TeamMem d(desc, true);
+    Poll own{kPollLimit, false};
+    lead<T, true, true>(B, d, sh, own);
+    lead<T, false, true>(B, d, sh, own);
 }
-
-size_t pad_rows(int n) { return ((size_t)n + kB - 1) / kB * kB; }
 
 }  // namespace
 
-// one job's workspace: counters, four slot vectors, the blocks' matrices
-size_t team_solve_bytes(int n) { return 256 + pad_rows(n) * (4 + 4 * kB) * sizeof(double); }
+// one job's workspace: counters, right-hand side and slot vectors, the blocks' matrices
+size_t team_solve_bytes(int n) { return 256 + pad_rows(n) * (1 + kSlotVecs + 4 * kB) * sizeof(double); }
 
 // Workgroups per team: the leader, two helpers, and one more per 28 KB of what a block's c_k reads.  Measured
 // (cycles a block, forward): half-width 326 in FP64 10,007 with one helper, 2,772 with 5, 2,340 with 7 and
@@ -580,6 +602,13 @@ static int team_size(int n, int bw, int prec)
     const int far = std::max(0, std::min(bw, n) - kB);
     const double bytes = (double)far * kB * (prec == KSH_FP64 ? 8.0 : 4.0) + 8.0 * kB * kB;
     return 3 + std::min(18, (int)(bytes / 28672.0));
+}
+
+// KSH_TEAM_POLLS=k: waits of at most k polls (any k gives the same bits)
+static unsigned poll_limit()
+{
+    const char *e = std::getenv("KSH_TEAM_POLLS");
+    return e && *e ? (unsigned)std::max(0, std::atoi(e)) : kPollLimit;
 }
 
 // The teams are for calls with few bands, whose time is the chain's: a block and sweep takes about 1 us
@@ -608,11 +637,8 @@ int team_solve(hipStream_t s, const std::vector<TeamJob> &jobs, int prec, void *
         d.n = j.n;
         d.bw = j.bw;
         d.ctl = (unsigned *)p;
-        d.y = (double *)(p + 256);
-        d.xo = d.y + np;
-        d.cf = d.xo + np;
-        d.cb = d.cf + np;
-        d.mat = d.cb + np;
+        d.b = (double *)(p + 256);
+        d.mat = d.b + np * (1 + kSlotVecs);
         p += team_solve_bytes(j.n);
         h.push_back(d);
         nblk = std::max(nblk, (int)(np / kB));
@@ -627,10 +653,10 @@ int team_solve(hipStream_t s, const std::vector<TeamJob> &jobs, int prec, void *
     const dim3 gp((unsigned)nblk, (unsigned)nb), gs((unsigned)(8 * size * ((nb + 7) / 8)));
     if (prec == KSH_FP64) {
         hipLaunchKernelGGL(k_team_prep<double>, gp, dim3(256), 0, s, h[0], many);
-        hipLaunchKernelGGL(k_team_solve<double>, gs, dim3(64 * kTW), 0, s, h[0], many, nb, size);
+        hipLaunchKernelGGL(k_team_solve<double>, gs, dim3(64 * kTW), 0, s, h[0], many, nb, size, poll_limit());
     } else {
         hipLaunchKernelGGL(k_team_prep<float>, gp, dim3(256), 0, s, h[0], many);
-        hipLaunchKernelGGL(k_team_solve<float>, gs, dim3(64 * kTW), 0, s, h[0], many, nb, size);
+        hipLaunchKernelGGL(k_team_solve<float>, gs, dim3(64 * kTW), 0, s, h[0], many, nb, size, poll_limit());
     }
     KSH_HIP(hipGetLastError());
     return KSH_SUCCESS;

@@ -7,7 +7,8 @@ Checked by the backward error of the solve, ||b - K x|| <= c eps G ||x||: G, the
 precision, and c = 8 bw + 64 + 512 covers one rounding per product along a band row, for the factor and
 the two sweeps, plus the 64-wide inverses and products of a block (eight of 64 terms).  And by the
 team's size changing nothing: every sum has one order, whoever forms it, so a leader alone, with one
-helper or with many gives the same bits."""
+helper or with many gives the same bits.  And so does one whose waits end early (KSH_TEAM_POLLS): a leader
+whose chain ends with NaN solves again by itself, so a wait that runs out costs time and nothing else."""
 import numpy as np
 import pytest
 
@@ -15,6 +16,7 @@ from gsstructuralanalysis_amd import _lib as L
 from gsstructuralanalysis_amd import geometry as g
 from oracle import ok
 from oracle.ok import Oracle
+from test_zz_no_alloc import DevArray
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +63,43 @@ def test_team_solve_at_block_edges(p, nx, ny, prec, ksh, monkeypatch):
             monkeypatch.setenv("KSH_TEAM", size)
             assert np.array_equal(A.solve(b), x), size
         monkeypatch.delenv("KSH_TEAM")
+
+
+def _device_solve(K, b):
+    """ksh_solve_dev without refinement, which looks at no result: what it leaves in the caller's vector."""
+    bd, xd = DevArray(K.n), DevArray(K.n)
+    try:
+        bd.upload(b)
+        xd.upload(np.full(K.n, np.nan))
+        L.check(L.load().ksh_solve_dev(K.handle, bd.p, xd.p, 0, 0.0))
+        L.check(L.load().ksh_synchronize(K.problem.handle))
+        return xd.download()
+    finally:
+        bd.free()
+        xd.free()
+
+
+@pytest.mark.parametrize("p,nx,ny", [(2, 1, 15), (3, 3, 12), (3, 13, 8), (3, 140, 2)])
+@pytest.mark.parametrize("prec", [L.FP64, L.FP32_IR])
+def test_waits_that_run_out_change_nothing(p, nx, ny, prec, ksh, monkeypatch):
+    from gsstructuralanalysis_amd.problem import BandMatrix, ShellProblem
+    pt = g.roof_problem(p=p, n=nx, ny=ny)
+    o = Oracle(pt)
+    sp = ShellProblem(pt)
+    rng = np.random.default_rng(29)
+    A = BandMatrix(sp, precision=prec)
+    A.upload(o.tangent_band(rng.standard_normal(o.nfree) * 1e-4))
+    A.set_inertia_guard(0.0)
+    A.factor()
+    b = rng.standard_normal(o.nfree)
+    x = A.solve(b)
+    assert np.all(np.isfinite(x))
+    for polls in ("0", "1", "4", "16", "64"):
+        monkeypatch.setenv("KSH_TEAM_POLLS", polls)
+        for size in ("2", "5", "12"):
+            monkeypatch.setenv("KSH_TEAM", size)
+            print(f"[case] team solve nfree={o.nfree} bw={o.bw} prec={prec} polls={polls} team={size}", flush=True)
+            assert np.array_equal(_device_solve(A, b), x), (polls, size)
+    monkeypatch.delenv("KSH_TEAM_POLLS")
+    b[o.nfree // 2] = np.nan  # the right-hand side's own NaN stays one
+    assert np.isnan(_device_solve(A, b)).all()
