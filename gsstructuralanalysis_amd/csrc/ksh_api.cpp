@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "ksh_internal.hpp"
+#include "ksh_profile.hpp"
 
 namespace ksh {
 
@@ -151,7 +152,7 @@ void destroy_problem(Problem *pb)
                     pb->d_desc, pb->modal_P, pb->modal_Phi, pb->modal_zfree};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
-    if (pb->stream) (void)hipStreamDestroy(pb->stream);
+    destroy_stream(pb->stream);
 }
 
 void destroy_matrix(Matrix *K)

@@ -29,11 +29,11 @@ BatchDevice::~BatchDevice()
 {
     if (m_early_stream) {
         (void)hipStreamSynchronize(m_early_stream);
-        (void)hipStreamDestroy(m_early_stream);
+        destroy_stream(m_early_stream);
     }
     if (m_rc_stream) {
         (void)hipStreamSynchronize(m_rc_stream);
-        (void)hipStreamDestroy(m_rc_stream);
+        destroy_stream(m_rc_stream);
     }
     for (auto &b : m_rcb) {
         if (b->done) (void)hipEventDestroy(b->done);
@@ -44,7 +44,7 @@ BatchDevice::~BatchDevice()
     if (m_ev_copied) (void)hipEventDestroy(m_ev_copied);
     if (m_ev_early) (void)hipEventDestroy(m_ev_early);
     if (m_hearly) (void)hipHostFree(m_hearly);
-    if (m_stream) (void)hipStreamDestroy(m_stream);
+    destroy_stream(m_stream);
 }
 
 int BatchDevice::init()

@@ -404,7 +404,7 @@ int ksh_mlp_destroy(ksh_mlp *m)
         (void)hipFree(m->dZ[l]);
     }
     (void)hipFree(m->idx);
-    if (m->s) (void)hipStreamDestroy(m->s);
+    destroy_stream(m->s);
     delete m;
     return KSH_SUCCESS;
 }

@@ -1,7 +1,9 @@
 // ksh_profile.cpp -- optional per-kernel timing with HIP events recorded on the launching stream.
 //
 // When enabled, each launcher brackets its kernel with a pair of events from a recycled pool;
-// ksh_profile_query() waits for the pending pairs and accumulates hipEventElapsedTime per kernel.
+// ksh_profile_query() waits for the pending pairs and accumulates hipEventElapsedTime per kernel.  The
+// pairs of a stream are read before it is destroyed: an event recorded on a destroyed stream counts for one
+// of whatever stream lives at its address later, and asking for it fails, and ends a capture there.
 #include <hip/hip_runtime.h>
 
 #include <map>
@@ -16,8 +18,12 @@ namespace ksh {
 
 namespace {
 
+struct Pending {
+    hipEvent_t start, stop;
+    hipStream_t stream;
+};
 struct Entry {
-    std::vector<std::pair<hipEvent_t, hipEvent_t>> pending;
+    std::vector<Pending> pending;
     double total_ms = 0.0;
     long long count = 0;
     double work = 0.0;
@@ -40,19 +46,25 @@ hipEvent_t take_event()
     return e;
 }
 
-void drain(Entry &en)
+// reads the pending pairs of one stream, or all of them
+void drain(Entry &en, const hipStream_t *stream = nullptr)
 {
+    std::vector<Pending> rest;
     for (auto &pr : en.pending) {
-        (void)hipEventSynchronize(pr.second);
+        if (stream && pr.stream != *stream) {
+            rest.push_back(pr);
+            continue;
+        }
+        (void)hipEventSynchronize(pr.stop);
         float ms = 0.f;
-        if (hipEventElapsedTime(&ms, pr.first, pr.second) == hipSuccess) {
+        if (hipEventElapsedTime(&ms, pr.start, pr.stop) == hipSuccess) {
             en.total_ms += ms;
             en.count += 1;
         }
-        g_pool.push_back(pr.first);
-        g_pool.push_back(pr.second);
+        g_pool.push_back(pr.start);
+        g_pool.push_back(pr.stop);
     }
-    en.pending.clear();
+    en.pending.swap(rest);
 }
 
 }  // namespace
@@ -64,6 +76,16 @@ void prof_count(const char *name, long long n)
     if (!g_on || n == 0) return;
     std::lock_guard<std::mutex> lk(g_mu);
     g_entries[name].count += n;
+}
+
+void destroy_stream(hipStream_t s)
+{
+    if (!s) return;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        for (auto &kv : g_entries) drain(kv.second, &s);
+    }
+    (void)hipStreamDestroy(s);
 }
 
 ProfScope::ProfScope(const char *name, hipStream_t s) : m_name(name), m_stream(s)
@@ -82,7 +104,7 @@ ProfScope::~ProfScope()
     std::lock_guard<std::mutex> lk(g_mu);
     (void)hipEventRecord(m_stop, m_stream);
     Entry &en = g_entries[m_name];
-    en.pending.emplace_back(m_start, m_stop);
+    en.pending.push_back({m_start, m_stop, m_stream});
     en.work += m_work;
 }
 

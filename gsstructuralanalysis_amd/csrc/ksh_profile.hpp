@@ -9,6 +9,9 @@ bool profiling();
 // adds n events to the counter `name` (reported by ksh_profile_query as launches, 0 ms)
 void prof_count(const char *name, long long n);
 
+// hipStreamDestroy, for every stream that a ProfScope may have recorded on
+void destroy_stream(hipStream_t s);
+
 class ProfScope {
 public:
     ProfScope(const char *name, hipStream_t s);
