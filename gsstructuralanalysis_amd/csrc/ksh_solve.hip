@@ -599,18 +599,15 @@ bool band_use_tiled_solve(int n, int bw, int prec)
     return (double)(bw + 1) * es >= 3072.0;
 }
 
-// Workspace of K's team solves, allocated on first use; false where it cannot be (a capturing stream, no
-// memory left), and the other solve paths take the call
-static bool team_workspace(Matrix &K)
+// With the matrix, so that no solve allocates (solves may be captured, or run beside another thread's
+// capture, which an allocation would end).  Without memory for it the other solves serve the matrix.
+void team_workspace(Matrix &K)
 {
-    if (K.team_ws) return true;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(K.pb->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
+    if (!team_solve_takes(K.n, K.bw, KSH_FP64, 1) && !team_solve_takes(K.n, K.bw, KSH_FP32, 1)) return;
     if (hipMalloc(&K.team_ws, team_solve_bytes(K.n)) != hipSuccess) {
         (void)hipGetLastError();
         K.team_ws = nullptr;
     }
-    return K.team_ws != nullptr;
 }
 
 static bool band_path_forced()
@@ -622,7 +619,7 @@ static bool band_path_forced()
 int band_solve(Matrix &K, const void *fac, int prec, double *x_dev)
 {
     Problem &pb = *K.pb;
-    if (!band_path_forced() && team_solve_takes(K.n, K.bw, prec, 1) && team_workspace(K)) {
+    if (!band_path_forced() && team_solve_takes(K.n, K.bw, prec, 1) && K.team_ws) {
         ProfScope ps("band_solve", pb.stream);
         ps.set_work(2.0 * K.n * (K.bw + 1.0) * (prec == KSH_FP64 ? 8.0 : 4.0) + 16.0 * K.n);
         return team_solve(pb.stream, {TeamJob{fac, K.n, K.bw, x_dev}}, prec, K.team_ws, nullptr);

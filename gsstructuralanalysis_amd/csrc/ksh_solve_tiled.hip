@@ -17,8 +17,8 @@
 // Rows touched by one launch belong to one workgroup, and the block rows are read but not
 // written, so launches on one stream need no other synchronization.  HBM traffic: the band once
 // per sweep, 2 n (bw+1) entries per solve.  Single bands take the resident teams (ksh_solve_team.hip: one
-// launch, 2.3 ms against 11.2 on that plate); these launches serve a stream that is being captured before
-// the team's workspace exists, a device without room for it, and KSH_BAND_PATH=tiled.  Replaces
+// launch, 2.3 ms against 11.2 on that plate); these launches serve a device without room for
+// the team's workspace, and KSH_BAND_PATH=tiled.  Replaces
 // SimplicialLDLT::solve
 // (src/gsEigenSolvers/gsEigenProblemBase.hpp:152-216 drives it through the shift-invert operator).
 #include <hip/hip_runtime.h>

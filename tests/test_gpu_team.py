@@ -9,6 +9,8 @@ the two sweeps, plus the 64-wide inverses and products of a block (eight of 64 t
 team's size changing nothing: every sum has one order, whoever forms it, so a leader alone, with one
 helper or with many gives the same bits.  And so does one whose waits end early (KSH_TEAM_POLLS): a leader
 whose chain ends with NaN solves again by itself, so a wait that runs out costs time and nothing else."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -103,3 +105,28 @@ def test_waits_that_run_out_change_nothing(p, nx, ny, prec, ksh, monkeypatch):
     monkeypatch.delenv("KSH_TEAM_POLLS")
     b[o.nfree // 2] = np.nan  # the right-hand side's own NaN stays one
     assert np.isnan(_device_solve(A, b)).all()
+
+
+def test_solves_allocate_nothing(ksh):
+    """The workspace comes with the matrix: the first solve with a factor leaves the device's free memory
+    as it was (7 MB of workspace at this size, over the allocator's 2 MiB granule)."""
+    from gsstructuralanalysis_amd.problem import ShellProblem
+    hip = C.CDLL("libamdhip64.so.7")
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    sp = ShellProblem(g.roof_problem(p=3, n=32))
+    print(f"[case] allocation of solves, roof 32x32 nfree={sp.nfree} bw={sp.bw}", flush=True)
+    rng = np.random.default_rng(31)
+    u, b = rng.standard_normal(sp.nfree) * 1e-4, rng.standard_normal(sp.nfree)
+    keep = []
+    for k in range(3):  # the first loads the kernels
+        K = sp.tangent(u)
+        K.factor()
+        before = free_bytes()
+        keep.append((K, K.solve(b)))
+        assert k == 0 or free_bytes() == before
+    assert np.array_equal(keep[0][1], keep[1][1]) and np.array_equal(keep[0][1], keep[2][1])
