@@ -257,44 +257,6 @@ int ensure_rc64(Matrix &K)
     return KSH_SUCCESS;
 }
 
-int matrix_create(ksh_problem *pb, int prec, bool solves, ksh_matrix **out)
-{
-    if (!pb || !out) return fail(KSH_OTHER_ERROR, "null argument");
-    if (prec != KSH_FP64 && prec != KSH_FP32_IR && prec != KSH_FP32) return fail(KSH_OTHER_ERROR, "unknown precision");
-    ksh_matrix *K = new ksh_matrix();
-    K->pb = pb;
-    K->n = pb->nfree;
-    K->bw = pb->bw;
-    K->ld = (size_t)pb->bw + 1;
-    K->prec = prec;
-    K->sprec = storage_prec(prec);
-    K->fprec = factor_prec(prec);
-    K->guard = pb->inertia_guard;
-    K->accept = pb->refine_accept;
-    int rc = 0;
-    size_t count = (size_t)K->n * K->ld, eb = elem_bytes(K->sprec), fb = elem_bytes(K->fprec);
-    auto bail = [&](int code) {
-        destroy_matrix(K);
-        delete K;
-        return code;
-    };
-    if (!(K->ab = dalloc<unsigned char>(count * eb, rc))) return bail(rc);
-    if (!(K->fac = dalloc<unsigned char>(count * fb, rc))) return bail(rc);
-    if (!(K->work = dalloc<double>((size_t)5 * K->n, rc))) return bail(rc);
-    if (!(K->flag = dalloc<int>(4, rc))) return bail(rc);
-    if (!(K->red = dalloc<double>(8, rc))) return bail(rc);
-    if (!(K->desc = dalloc<unsigned char>(factor_desc_bytes(1), rc))) return bail(rc);
-    if (K->sprec == KSH_FP32 && !(K->u_at = dalloc<double>(K->n, rc))) return bail(rc);
-    // zeroed before return: the matrix may next be written on another stream (a batch engine's),
-    // which must not race with this clear
-    if (hipMemsetAsync(K->ab, 0, count * eb, pb->stream) != hipSuccess || hipStreamSynchronize(pb->stream) != hipSuccess)
-        return bail(fail(KSH_OTHER_ERROR, "memset"));
-    K->ab_clean = true;
-    if (solves) team_workspace(*K);
-    *out = K;
-    return KSH_SUCCESS;
-}
-
 }  // namespace ksh
 
 using namespace ksh;
@@ -529,7 +491,42 @@ int ksh_assemble_residual(ksh_problem *pb, const double *u_free, double lambda, 
     return KSH_SUCCESS;
 }
 
-int ksh_matrix_create(ksh_problem *pb, int prec, ksh_matrix **out) { return matrix_create(pb, prec, true, out); }
+int ksh_matrix_create(ksh_problem *pb, int prec, ksh_matrix **out)
+{
+    if (!pb || !out) return fail(KSH_OTHER_ERROR, "null argument");
+    if (prec != KSH_FP64 && prec != KSH_FP32_IR && prec != KSH_FP32) return fail(KSH_OTHER_ERROR, "unknown precision");
+    ksh_matrix *K = new ksh_matrix();
+    K->pb = pb;
+    K->n = pb->nfree;
+    K->bw = pb->bw;
+    K->ld = (size_t)pb->bw + 1;
+    K->prec = prec;
+    K->sprec = storage_prec(prec);
+    K->fprec = factor_prec(prec);
+    K->guard = pb->inertia_guard;
+    K->accept = pb->refine_accept;
+    int rc = 0;
+    size_t count = (size_t)K->n * K->ld, eb = elem_bytes(K->sprec), fb = elem_bytes(K->fprec);
+    auto bail = [&](int code) {
+        destroy_matrix(K);
+        delete K;
+        return code;
+    };
+    if (!(K->ab = dalloc<unsigned char>(count * eb, rc))) return bail(rc);
+    if (!(K->fac = dalloc<unsigned char>(count * fb, rc))) return bail(rc);
+    if (!(K->work = dalloc<double>((size_t)5 * K->n, rc))) return bail(rc);
+    if (!(K->flag = dalloc<int>(4, rc))) return bail(rc);
+    if (!(K->red = dalloc<double>(8, rc))) return bail(rc);
+    if (!(K->desc = dalloc<unsigned char>(factor_desc_bytes(1), rc))) return bail(rc);
+    if (K->sprec == KSH_FP32 && !(K->u_at = dalloc<double>(K->n, rc))) return bail(rc);
+    // zeroed before return: the matrix may next be written on another stream (a batch engine's),
+    // which must not race with this clear
+    if (hipMemsetAsync(K->ab, 0, count * eb, pb->stream) != hipSuccess || hipStreamSynchronize(pb->stream) != hipSuccess)
+        return bail(fail(KSH_OTHER_ERROR, "memset"));
+    K->ab_clean = true;
+    *out = K;
+    return KSH_SUCCESS;
+}
 
 int ksh_matrix_destroy(ksh_matrix *K)
 {
@@ -676,6 +673,7 @@ int ksh_factor(ksh_matrix *K)
     K->rho = 0.0;
     K->rho_obs = 0;
     K->rho_pw = -1.0;
+    if (!K->team_ws) team_workspace(*K);
     double st[4] = {0, 0, 0, 0};
     int rc = band_factor(*K, K->fac, K->fprec, st);
     K->factored = true;

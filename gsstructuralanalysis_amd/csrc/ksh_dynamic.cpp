@@ -54,7 +54,7 @@ struct Matrices {
     {
         ksh_matrix *K = nullptr;
         int rc;
-        if ((rc = matrix_create(static_cast<ksh_problem *>(pb), prec, false, &K))) return rc;
+        if ((rc = ksh_matrix_create(static_cast<ksh_problem *>(pb), prec, &K))) return rc;
         ms.push_back(K);
         *out = K;
         return KSH_SUCCESS;

@@ -230,7 +230,7 @@ constexpr size_t kBandWorkBytes = 3 * 8704;
 inline size_t factor_desc_offset(size_t n) { return (n * kBandDescBytes + 255) / 256 * 256; }
 inline size_t factor_desc_bytes(size_t n) { return factor_desc_offset(n) + n * kBandWorkBytes; }
 int band_solve(Matrix &K, const void *fac, int prec, double *x_dev);
-// K's team solve workspace, where a team takes its solves and there is memory for it
+// K's team solve workspace, where a team takes its solves and there is memory for it (ksh_factor)
 void team_workspace(Matrix &K);
 // solve of one large band by stepped launches (ksh_solve_tiled.hip); z: n doubles of workspace
 int band_solve_tiled(hipStream_t s, const void *fac, int prec, int n, int bw, double *x, double *z);
@@ -271,9 +271,3 @@ int vec_norm2(hipStream_t s, int n, const double *x, double *scratch, double *ho
 
 struct ksh_problem : ksh::Problem {};
 struct ksh_matrix : ksh::Matrix {};
-
-namespace ksh {
-// ksh_matrix_create; `solves`: ksh_solve[_dev] will be called for it (the engines' batched solves need no
-// workspace of the matrix)
-int matrix_create(ksh_problem *pb, int prec, bool solves, ksh_matrix **out);
-}  // namespace ksh

@@ -241,7 +241,7 @@ private:
             if (m_o.refine_accept > 0) I.pb->refine_accept = m_o.refine_accept;
             ksh_matrix *K = nullptr;
             int rc;
-            if ((rc = matrix_create(static_cast<ksh_problem *>(I.pb), m_o.precision, false, &K))) return rc;
+            if ((rc = ksh_matrix_create(static_cast<ksh_problem *>(I.pb), m_o.precision, &K))) return rc;
             m_mats.ms.push_back(K);
             I.K = K;
             I.arc = I.arc0 = I.arc_prev = m_o.lengths ? m_o.lengths[i] : m_o.length;
@@ -1288,7 +1288,7 @@ private:
         for (Inst *I : g)
             if (!I->Keps) {
                 ksh_matrix *K = nullptr;
-                if ((rc = matrix_create(static_cast<ksh_problem *>(I->pb), KSH_FP64, false, &K))) return rc;
+                if ((rc = ksh_matrix_create(static_cast<ksh_problem *>(I->pb), KSH_FP64, &K))) return rc;
                 m_mats.ms.push_back(K);
                 I->Keps = K;
             }
@@ -1552,7 +1552,7 @@ public:
             if (o.inertia_guard != 0) I.pb->inertia_guard = o.inertia_guard > 0 ? o.inertia_guard : 0.0;
             if (o.refine_accept > 0) I.pb->refine_accept = o.refine_accept;
             ksh_matrix *K = nullptr;
-            if ((rc = matrix_create(static_cast<ksh_problem *>(I.pb), o.precision, false, &K))) return rc;
+            if ((rc = ksh_matrix_create(static_cast<ksh_problem *>(I.pb), o.precision, &K))) return rc;
             m_mats.ms.push_back(K);
             I.K = K;
             if (o.nsteps == 0) I.ph = Phase::Done;

@@ -108,25 +108,33 @@ def test_waits_that_run_out_change_nothing(p, nx, ny, prec, ksh, monkeypatch):
 
 
 def test_solves_allocate_nothing(ksh):
-    """The workspace comes with the matrix: the first solve with a factor leaves the device's free memory
-    as it was (7 MB of workspace at this size, over the allocator's 2 MiB granule)."""
+    """The workspace comes with the factor: the first solve with a factor runs beside a capture that is open
+    in global mode on another stream, which any allocation in the process would end, and gives the bits of
+    a later solve."""
     from gsstructuralanalysis_amd.problem import ShellProblem
-    hip = C.CDLL("libamdhip64.so.7")
-
-    def free_bytes():
-        free, total = C.c_size_t(), C.c_size_t()
-        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
-        return free.value
-
-    sp = ShellProblem(g.roof_problem(p=3, n=32))
-    print(f"[case] allocation of solves, roof 32x32 nfree={sp.nfree} bw={sp.bw}", flush=True)
+    hip, lib = C.CDLL("libamdhip64.so.7"), L.load()
+    sp = ShellProblem(g.roof_problem(p=3, n=12))
+    print(f"[case] solve beside a capture, roof 12x12 nfree={sp.nfree} bw={sp.bw}", flush=True)
     rng = np.random.default_rng(31)
     u, b = rng.standard_normal(sp.nfree) * 1e-4, rng.standard_normal(sp.nfree)
-    keep = []
-    for k in range(3):  # the first loads the kernels
-        K = sp.tangent(u)
-        K.factor()
-        before = free_bytes()
-        keep.append((K, K.solve(b)))
-        assert k == 0 or free_bytes() == before
-    assert np.array_equal(keep[0][1], keep[1][1]) and np.array_equal(keep[0][1], keep[2][1])
+    K = sp.tangent(u)
+    K.factor()
+    bd, xd = DevArray(K.n), DevArray(K.n)
+    s, graph = C.c_void_p(), C.c_void_p()
+    try:
+        bd.upload(b)
+        assert hip.hipStreamCreateWithFlags(C.byref(s), 1) == 0  # non-blocking
+        assert hip.hipStreamBeginCapture(s, 0) == 0              # global mode
+        rc = lib.ksh_solve_dev(K.handle, bd.p, xd.p, 0, 0.0)
+        ended = hip.hipStreamEndCapture(s, C.byref(graph))
+        L.check(rc)
+        assert ended == 0
+        L.check(lib.ksh_synchronize(sp.handle))
+        assert np.array_equal(xd.download(), K.solve(b))
+    finally:
+        if graph:
+            hip.hipGraphDestroy(graph)
+        if s:
+            hip.hipStreamDestroy(s)
+        bd.free()
+        xd.free()
