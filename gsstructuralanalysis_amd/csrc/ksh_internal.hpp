@@ -234,17 +234,11 @@ int band_solve(Matrix &K, const void *fac, int prec, double *x_dev);
 void team_workspace(Matrix &K);
 // solve of one large band by stepped launches (ksh_solve_tiled.hip); z: n doubles of workspace
 int band_solve_tiled(hipStream_t s, const void *fac, int prec, int n, int bw, double *x, double *z);
-// solves by resident teams of workgroups (ksh_solve_team.hip); work: the sum of team_solve_bytes(n) over
-// the jobs, kept by the caller until the solve is done; d_descs: kTeamDescBytes a job (unused for one)
-struct TeamJob {
-    const void *fac;
-    int n, bw;
-    double *x;
-};
-constexpr size_t kTeamDescBytes = 80;
+// solve by a resident team of workgroups (ksh_solve_team.hip); work: team_solve_bytes(n), kept by the
+// caller until the solve is done
 size_t team_solve_bytes(int n);
-bool team_solve_takes(int n, int bw, int prec, int count);
-int team_solve(hipStream_t s, const std::vector<TeamJob> &jobs, int prec, void *work, void *d_descs);
+bool team_solve_takes(int n, int bw, int prec);
+int team_solve(hipStream_t s, const void *fac, int n, int bw, double *x, int prec, void *work);
 // path of a single-band factor / solve: 1 = multi-workgroup (tiled), 0 = one workgroup
 bool band_use_tiled_factor(int n, int bw, int prec);
 bool band_use_tiled_solve(int n, int bw, int prec);

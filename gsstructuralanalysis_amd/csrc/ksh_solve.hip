@@ -605,7 +605,7 @@ bool band_use_tiled_solve(int n, int bw, int prec)
 // the matrix.
 void team_workspace(Matrix &K)
 {
-    if (!team_solve_takes(K.n, K.bw, KSH_FP64, 1) && !team_solve_takes(K.n, K.bw, KSH_FP32, 1)) return;
+    if (!team_solve_takes(K.n, K.bw, KSH_FP32)) return;
     if (hipMalloc(&K.team_ws, team_solve_bytes(K.n)) != hipSuccess) {
         (void)hipGetLastError();
         K.team_ws = nullptr;
@@ -621,10 +621,10 @@ static bool band_path_forced()
 int band_solve(Matrix &K, const void *fac, int prec, double *x_dev)
 {
     Problem &pb = *K.pb;
-    if (!band_path_forced() && team_solve_takes(K.n, K.bw, prec, 1) && K.team_ws) {
+    if (!band_path_forced() && team_solve_takes(K.n, K.bw, prec) && K.team_ws) {
         ProfScope ps("band_solve", pb.stream);
         ps.set_work(2.0 * K.n * (K.bw + 1.0) * (prec == KSH_FP64 ? 8.0 : 4.0) + 16.0 * K.n);
-        return team_solve(pb.stream, {TeamJob{fac, K.n, K.bw, x_dev}}, prec, K.team_ws, nullptr);
+        return team_solve(pb.stream, fac, K.n, K.bw, x_dev, prec, K.team_ws);
     }
     if (band_use_tiled_solve(K.n, K.bw, prec)) {
         ProfScope ps("band_solve_tiled", pb.stream);

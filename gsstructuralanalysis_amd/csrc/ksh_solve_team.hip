@@ -1,4 +1,4 @@
-// ksh_solve_team.hip -- L D L^T solve of one band, or of a few, by a team of workgroups each.
+// ksh_solve_team.hip -- L D L^T solve of one band by a team of workgroups.
 //
 // A band solve is a chain: 64-row block k needs the solution of the block before it.  One workgroup
 // per band (ksh_solve.hip) streams the whole band through one CU, 5 us per block and sweep at half-width
@@ -34,7 +34,6 @@
 
 #include <algorithm>
 #include <cstdlib>
-#include <vector>
 
 #include "ksh_devutil.hpp"
 #include "ksh_internal.hpp"
@@ -71,8 +70,8 @@ constexpr int kM = 0, kMt = 1, kMq = 2, kMp = 3;
 // entry (row, col) of such a matrix: pairs of columns interleaved, so that a lane (= row) loads 16 bytes
 __host__ __device__ constexpr int mat_at(int row, int col) { return (col >> 1) * 128 + 2 * row + (col & 1); }
 
-// Pointers of a descriptor read from memory are generic to the compiler, and flat accesses drain every load
-// in flight at each wait; the kernels below use them as what they are, global memory.
+// The team's kernel takes its pointers as what they are, global memory: through generic ones every access would
+// be a flat one, which drains every load in flight at each wait.
 typedef __attribute__((address_space(1))) double gdouble;
 typedef __attribute__((address_space(1))) const double cgdouble;
 typedef __attribute__((address_space(1))) unsigned long long gu64;
@@ -175,7 +174,7 @@ __device__ __forceinline__ double dot_bcast(double acc, double v, const float (&
 // columns 16 w .. 16 w + 15 by 16-row blocks on MFMA, substitution between them.  Q_k and P_k^T = L_{k+1,k}
 // M_k are products on MFMA.  FP64 for both factor precisions.
 template <typename T>
-__global__ __launch_bounds__(256) void k_team_prep(TeamDesc one, const TeamDesc *many)
+__global__ __launch_bounds__(256) void k_team_prep(TeamDesc d)
 {
     using M = Mfma16<double>;
     constexpr int Q = 16;
@@ -183,15 +182,8 @@ __global__ __launch_bounds__(256) void k_team_prep(TeamDesc one, const TeamDesc 
     __shared__ double ns[kB][kB + 1];  // L_{k,k-1}
     __shared__ double ms[kB][kB + 1];  // M_k
     __shared__ double op[4][4 * 64];   // inverse of 16 x 16 block c as an MFMA operand
-    TeamDesc d = many ? many[blockIdx.y] : one;
-    d.fac = uniform_ptr(d.fac);  // else the band is read in loops over distinct resources
-    d.x = global_ptr(d.x);
-    d.b = global_ptr(d.b);
-    d.ctl = global_ptr(d.ctl);
-    d.mat = global_ptr(uniform_ptr(d.mat));
-    const int n = __builtin_amdgcn_readfirstlane(d.n), bw = __builtin_amdgcn_readfirstlane(d.bw);
-    const int nblk = (n + kB - 1) / kB, k = (int)blockIdx.x;
-    if (k >= nblk) return;
+    const int n = d.n, bw = d.bw;
+    const int k = (int)blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r0 = k * kB;
@@ -524,15 +516,18 @@ __device__ __forceinline__ void lead(const Band<T> &B, const TeamMem &d, TeamLds
     }
 }
 
-// Teams of `size` workgroups: workgroup id 8 m + c serves band c + 8 (m / size) (workgroups go to the XCDs
-// round robin, so a team's share one)
+// A team of up to `size` workgroups: every eighth one of the grid (workgroups go to the XCDs round robin, so
+// they share one), the others leave
 template <typename T>
-__global__ __launch_bounds__(64 * kTW) void k_team_solve(TeamDesc one, const TeamDesc *many, int nb, int size, unsigned polls)
+__global__ __launch_bounds__(64 * kTW) void k_team_solve(TeamDesc desc, int size, unsigned polls)
 {
     __shared__ TeamLds sh;
-    const int id = (int)blockIdx.x, band = (id & 7) + 8 * ((id >> 3) / size);
-    if (band >= nb) return;
-    const TeamDesc desc = many ? many[band] : one;
+    if (blockIdx.x % 8 != 0) return;
+    // (as values of this kernel; as its arguments the compiler places the helpers' loads worse: 1.5% of a solve)
+    desc.fac = uniform_ptr(desc.fac);
+    desc.x = uniform_ptr(desc.x);
+    desc.b = uniform_ptr(desc.b);
+    desc.mat = uniform_ptr(desc.mat);
     if (threadIdx.x == 0) {
         gu32 *ctl = (gu32 *)desc.ctl;
         const unsigned rank = __hip_atomic_fetch_add(&ctl[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -587,7 +582,7 @@ __global__ __launch_bounds__(64 * kTW) void k_team_solve(TeamDesc one, const Tea
 
 }  // namespace
 
-// one job's workspace: counters, right-hand side and slot vectors, the blocks' matrices
+// workspace: counters, right-hand side and slot vectors, the blocks' matrices
 size_t team_solve_bytes(int n) { return 256 + pad_rows(n) * (1 + kSlotVecs + 4 * kB) * sizeof(double); }
 
 // Workgroups per team: the leader, two helpers, and one more per 28 KB of what a block's c_k reads.  Measured
@@ -611,52 +606,36 @@ static unsigned poll_limit()
     return e && *e ? (unsigned)std::max(0, std::atoi(e)) : kPollLimit;
 }
 
-// The teams are for calls with few bands, whose time is the chain's: a block and sweep takes about 1 us
+// The team is for calls with one band, whose time is the chain's: a block and sweep takes about 1 us
 // against 5 us in the one-workgroup kernel (roof 32 x 32: 562 -> 120 us a solve, of which 11 us form the
 // matrices) and 7 us in the stepped one (128 x 128 plate: 11.2 -> 2.3 ms).  Up to two blocks the
 // one-workgroup kernel is as fast.  With all the chip's CUs on bands of their own (batches), that kernel's
 // traffic, the band alone, is the lower one.
-bool team_solve_takes(int n, int bw, int prec, int count)
+bool team_solve_takes(int n, int bw, int prec)
 {
     const size_t es = prec == KSH_FP64 ? sizeof(double) : sizeof(float);
-    if ((size_t)n * (size_t)(bw + 1) * es >= 0x7F000000ull) return false;
-    return n > 2 * kB && (count + 7) / 8 * team_size(n, bw, prec) <= 32;
+    return n > 2 * kB && (size_t)n * (size_t)(bw + 1) * es < 0x7F000000ull;
 }
 
-int team_solve(hipStream_t s, const std::vector<TeamJob> &jobs, int prec, void *work, void *d_descs)
+int team_solve(hipStream_t s, const void *fac, int n, int bw, double *x, int prec, void *work)
 {
-    if (jobs.empty()) return KSH_SUCCESS;
-    std::vector<TeamDesc> h;
-    unsigned char *p = (unsigned char *)work;
-    int nblk = 0, size = 1;
-    for (const TeamJob &j : jobs) {
-        const size_t np = pad_rows(j.n);
-        TeamDesc d;
-        d.fac = j.fac;
-        d.x = j.x;
-        d.n = j.n;
-        d.bw = j.bw;
-        d.ctl = (unsigned *)p;
-        d.b = (double *)(p + 256);
-        d.mat = d.b + np * (1 + kSlotVecs);
-        p += team_solve_bytes(j.n);
-        h.push_back(d);
-        nblk = std::max(nblk, (int)(np / kB));
-        size = std::max(size, team_size(j.n, j.bw, prec));
-    }
-    const int nb = (int)h.size();
-    const TeamDesc *many = nullptr;
-    if (nb > 1) {
-        KSH_HIP(hipMemcpyAsync(d_descs, h.data(), sizeof(TeamDesc) * h.size(), hipMemcpyHostToDevice, s));
-        many = (const TeamDesc *)d_descs;
-    }
-    const dim3 gp((unsigned)nblk, (unsigned)nb), gs((unsigned)(8 * size * ((nb + 7) / 8)));
+    TeamDesc d;
+    d.fac = fac;
+    d.x = x;
+    d.n = n;
+    d.bw = bw;
+    d.ctl = (unsigned *)work;
+    d.b = (double *)((unsigned char *)work + 256);
+    d.mat = d.b + pad_rows(n) * (1 + kSlotVecs);
+    const int size = team_size(n, bw, prec);
+    const unsigned polls = poll_limit();
+    const dim3 gp((unsigned)(pad_rows(n) / kB)), gs((unsigned)(8 * size));
     if (prec == KSH_FP64) {
-        hipLaunchKernelGGL(k_team_prep<double>, gp, dim3(256), 0, s, h[0], many);
-        hipLaunchKernelGGL(k_team_solve<double>, gs, dim3(64 * kTW), 0, s, h[0], many, nb, size, poll_limit());
+        hipLaunchKernelGGL(k_team_prep<double>, gp, dim3(256), 0, s, d);
+        hipLaunchKernelGGL(k_team_solve<double>, gs, dim3(64 * kTW), 0, s, d, size, polls);
     } else {
-        hipLaunchKernelGGL(k_team_prep<float>, gp, dim3(256), 0, s, h[0], many);
-        hipLaunchKernelGGL(k_team_solve<float>, gs, dim3(64 * kTW), 0, s, h[0], many, nb, size, poll_limit());
+        hipLaunchKernelGGL(k_team_prep<float>, gp, dim3(256), 0, s, d);
+        hipLaunchKernelGGL(k_team_solve<float>, gs, dim3(64 * kTW), 0, s, d, size, polls);
     }
     KSH_HIP(hipGetLastError());
     return KSH_SUCCESS;
