@@ -43,6 +43,7 @@
 
 #include "ksh_devutil.hpp"
 #include "ksh_elim_steps.hpp"
+#include "ksh_factor_order.hpp"
 #include "ksh_internal.hpp"
 #include "ksh_mfma.hpp"
 #include "ksh_profile.hpp"
@@ -101,15 +102,13 @@ __device__ __forceinline__ void eliminate(C (&e)[kQ], C (&w)[4], C (&dsel)[4], i
 // What the row solves of a panel need beside its factored block, per band: the operands of the four
 // 16 x 16 inverses (step s of sub-block c at [(4 c + s) * 64 + lane]), then 1 / d of the 64 columns.
 constexpr int kWorkInv = 4 * 4 * 64;
-// Three slots a band, by panel: in the fused schedule a launch writes the next panel's while it still reads
-// this one's and the last one's.
 constexpr size_t kWorkSlot = (kWorkInv + kNB) * sizeof(double);
 template <typename C>
 __device__ __forceinline__ C *panel_work(void *work, int band, int c0)
 {
-    return (C *)((unsigned char *)work + (size_t)band * kBandWorkBytes + (size_t)(c0 / kNB % 3) * kWorkSlot);
+    return (C *)((unsigned char *)work + (size_t)band * kBandWorkBytes + (size_t)panel_slot(c0) * kWorkSlot);
 }
-static_assert(3 * kWorkSlot <= kBandWorkBytes, "factor workspace");
+static_assert(kPanelSlots * kWorkSlot <= kBandWorkBytes && kNB == 64, "factor workspace");
 
 // Row tiles of the panel at c0 (tile t: rows c0 + 64 + 16 t .. + 15, its 64 columns) against the factored
 // diagonal block, one wave: X = A L^-T by blocks of 16 columns (substitution between them, the 16 x 16
@@ -382,27 +381,6 @@ __device__ __forceinline__ void diag_panel(const BandDesc &d, int c0, C *work, c
     }
 }
 
-// lower-triangle block index p -> (bi, bj), bj <= bi
-__device__ __forceinline__ void tri_decode(int p, int &bi, int &bj)
-{
-    int b = (int)((sqrtf(8.0f * (float)p + 1.0f) - 1.0f) * 0.5f);
-    if ((b + 1) * (b + 2) / 2 <= p) ++b;
-    if (b * (b + 1) / 2 > p) --b;
-    bi = b;
-    bj = p - b * (b + 1) / 2;
-}
-
-// Parts of a step's trailing update (32 x 32 blocks (bi, bj), bj <= bi, of the window):
-// kAll every block; kNext block columns 0 and 1 (the next panel's columns); kRest the others.  The
-// three blocks of the next diagonal block, (0,0), (1,0) and (1,1), are left out of kAll and kNext:
-// the workgroup that factors it updates it (diag_panel).
-enum TrailPart { kAll = 0, kNext = 1, kRest = 2 };
-__host__ __device__ inline int trail_blocks(int nbk, int part)
-{
-    const int tail = nbk > 2 ? nbk - 2 : 0;  // block rows below the diagonal block
-    return part == kRest ? tail * (tail + 1) / 2 : part == kNext ? 2 * tail : tail * (tail + 1) / 2 + 2 * tail;
-}
-
 // Blocks p[0] < p[1] < ... of the given part (wave-uniform), computed together (independent
 // accumulators, the loads of all of them in flight at once): A[i][j] -= sum_k L[i][k] d_k L[j][k]
 // over the window rows/columns [w, nr) of the frame at c0.  Indices past the part's block count
@@ -435,16 +413,7 @@ __device__ __forceinline__ void trailing_blocks(const BandDesc &d, int c0, int p
         valid[s] = p[s] < nblock;
         const int q = valid[s] ? p[s] : p[0];
         int bi, bj;
-        if (part == kNext) {
-            bj = q < nbk - 2 ? 0 : 1;
-            bi = 2 + (bj == 0 ? q : q - (nbk - 2));
-        } else {
-            tri_decode(part == kAll ? q + 3 : q, bi, bj);
-            if (part == kRest) {
-                bi += 2;
-                bj += 2;
-            }
-        }
+        trail_decode(q, nbk, part, bi, bj);
         diag[s] = bi == bj;
         ri0[s] = w + 32 * bi + li;
         rj0[s] = w + 32 * bj + li;
@@ -525,34 +494,15 @@ __global__ __launch_bounds__(64 * kUW) void k_band_diag(const BandDesc *descs, v
     diag_panel<T, C, kFirst>(d, 0, panel_work<C>(work, (int)blockIdx.x, 0), nullptr, sh);
 }
 
-// XCD-aware assignment of a launch's workgroups to (band, index within the band).  Workgroups are
-// dispatched to the 8 XCDs round robin (id mod 8), each XCD with its own L2.  Every trailing block
-// of a band reads that band's panel, so with 8 or more bands the workgroups of band b take the ids
-// h = b (mod 8): all of them run on one XCD and its L2 serves the panel, which otherwise every
-// XCD would fetch once per band.  The panel kernels already put band b on workgroup b, the same
-// XCD.  With fewer bands than XCDs the plain mapping keeps every XCD busy.  Returns false for
-// the padding workgroups of the XCD-aware grid (8 ceil(active / 8) wg of them).
-constexpr int kXcds = 8;
+// a launch's workgroup h as (band, index within the band); false for a padding one
 __device__ __forceinline__ bool band_of_workgroup(int h, int active, int wg, int &band, int &local)
 {
-    if (active < kXcds) {
-        band = h / wg;
-        local = h % wg;
-    } else {
-        const int s = h / kXcds;
-        band = h % kXcds + kXcds * (s / wg);
-        local = s % wg;
-    }
+    workgroup_decode(h, active, wg, band, local);
     // the divisions run on the vector unit: back to scalars
     band = __builtin_amdgcn_readfirstlane(band);
     local = __builtin_amdgcn_readfirstlane(local);
     return band < active;
 }
-inline unsigned band_grid(int active, int wg)
-{
-    return (unsigned)(active < kXcds ? active * wg : ((active + kXcds - 1) / kXcds) * kXcds * wg);
-}
-
 // Rows of the panel at c0, kUW waves per workgroup and `tiles` 16-row tiles per wave
 template <typename T, typename C>
 __global__ __launch_bounds__(64 * kUW) void k_band_rows(const BandDesc *descs, void *work, int c0, int wg_per_band, int tiles,
