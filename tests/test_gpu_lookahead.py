@@ -1,6 +1,6 @@
-"""Lookahead schedules of the multi-workgroup factor (the next panel factored while the rest of the
-trailing update runs; KSH_LOOKAHEAD=1, 2: 8 waves x 1 block, 8 x 2 per workgroup)
-against the plain schedule (panel, then the whole update, per step, KSH_LOOKAHEAD=0).  Every
+"""The lookahead schedule of the multi-workgroup factor (KSH_LOOKAHEAD=1: the next panel solved while the
+rest of the trailing update runs) and the fused one (2, up to 8 bands: one launch a step; more bands are in
+test_gpu_panel.py) against the plain schedule (panel, then the whole update, per step, KSH_LOOKAHEAD=0).  Every
 32 x 32 block takes the same arithmetic on the same inputs in all of them, so pivots, solutions
 and paths must be bit-identical; the oracle comparisons of the factor itself are in
 test_gpu_tiled.py."""

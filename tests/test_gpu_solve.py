@@ -1,8 +1,8 @@
 """GPU band solves (forward, diagonal, backward substitution) against the oracle's band LDL^T solve.
 
-The shapes cover the kernel's cases: order below one 64-row block and band narrower than the
-block, orders that are not multiples of 64, the widest bands of the batch workload (bw 470), and
-a band wider than 512, which takes the multi-workgroup solve.  FP64 factors must reproduce the oracle's
+The shapes cover the cases: order below one 64-row block and band narrower than the block (the
+one-workgroup kernel, up to 128 rows), orders that are not multiples of 64, the widest bands of the batch
+workload (bw 470), and a band wider than 512 (team solves).  FP64 factors must reproduce the oracle's
 solution to rounding; FP32 factors (FP64 K) must reach it through FP64 refinement.
 """
 import numpy as np
@@ -35,8 +35,8 @@ def test_solve_matches_oracle(p, n, ny, prec, ksh):
         xr = fac.solve(b)
         if prec == 0:
             x = K.solve(b)
-            # forward error: rounding of another summation order (the multi-workgroup solve
-            # above bw 383 updates column-wise), grown by cond(K); backward error: rounding
+            # forward error: rounding of another summation order (a team's is by 64-row blocks), grown by
+            # cond(K); backward error: rounding
             Kb = o.tangent_band(u)
             r = b - ok.band_symv(Kb, o.nfree, o.bw, x)
             assert np.linalg.norm(r) <= 1e-14 * np.abs(Kb).max() * np.sqrt(o.bw) * np.linalg.norm(x)

@@ -121,20 +121,30 @@ def test_wide_band_takes_the_tiled_path(prec, ksh):
 
 
 @pytest.mark.parametrize("prec", [L.FP64, L.FP32_IR])
-def test_one_launch_stepped_solve_matches_the_stepped_launches(prec, ksh, monkeypatch):
-    """The opt-in one-launch form of the stepped solve (KSH_SOLVE_PERSIST=1: a cooperative launch
-    whose steps are separated by a grid barrier) computes the same steps as the stepped launches:
-    the same bits."""
-    from gsstructuralanalysis_amd.problem import ShellProblem
+def test_wide_solves_without_a_team(prec, ksh, monkeypatch):
+    """The solves that serve a wide band where a team does not (no memory for its workspace): the stepped
+    launches (KSH_BAND_PATH=tiled) and one workgroup streaming the band (wg).  Checked like the team solve by
+    ||b - K x|| <= c eps G ||x||, with G the largest entry of |L| |D| |L|^T of the oracle's factor, eps the
+    factor's precision, and c = 8 bw + 64 for one rounding per product along a band row, for the
+    factor and the two sweeps."""
+    from gsstructuralanalysis_amd.problem import BandMatrix, ShellProblem
+    from test_gpu_panel import _growth
     pt = g.roof_problem(p=3, n=140, ny=3, rho=1e3)
+    o = Oracle(pt)
     sp = ShellProblem(pt)
-    print(f"[case] one-launch stepped solve roof p=3 n=140 ny=3 nfree={sp.nfree} bw={sp.bw} prec={prec}", flush=True)
-    u = np.random.default_rng(9).standard_normal(sp.nfree) * 1e-3
-    K = sp.tangent(u, precision=prec)
+    print(f"[case] wide solves without a team roof p=3 n=140 ny=3 nfree={sp.nfree} bw={sp.bw} prec={prec}", flush=True)
+    rng = np.random.default_rng(9)
+    Kb = o.tangent_band(rng.standard_normal(sp.nfree) * 1e-3)
+    ref = ok.BandLDLT(Kb, o.nfree, o.bw)
+    K = BandMatrix(sp, precision=prec)
+    K.upload(Kb)
+    K.set_inertia_guard(0.0)
     K.factor()
-    b = np.random.default_rng(10).standard_normal(sp.nfree)
-    x0 = K.solve(b)
-    monkeypatch.setenv("KSH_SOLVE_PERSIST", "1")
-    x1 = K.solve(b)
-    assert np.all(np.isfinite(x1))
-    assert np.array_equal(x0, x1)
+    b = rng.standard_normal(sp.nfree)
+    eps = np.finfo(np.float64 if prec == L.FP64 else np.float32).eps
+    bound = (8 * o.bw + 64) * eps * _growth(ref, o.nfree, o.bw)
+    for path in ("tiled", "wg"):
+        monkeypatch.setenv("KSH_BAND_PATH", path)
+        x = K.solve(b)
+        r = b - ok.band_symv(Kb, o.nfree, o.bw, x)
+        assert np.linalg.norm(r) <= bound * np.linalg.norm(x), path
