@@ -398,7 +398,7 @@ def main():
     tuned = {}
     shapes = {"tangent_tiles": lambda v: f"{1 << v} elements per workgroup",
               "band_gather": lambda v: f"{128 << v} threads per block",
-              "band_factor": lambda v: ("plain", "lookahead 8 waves x 1 block", "lookahead 8 waves x 2 blocks")[v]}
+              "band_factor": lambda v: ("plain", "lookahead 8 waves x 1 block", "fused (lookahead x 2 blocks above 8 bands)")[v]}
     for k, shape in shapes.items():
         v, nv = C.c_int64(), C.c_int64()
         lib.ksh_tune_choice(k.encode(), C.byref(v), C.byref(nv))
