@@ -46,6 +46,19 @@ KSH_INDEX void trail_decode(int q, int nbk, int part, int &bi, int &bj)
     }
 }
 
+// Most bands of a call that schedule 2 serves by fused steps (one launch a step); more take the lookahead
+// schedule with two blocks per wave.
+constexpr int kFusedBands = 8;
+// The autotuner's bucket for the number of bands, ceil(log2): its edges lie where a schedule changes, so no
+// choice timed on fused steps serves calls that cannot have them (9 to 15 bands of 32 x 32 roofs took
+// 17% to 21% longer with schedule 2 than with the best, which 8 bands have as their best).
+KSH_INDEX int count_bucket(int bands)
+{
+    int b = 0;
+    while (1 << b < bands) ++b;
+    return b;
+}
+
 // Panel workspaces of a band: three, by panel, since a launch of the fused schedule writes the next panel's
 // while it still reads this one's and the last one's.
 constexpr int kPanelSlots = 3;

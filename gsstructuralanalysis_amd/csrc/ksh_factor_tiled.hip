@@ -715,9 +715,8 @@ __global__ __launch_bounds__(1024) void k_pivot_stats(const BandDesc *descs)
 // Plain has the rest of the update beside the diagonal block's chain, lookahead beside the rows, fused the
 // shortest chain and the most arithmetic; which one is fastest depends on the number and shape of the
 // bands, so the autotuner picks per shape bucket (KSH_LOOKAHEAD=k forces k).
-// Fused up to 8 bands: a band's workgroups (22 at bw 326, 192 at bw 1166) then stay around the chip's 256
-// CUs; with more, the threefold arithmetic is what bounds the step.
-constexpr int kFusedBands = 8;
+// Fused up to kFusedBands bands: a band's workgroups (22 at bw 326, 192 at bw 1166) then stay around the
+// chip's 256 CUs; with more, the threefold arithmetic is what bounds the step.
 constexpr int kSchedules = 3;
 
 int schedule_forced()
@@ -900,7 +899,7 @@ int run_factor(hipStream_t s, const BandDesc *d_descs, const std::vector<int> &n
     const int forced = schedule_forced();
     if (forced >= 0) return run_tiled_graph<T>(s, d_descs, ns, maxbw, prec, forced);
     const long long bucket =
-        ((((long long)prec * 64 + tune_bucket(maxbw)) * 64 + tune_bucket((double)ns.size())) * 64) + tune_bucket(ns[0]);
+        ((((long long)prec * 64 + tune_bucket(maxbw)) * 64 + count_bucket((int)ns.size())) * 64) + tune_bucket(ns[0]);
     int rc = KSH_SUCCESS;
     tune_launch("band_factor", bucket, kSchedules, 0, s,
                 [&](int v) { rc = run_tiled_graph<T>(s, d_descs, ns, maxbw, prec, v); });

@@ -54,6 +54,8 @@ int main()
         std::printf("tri %d %d\n", bi, bj);
     }
     for (int k = 0; k < 100; ++k) std::printf("slot %d\n", panel_slot(64 * k));
+    std::printf("fused %d\n", kFusedBands);
+    for (int n = 1; n <= 1024; ++n) std::printf("bucket %d %d\n", n, count_bucket(n));
     for (int active : {1, 3, 7, 8, 9, 16, 37, 256})
         for (int wg : {1, 2, 5})
             for (int h = 0; h < (int)band_grid(active, wg); ++h) {
@@ -70,7 +72,7 @@ class Order:
     """The kernels' index arithmetic, as tables."""
 
     def __init__(self, text):
-        self.parts, self.tri, self.slots, self.wg = {}, [], [], {}
+        self.parts, self.tri, self.slots, self.wg, self.buckets = {}, [], [], {}, {}
         for line in text.splitlines():
             kind, *v = line.split()
             v = [int(x) for x in v]
@@ -80,6 +82,10 @@ class Order:
                 self.tri.append((v[0], v[1]))
             elif kind == "slot":
                 self.slots.append(v[0])
+            elif kind == "fused":
+                self.fused_bands = v[0]
+            elif kind == "bucket":
+                self.buckets.setdefault(v[1], []).append(v[0])
             else:
                 self.wg.setdefault((v[0], v[1]), []).append(tuple(v[2:]))
 
@@ -412,6 +418,15 @@ def test_parts_cover_every_block_once(nbk, order):
     assert len(every) == len(allb) and set(every) == allb
     assert sorted(nxt + rest) == sorted(allb)
     assert all(bj <= 1 for _, bj in nxt) and all(bj >= 2 for _, bj in rest)
+
+
+def test_tuning_buckets_end_where_the_schedule_changes(order):
+    """Counts that share a tuned choice have the same launches under every schedule, and are within a factor
+    of two of each other."""
+    for counts in order.buckets.values():
+        assert max(counts) <= order.fused_bands or min(counts) > order.fused_bands
+        assert max(counts) <= 2 * min(counts)
+    assert sorted(n for counts in order.buckets.values() for n in counts) == list(range(1, 1025))
 
 
 def test_tile_numbers(order):
